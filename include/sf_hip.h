@@ -178,6 +178,17 @@ typedef struct sf_attn_desc {
      * with P as an fp16 (hi, lo) pair.  SF_ENOTSUP with another in_dtype or
      * with exact_pv. */
     int32_t v_f16;
+    /* o_frag != 0: out is written as the [B*Sq][H*64] operand of
+     * sf_gemm_frag in fragment order (row b*Sq + q, column h*64 + d; bf16 or
+     * fp16) instead of through o_stride (ignored; SF_ENOTSUP for SF_F32). */
+    int32_t o_frag;
+    /* q_rows32 != NULL (in_dtype SF_BF16, no q_partials, no q_f16): Q given
+     * as the fp32 rows [B*Sq][H*64] of a finished projection instead of q
+     * (which may then be NULL): row b*Sq + s, column h*64 + d, normalised
+     * with q_gamma (when set) and rounded to bf16 as it is loaded, on any
+     * grid (key sets of at most 128 then run the ring kernel).  16-byte
+     * aligned, at most 2 GB; SF_ENOTSUP with k_gamma. */
+    const float* q_rows32;
 } sf_attn_desc;
 
 /* Fills a descriptor for contiguous [B,H,S,D] tensors (the layout
@@ -479,6 +490,93 @@ typedef struct sf_w16_job {
     int32_t N, K;
 } sf_w16_job;
 int sf_weights_to_f16(const sf_w16_job* jobs, int32_t count, void* stream);
+
+/* ---------------------------------------------------------------------------
+ * Fragment-ordered projections: one launch per projection for few rows.
+ *
+ * Fragment order of X[R][K] in 16 bits: blocks of 16 rows x 32 columns, block
+ * (r / 16, k / 32) at index (r / 16) * (K / 32) + k / 32, 512 elements each;
+ * inside a block, element (r, k) at (((k % 32) / 8) * 16 + r % 16) * 8 + k % 8.
+ * R is padded to a multiple of 16; the padding rows are never written and may
+ * hold anything.  int8: blocks of 16 rows x 64 columns, 1024 bytes, code
+ * (r, k) at (((k % 32) / 8) * 16 + r % 16) * 16 + ((k % 64) / 32) * 8 + k % 8.
+ * No counterpart in the reference: the layout lets a wave load an MFMA
+ * operand as 1 KB of contiguous memory.
+ * ------------------------------------------------------------------------- */
+/* Elements of a fragment-ordered [rows][cols] buffer. */
+size_t sf_frag_elems(int64_t rows, int64_t cols);
+
+/* Row-major weights w [N][ldw] -> out in fragment order, up to
+ * SF_CODES_MAX_JOBS matrices per launch: bf16 -> bf16, bf16 -> fp16 (rounded
+ * as sf_weights_to_f16 does), fp16 -> fp16, int8 -> int8.  N a multiple of
+ * 16, K of 64, ldw of 8, pointers 16-byte aligned. */
+typedef struct sf_frag_job {
+    const void* w;
+    int32_t w_dtype;
+    int64_t ldw;
+    void* out;
+    int32_t out_dtype;
+    int32_t N, K;
+} sf_frag_job;
+int sf_frag_pack(const sf_frag_job* jobs, int32_t count, void* stream);
+
+/* RMSNorm of fp32 rows (cols a multiple of 64, at most 4096; rows and gamma
+ * 16-byte aligned) into fragment order in SF_BF16 or SF_F16
+ * (rms_norm_kernel_impl, norm.cuh:89-122).  ss != NULL: the deferred form of
+ * sf_rmsnorm_deferred instead: x * gamma, and ss [rows][cols / 64] (row-major
+ * here) the sums of squares of 64 columns. */
+int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int32_t out_dtype, float* ss,
+                 int32_t rows, int32_t cols, float eps, void* stream);
+
+/* C = act((A . W^T) * w_scale * row scale + bias) (act with SF_EPI_PLAIN,
+ * the row scale not with SF_EPI_ADD_NORM) with A and W in fragment
+ * order, one launch, no workspace: sf_gemm's arithmetic (gemm_bias_act,
+ * cuda_backend.cu:337-467) and epilogues over all of K in one workgroup.
+ * M <= 160, N a multiple of 32, K of 64.  a_dtype SF_BF16 or SF_F16; w_dtype
+ * the same, or SF_I8 with w_scale.  Epilogues:
+ *   SF_EPI_PLAIN     C row-major (ldc a multiple of 4) in c_dtype, with
+ *                    accumulate for SF_F32; or, with c_frag, in fragment
+ *                    order (SF_BF16 / SF_F16).
+ *   SF_EPI_HEADS     as sf_gemm's: bf16 per-head outputs with the optional
+ *                    per-head RMSNorm.
+ *   SF_EPI_ADD_NORM  the deferred form only: C (fp32) += result, norm_out
+ *                    (fragment order, norm_dtype) = C * norm_gamma, and
+ *                    norm_ss[m * T + t] = the sum of C[m][n]^2 over tile t's
+ *                    columns, T = sf_gemm_frag_ss_tiles(N) <= 64 tiles.
+ * a_row_ss (SF_EPI_PLAIN, SF_EPI_HEADS): as sf_gemm_desc's, but row-major,
+ * [M][a_row_tiles].  Row m's result depends on
+ * row m, the weights and the summation order that K fixes, not on M. */
+typedef struct sf_frag_gemm_desc {
+    int32_t M, N, K;
+    const void* A;
+    int32_t a_dtype;
+    const void* W;
+    int32_t w_dtype;
+    const float* w_scale;
+    const float* bias;
+    int32_t act;
+    int32_t epilogue;
+    void* C;
+    int64_t ldc;
+    int32_t c_dtype;
+    int32_t c_frag;
+    int32_t accumulate;
+    int32_t H, S;
+    float eps;
+    const float* head_gamma[3];
+    void* head_out[3];
+    int64_t head_stride[3][3];
+    const float* norm_gamma;
+    void* norm_out;
+    int32_t norm_dtype;
+    float* norm_ss;
+    const float* a_row_ss;
+    int32_t a_row_tiles;
+    int32_t a_row_n;
+    float a_row_eps;
+} sf_frag_gemm_desc;
+int sf_gemm_frag(const sf_frag_gemm_desc* desc, void* stream);
+int32_t sf_gemm_frag_ss_tiles(int32_t N);
 
 /* Static text for a status code. */
 const char* sf_strerror(int status);

@@ -63,6 +63,8 @@ class AttnDesc(ctypes.Structure):
         ("q_row_n", ctypes.c_int32),
         ("q_row_eps", ctypes.c_float),
         ("v_f16", ctypes.c_int32),
+        ("o_frag", ctypes.c_int32),
+        ("q_rows32", ctypes.c_void_p),
     ]
 
 
@@ -104,6 +106,41 @@ class GemmDesc(ctypes.Structure):
         ("a_row_n", ctypes.c_int32),
         ("a_row_eps", ctypes.c_float),
     ]
+
+
+class FragGemmDesc(ctypes.Structure):
+    """Mirror of `sf_frag_gemm_desc`."""
+
+    _fields_ = [
+        ("M", ctypes.c_int32), ("N", ctypes.c_int32), ("K", ctypes.c_int32),
+        ("A", ctypes.c_void_p), ("a_dtype", ctypes.c_int32),
+        ("W", ctypes.c_void_p), ("w_dtype", ctypes.c_int32),
+        ("w_scale", ctypes.c_void_p),
+        ("bias", ctypes.c_void_p),
+        ("act", ctypes.c_int32),
+        ("epilogue", ctypes.c_int32),
+        ("C", ctypes.c_void_p), ("ldc", ctypes.c_int64), ("c_dtype", ctypes.c_int32),
+        ("c_frag", ctypes.c_int32),
+        ("accumulate", ctypes.c_int32),
+        ("H", ctypes.c_int32), ("S", ctypes.c_int32), ("eps", ctypes.c_float),
+        ("head_gamma", ctypes.c_void_p * 3),
+        ("head_out", ctypes.c_void_p * 3),
+        ("head_stride", (ctypes.c_int64 * 3) * 3),
+        ("norm_gamma", ctypes.c_void_p), ("norm_out", ctypes.c_void_p),
+        ("norm_dtype", ctypes.c_int32),
+        ("norm_ss", ctypes.c_void_p),
+        ("a_row_ss", ctypes.c_void_p),
+        ("a_row_tiles", ctypes.c_int32),
+        ("a_row_n", ctypes.c_int32),
+        ("a_row_eps", ctypes.c_float),
+    ]
+
+
+class FragJob(ctypes.Structure):
+    """Mirror of `sf_frag_job`."""
+
+    _fields_ = [("w", ctypes.c_void_p), ("w_dtype", ctypes.c_int32), ("ldw", ctypes.c_int64),
+                ("out", ctypes.c_void_p), ("out_dtype", ctypes.c_int32), ("N", ctypes.c_int32), ("K", ctypes.c_int32)]
 
 
 class CodesJob(ctypes.Structure):
@@ -186,6 +223,16 @@ def lib() -> ctypes.CDLL:
     L.sf_int8_codes_to_bf16.restype = ctypes.c_int
     L.sf_weights_to_f16.argtypes = [ctypes.POINTER(W16Job), i32, vp]
     L.sf_weights_to_f16.restype = ctypes.c_int
+    L.sf_frag_elems.argtypes = [i64, i64]
+    L.sf_frag_elems.restype = ctypes.c_size_t
+    L.sf_frag_pack.argtypes = [ctypes.POINTER(FragJob), i32, vp]
+    L.sf_frag_pack.restype = ctypes.c_int
+    L.sf_norm_frag.argtypes = [vp, i64, vp, vp, i32, vp, i32, i32, ctypes.c_float, vp]
+    L.sf_norm_frag.restype = ctypes.c_int
+    L.sf_gemm_frag.argtypes = [ctypes.POINTER(FragGemmDesc), vp]
+    L.sf_gemm_frag.restype = ctypes.c_int
+    L.sf_gemm_frag_ss_tiles.argtypes = [i32]
+    L.sf_gemm_frag_ss_tiles.restype = i32
     L.sf_gemm_num_splits.argtypes = [ctypes.POINTER(GemmDesc)]
     L.sf_gemm_num_splits.restype = ctypes.c_int32
     L.sf_gemm_int8_direct.argtypes = [ctypes.POINTER(GemmDesc)]

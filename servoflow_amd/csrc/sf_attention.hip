@@ -67,6 +67,7 @@ struct AttnArgs {
     int nsplit;
     int nqc;          // query chunks
     int out_kind;     // OutKind
+    int o_frag;       // o in fragment order (rows b * Sq + q, columns h * 64 + d)
     int causal;
     float scale_log2;   // scale * log2(e)
     // Q from split-K partials (the kQP instance): [q_splits][B*Sq][H*64]
@@ -88,9 +89,15 @@ struct AttnArgs {
 
 enum OutKind { kOutBF16 = 0, kOutF32 = 1, kOutF16 = 2 };
 
+// Element offset of out[b][h][q][d .. d + 3] (d a multiple of 4).
+__device__ __forceinline__ int64_t out_off(const AttnArgs& a, int b, int h, int q, int d) {
+    if (a.o_frag) return frag_off(b * a.Sq + q, h * kD + d, a.H * kD);
+    return b * a.o_sb + h * a.o_sh + q * a.o_ss + d;
+}
+
 __device__ __forceinline__ void store_out(const AttnArgs& a, int b, int h, int q,
                                           int d, float val) {
-    const int64_t off = b * a.o_sb + h * a.o_sh + q * a.o_ss + d;
+    const int64_t off = out_off(a, b, h, q, d & ~3) + (d & 3);
     if (a.out_kind == kOutF32) {
         reinterpret_cast<float*>(a.o)[off] = val;
     } else if (a.out_kind == kOutF16) {
@@ -390,7 +397,7 @@ __device__ __forceinline__ void attn_split_epilogue(const AttnArgs& a, float* xo
         if (q >= a.Sq) continue;
         if (nsplit == 1) {
             o *= L > 0.f ? __builtin_amdgcn_rcpf(L) : 0.f;
-            store_out4(a, b * a.o_sb + h * a.o_sh + q * a.o_ss + d0, o);
+            store_out4(a, out_off(a, b, h, q, d0), o);
         } else {
             // non-temporal: the merge kernel reads the partials once, and
             // stores that do not linger dirty in L2 leave less to write back
@@ -464,10 +471,12 @@ __device__ __forceinline__ void ring_wait_k() {
 // type and P as a (hi, lo) pair of that type.  kF16: Q/K/V are fp16 (S on
 // the fp16 MFMA) instead of bf16.  QB: 16-row query blocks per workgroup
 // (kQB on the (split x chunk, H, B) grid; 1 on the XCD-grouped 1-D grid).
-// kQP (QB = 1, bf16): Q is finished here from its projection's split-K
-// partials (sum, scale, bias, per-head RMSNorm, bf16) instead of loaded.
+// kQP (bf16): Q is finished here from at most kQP split-K partials of its
+// projection (sum, scale, bias, per-head RMSNorm, bf16) instead of loaded: 8
+// on the query-block grid; 1 on the 80-row grid, whose key splits each fetch
+// a head's rows (17 KB from one partial; eight would be 137 KB for each).
 // kVH (bf16 Q/K, fp16 form): V is given in fp16 and used as loaded.
-template <bool kExactPV, bool kF16, int QB, bool kQP = false, bool kVH = false>
+template <bool kExactPV, bool kF16, int QB, int kQP = 0, bool kVH = false>
 __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
     static_assert(!(kVH && (kExactPV || kF16)), "fp16 V: the fp16 P.V form of bf16 Q/K");
     using v8 = typename In16<kF16>::v8;
@@ -527,28 +536,35 @@ __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
 
     // Q fragments (B operand of S^T = K.Q^T): row 16qb + r, dims 32hh + 8g..
     v8 qf[QB][2];
-    // kQP: wave w finishes rows q0 + 4w .. q0 + 4w + 3, lane l row
-    // q0 + 4w + l/16 and dims 4(l%16) .. +3 -- the reduce_heads epilogue's
-    // layout and arithmetic, so Q is bit-identical to the unfused path.
-    // Every split's loads go out here, before the ring's first tiles; rows
-    // past Sq and splits past q_splits read as zeros.
-    constexpr int kQPMax = 8;
-    f32x4 qpv[kQP ? kQPMax : 1];
+    // kQP: wave w finishes rows 4 QB w .. 4 QB w + 4 QB - 1 of the block, four
+    // at a time: lane l row 4 QB w + 4 j + l/16 and dims 4(l%16) .. +3 -- the
+    // reduce_heads epilogue's layout and arithmetic, so Q is bit-identical to
+    // the unfused path.  Every split's loads go out here, before the ring's
+    // first tiles; rows past Sq and splits past q_splits read as zeros.
+    constexpr int kQPMax = kQP ? kQP : 1;
+    constexpr int kQPRows = kQP ? QB : 1;
+    f32x4 qpv[kQPRows][kQPMax];
     f32x4 qbias, qscale, qgam;
     float qrss[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (kQP) {
-        static_assert(QB == 1 && !kF16, "Q from partials: the bf16 query-block instance");
-        const int row = q0 + 4 * w + (lane >> 4);
+    if constexpr (kQP > 0) {
+        static_assert(!kF16 && (QB == 1 || kQP == 1), "Q from partials: bf16; one partial on the 80-row grid");
         const int c4 = 4 * (lane & 15);
-        const bool rlive = row < a.Sq;
-        const uint32_t rowoff = rlive ? (uint32_t)(((int64_t)b * a.Sq + row) * (a.H * 64) + h * 64 + c4) : 0u;
         const uint32_t sstride = (uint32_t)((int64_t)a.B * a.Sq * a.H * 64);
         const __amdgpu_buffer_rsrc_t prs = make_rsrc(a.qp, a.qp_bytes);
 #pragma unroll
-        for (int j = 0; j < kQPMax; ++j) {
-            const uint32_t off = j < a.q_splits && rlive ? (rowoff + j * sstride) * 4u
-                                                         : 0x80000000u;   // past the buffer range: zeros
-            qpv[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(prs, off, 0, kKvPolicy));
+        for (int jr = 0; jr < kQPRows; ++jr) {
+            const int row = q0 + 4 * QB * w + 4 * jr + (lane >> 4);
+            const bool rlive = row < a.Sq;
+            const uint32_t rowoff = rlive ? (uint32_t)(((int64_t)b * a.Sq + row) * (a.H * 64) + h * 64 + c4) : 0u;
+#pragma unroll
+            for (int j = 0; j < kQPMax; ++j) {
+                const uint32_t off = j < a.q_splits && rlive ? (rowoff + j * sstride) * 4u
+                                                             : 0x80000000u;   // past the buffer range: zeros
+                // read once per call on the query-block grid, by every key
+                // split of the head on the 80-row one
+                qpv[jr][j] = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(prs, off, 0, QB == 1 ? kKvPolicy : 0));
+            }
         }
         const int nb = h * 64 + c4;
         const __amdgpu_buffer_rsrc_t brs = make_rsrc(a.q_bias, a.q_bias ? (uint32_t)(a.H * 64 * 4) : 0u);
@@ -557,8 +573,9 @@ __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
         qbias = __builtin_bit_cast(f32x4, buffer_load16(brs, (uint32_t)(nb * 4)));
         qscale = __builtin_bit_cast(f32x4, buffer_load16(srs, (uint32_t)(nb * 4)));
         qgam = __builtin_bit_cast(f32x4, buffer_load16(grs, (uint32_t)(c4 * 4)));
-        if (a.q_row_ss) {   // the deferred norm's tile sums of this lane's row
-            const int64_t prow = (int64_t)b * a.Sq + (rlive ? row : 0);
+        if (QB == 1 && a.q_row_ss) {   // the deferred norm's tile sums of this lane's row
+            const int row = q0 + 4 * w + (lane >> 4);
+            const int64_t prow = (int64_t)b * a.Sq + (row < a.Sq ? row : 0);
             const int64_t M = (int64_t)a.B * a.Sq;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -576,7 +593,7 @@ __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
     }
     // q_norm weight for Q rows normalised as they are loaded (bf16)
     f32x4 qgm[2][2];
-    if constexpr (!kQP) load_norm_gamma(a.q_gamma, g, qgm);
+    if constexpr (kQP == 0) load_norm_gamma(a.q_gamma, g, qgm);
 
     // DMA of one tile into a stage: wave w, op j fills LDS chunks
     // (4w + j) * 64 + lane = key * 8 + slot of K (and of V), loading global
@@ -628,48 +645,54 @@ __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
     // the mask words, and ring_wait waits for one tile at a time.
     issue(0);
     issue(1);
-    if constexpr (kQP) {
+    if constexpr (kQP > 0) {
         // Q = rmsnorm_64(sum_j part_j * scale + bias) * gamma in bf16, as
         // reduce_heads_kernel computes it (slices summed in ascending order;
         // no scale = 1, no bias = 0, no gamma = no norm), rows exchanged
-        // through LDS so that every wave holds the fragments of all 16.  The
-        // LDS accesses are inline asm: the compiler would otherwise wait for
-        // the in-flight ring DMA in front of them.
-        __shared__ __attribute__((aligned(16))) uint16_t qlds[16 * 64];
-        f32x4 v = qpv[0];
-#pragma unroll
-        for (int j = 1; j < kQPMax; ++j)
-            if (j < a.q_splits) v += qpv[j];
-        if (a.q_row_ss) {   // as reduce_heads_kernel over x * gamma rows (deferred_row_scale)
-            float tsum = 0.f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if ((lane & 15) + 16 * k < a.q_row_tiles) tsum += qrss[k];
-            const float rs = deferred_rsqrt(row16_sum(tsum), a.q_row_inv_n, a.q_row_eps);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = deferred_affine(v[i], a.q_scale ? qscale[i] : 1.f, rs, qbias[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = v[i] * (a.q_scale ? qscale[i] : 1.f) + qbias[i];
-        }
-        if (a.q_gamma) {
-            float ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-            ss = row16_sum(ss);
-            const float inv_rms = 1.f / sqrtf(ss / 64.f + a.q_eps);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = v[i] * inv_rms * qgam[i];
-        }
+        // through LDS so that every wave holds the fragments of all of them.
+        // The LDS accesses are inline asm: the compiler would otherwise wait
+        // for the in-flight ring DMA in front of them.
+        __shared__ __attribute__((aligned(16))) uint16_t qlds[QR * 64];
         const uint32_t qbase = lds_addr(qlds);
-        const uint32_t waddr = qbase + (uint32_t)(((4 * w + (lane >> 4)) * 64 + 4 * (lane & 15)) * 2);
-        const uint32_t wlo = pack_bf16x2(v[0], v[1]), whi = pack_bf16x2(v[2], v[3]);
-        asm volatile("ds_write_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier"
-                     :: "v"(waddr), "v"(uint2{wlo, whi}) : "memory");
-        u32x4 q0w, q1w;
-        const uint32_t raddr = qbase + (uint32_t)((r * 64 + 8 * g) * 2);
-        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(q0w), "=&v"(q1w) : "v"(raddr) : "memory");
-        qf[0][0] = __builtin_bit_cast(v8, q0w);
-        qf[0][1] = __builtin_bit_cast(v8, q1w);
+#pragma unroll
+        for (int jr = 0; jr < kQPRows; ++jr) {
+            f32x4 v = qpv[jr][0];
+#pragma unroll
+            for (int j = 1; j < kQPMax; ++j)
+                if (j < a.q_splits) v += qpv[jr][j];
+            if (QB == 1 && a.q_row_ss) {   // as reduce_heads_kernel over x * gamma rows (deferred_row_scale)
+                float tsum = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if ((lane & 15) + 16 * k < a.q_row_tiles) tsum += qrss[k];
+                const float rs = deferred_rsqrt(row16_sum(tsum), a.q_row_inv_n, a.q_row_eps);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = deferred_affine(v[i], a.q_scale ? qscale[i] : 1.f, rs, qbias[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = v[i] * (a.q_scale ? qscale[i] : 1.f) + qbias[i];
+            }
+            if (a.q_gamma) {
+                float ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+                ss = row16_sum(ss);
+                const float inv_rms = 1.f / sqrtf(ss / 64.f + a.q_eps);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = v[i] * inv_rms * qgam[i];
+            }
+            const uint32_t waddr = qbase + (uint32_t)(((4 * QB * w + 4 * jr + (lane >> 4)) * 64 + 4 * (lane & 15)) * 2);
+            const uint32_t wlo = pack_bf16x2(v[0], v[1]), whi = pack_bf16x2(v[2], v[3]);
+            asm volatile("ds_write_b64 %0, %1" :: "v"(waddr), "v"(uint2{wlo, whi}) : "memory");
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            u32x4 q0w, q1w;
+            const uint32_t raddr = qbase + (uint32_t)(((16 * qb + r) * 64 + 8 * g) * 2);
+            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(q0w), "=&v"(q1w) : "v"(raddr) : "memory");
+            qf[qb][0] = __builtin_bit_cast(v8, q0w);
+            qf[qb][1] = __builtin_bit_cast(v8, q1w);
+        }
     }
     // Wait for the Q fragments here, behind the first tiles' loads.  Inside
     // the tile loop the compiler would otherwise still count them as
@@ -679,7 +702,7 @@ __global__ __launch_bounds__(256, 2) void attn_ring_kernel(const AttnArgs a) {
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) asm volatile("" ::"v"(qf[qb][hh]));
-    if constexpr (!kQP) {
+    if constexpr (kQP == 0) {
         if constexpr (!kF16) {
             if (a.q_f16) {   // fp16 rows: normalised (with q_gamma) and rounded to bf16
 #pragma unroll
@@ -1217,7 +1240,7 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
     // O^T lane layout: head dims 16db + 4g + i of query qrow
 #pragma unroll
     for (int db = 0; db < 4; ++db)
-        store_out4(a, b * a.o_sb + h * a.o_sh + qrow * a.o_ss + 16 * db + 4 * g, acc[db] * inv);
+        store_out4(a, out_off(a, b, h, qrow, 16 * db + 4 * g), acc[db] * inv);
 }
 
 // ---------------------------------------------------------------------------
@@ -1336,7 +1359,7 @@ __global__ __launch_bounds__(64) void attn_f32_kernel(const AttnArgs a) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
         for (int db = 0; db < 4; ++db)
-            store_out4(a, b * a.o_sb + h * a.o_sh + qrow * a.o_ss + 16 * db + 4 * g, acc[db] * inv);
+            store_out4(a, out_off(a, b, h, qrow, 16 * db + 4 * g), acc[db] * inv);
     } else {
         const size_t row = (((size_t)b * a.H + h) * nsplit + split) * (size_t)a.Sq + qrow;
 #pragma unroll
@@ -1393,6 +1416,9 @@ int choose_splits(const sf_attn_desc* d) {
     return (int)ns;
 }
 
+// Key sets of the short-key kernel.
+bool short_key_call(const sf_attn_desc* d) { return d->Sk <= sfk::kShortMaxKeys && d->num_splits <= 1; }
+
 template <int NW, bool F16, bool VH>
 void launch_short_kb(int kb, dim3 grid, hipStream_t s, const sfk::AttnArgs& a) {
     const dim3 block(64 * NW);
@@ -1419,18 +1445,20 @@ void launch_ring(bool exact, bool f16, bool vh, dim3 grid, hipStream_t s, const 
         if (f16) hipLaunchKernelGGL((sfk::attn_ring_kernel<true, true, QB>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((sfk::attn_ring_kernel<true, false, QB>), grid, dim3(256), 0, s, a);
     } else if (vh) {
-        hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, QB, false, true>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, QB, 0, true>), grid, dim3(256), 0, s, a);
     } else {
         if (f16) hipLaunchKernelGGL((sfk::attn_ring_kernel<false, true, QB>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, QB>), grid, dim3(256), 0, s, a);
     }
 }
 
-// The query-block grid with Q finished from split-K partials (bf16).
+// Q finished from split-K partials (bf16): up to 8 on the query-block grid,
+// one on the 80-row grid.
+template <int QB, int QP>
 void launch_ring_qp(bool exact, bool vh, dim3 grid, hipStream_t s, const sfk::AttnArgs& a) {
-    if (exact) hipLaunchKernelGGL((sfk::attn_ring_kernel<true, false, 1, true>), grid, dim3(256), 0, s, a);
-    else if (vh) hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, 1, true, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, 1, true>), grid, dim3(256), 0, s, a);
+    if (exact) hipLaunchKernelGGL((sfk::attn_ring_kernel<true, false, QB, QP>), grid, dim3(256), 0, s, a);
+    else if (vh) hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, QB, QP, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((sfk::attn_ring_kernel<false, false, QB, QP>), grid, dim3(256), 0, s, a);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1468,8 +1496,16 @@ int validate(const sf_attn_desc* d) {
     } else if (d->q_row_ss) {
         return SF_EINVAL;   // a row scale applies to Q given as partials only
     }
+    if (d->q_rows32) {   // Q as the fp32 rows of a finished projection
+        if (d->in_dtype != SF_BF16 || d->q_partials || d->q_f16 || d->k_gamma) return SF_ENOTSUP;
+        if ((reinterpret_cast<uintptr_t>(d->q_rows32) | reinterpret_cast<uintptr_t>(d->q_gamma)) & 15) return SF_EINVAL;
+        if ((int64_t)d->B * d->Sq * d->H * 64 * 4 > 0x7fffffffLL) return SF_ENOTSUP;
+    }
     if (d->q_f16) {   // fp16 Q rows against bf16 K / V
         if (d->in_dtype != SF_BF16 || d->q_partials) return SF_ENOTSUP;
+    }
+    if (d->o_frag) {   // 16-bit rows b * Sq + q
+        if (d->out_dtype == SF_F32 || (int64_t)d->B * d->Sq > 0x7fffffffLL) return SF_ENOTSUP;
     }
     if (d->v_f16) {   // fp16 V against bf16 Q / K, fp16 P.V form
         if (d->in_dtype != SF_BF16 || d->exact_pv) return SF_ENOTSUP;
@@ -1559,13 +1595,13 @@ extern "C" void sf_attn_desc_init_bhsd(sf_attn_desc* d, int32_t B, int32_t H, in
 
 extern "C" int32_t sf_attn_num_splits(const sf_attn_desc* d) {
     if (validate(d) != SF_OK) return 0;
-    if (d->Sk <= sfk::kShortMaxKeys && d->num_splits <= 1) return 1;
+    if (short_key_call(d)) return 1;
     return choose_splits(d);
 }
 
 extern "C" size_t sf_attn_workspace_bytes(const sf_attn_desc* d) {
     if (validate(d) != SF_OK) return 0;
-    if (d->Sk <= sfk::kShortMaxKeys && d->num_splits <= 1) return 0;
+    if (short_key_call(d)) return 0;
     const int ns = choose_splits(d);
     if (ns <= 1) return 0;
     const size_t rows = (size_t)d->B * d->H * ns * d->Sq;
@@ -1577,14 +1613,17 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
     int st = validate(d);
     if (st != SF_OK) return st;
     if ((long)d->B * d->H * d->Sq == 0) return SF_OK;
-    const bool q_from_partials = d->q_partials != nullptr;
+    // fp32 rows of a finished projection are one "partial"
+    const float* qpart = d->q_partials ? d->q_partials : d->q_rows32;
+    const int qsplits = d->q_partials ? d->q_splits : 1;
+    const bool q_from_partials = qpart != nullptr;
     if (!q_from_partials && !q) return SF_EINVAL;
     if (!k || !v || !out) return SF_EINVAL;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return SF_EINVAL;
     if (d->B > 65535 || d->H > 65535) return SF_ENOTSUP;
 
-    // (Q from partials runs the query-block grid whatever the key count)
-    const bool short_keys = d->Sk <= sfk::kShortMaxKeys && d->num_splits <= 1 && !q_from_partials;
+    // (Q from fp32 rows runs the ring kernel whatever the key count)
+    const bool short_keys = short_key_call(d) && !q_from_partials;
     const int ns = short_keys ? 1 : choose_splits(d);
     // one workgroup per 16-row query block: no key split, and a grid of
     // 80-row chunks that would leave CUs idle
@@ -1592,15 +1631,15 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
     const bool qblocks = !short_keys && ns == 1 && d->in_dtype != SF_F32 && d->Sk <= kQGroupMaxKeys &&
                          bh * query_chunks(d) < kNumCUs;
     const int nqc = qblocks ? (d->Sq + 15) / 16 : query_chunks(d);
-    if (q_from_partials && !qblocks) return SF_ENOTSUP;
+    if (d->q_partials && !qblocks) return SF_ENOTSUP;
     sfk::AttnArgs a{};
     a.q = static_cast<const uint16_t*>(q_from_partials && !q ? k : q);   // not read with partials
     if (q_from_partials) {
-        a.qp = d->q_partials;
-        a.q_splits = d->q_splits;
-        a.qp_bytes = (uint32_t)((int64_t)d->q_splits * d->B * d->Sq * d->H * 64 * 4);
-        a.q_bias = d->q_bias;
-        a.q_scale = d->q_scale;
+        a.qp = qpart;
+        a.q_splits = qsplits;
+        a.qp_bytes = (uint32_t)((int64_t)qsplits * d->B * d->Sq * d->H * 64 * 4);
+        a.q_bias = d->q_partials ? d->q_bias : nullptr;
+        a.q_scale = d->q_partials ? d->q_scale : nullptr;
     }
     a.q_gamma = d->q_gamma;
     a.q_eps = d->q_eps;
@@ -1624,6 +1663,7 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
     a.nsplit = ns;
     a.nqc = nqc;
     a.out_kind = d->out_dtype == SF_F32 ? sfk::kOutF32 : (d->out_dtype == SF_F16 ? sfk::kOutF16 : sfk::kOutBF16);
+    a.o_frag = d->o_frag != 0;
     a.causal = d->is_causal != 0;
     const float scale = d->scale != 0.f ? d->scale : 1.f / sqrtf((float)d->D);
     a.scale_log2 = scale * 1.4426950408889634f;
@@ -1660,10 +1700,12 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
             const long groups = (bh + 7) / 8;
             if (8L * nqc * groups > 0x7fffffffL) return SF_ENOTSUP;
             const dim3 grid((unsigned)(8L * nqc * groups));
-            if (q_from_partials) launch_ring_qp(d->exact_pv != 0, vh, grid, s, a);
+            if (q_from_partials) launch_ring_qp<1, 8>(d->exact_pv != 0, vh, grid, s, a);
             else launch_ring<1>(d->exact_pv != 0, f16, vh, grid, s, a);
         } else {
-            launch_ring<sfk::kQB>(d->exact_pv != 0, f16, vh, dim3(ns * nqc, d->H, d->B), s, a);
+            const dim3 grid(ns * nqc, d->H, d->B);
+            if (q_from_partials) launch_ring_qp<sfk::kQB, 1>(d->exact_pv != 0, vh, grid, s, a);
+            else launch_ring<sfk::kQB>(d->exact_pv != 0, f16, vh, grid, s, a);
         }
     }
     if (hipGetLastError() != hipSuccess) return SF_ELAUNCH;

@@ -102,6 +102,12 @@ __device__ __forceinline__ float deferred_affine(float v, float wscale, float rs
     return __builtin_fmaf(v * wscale, rs, bias);
 }
 
+// Element offset of (row, col .. col + 3), col a multiple of 4, in a
+// fragment-ordered [rows][cols] matrix of 16-bit elements (sf_hip.h).
+__device__ __forceinline__ int64_t frag_off(int row, int col, int cols) {
+    return (((int64_t)(row >> 4) * (cols >> 5) + (col >> 5)) * 64 + ((col >> 3) & 3) * 16 + (row & 15)) * 8 + (col & 7);
+}
+
 __device__ __forceinline__ float fast_exp2(float x) {
     return __builtin_amdgcn_exp2f(x);
 }

@@ -1,0 +1,693 @@
+// Fragment-ordered projections for the denoise loop's few rows (gfx950).
+//
+// Replaces, for the block projections of a model step with at most 160 rows
+// (batch 1 and 2), gemm_bias_act (src/backend/cuda/cuda_backend.cu:337-467)
+// with the ops around it -- split_qkv + apply_qk_norm, the residual add and
+// the RMSNorm that follows (dit_block.cu:198-387) -- by ONE launch per
+// projection.
+//
+// Fragment order.  A matrix X[R][K] of 16-bit elements is stored as 1 KB
+// blocks of 16 rows x 32 columns, block (r / 16, k / 32) at index
+// (r / 16) * (K / 32) + k / 32, and inside a block lane l = 16 ((k % 32) / 8)
+// + r % 16 of a wave holds the 8 elements k % 8: exactly the operand of one
+// v_mfma_f32_16x16x32.  int8 codes: blocks of 16 rows x 64 columns, lane l
+// holds the 8 codes of step 64 kc + 8 (l / 16) .. + 7 and the 8 of the step
+// 32 columns further.  So an operand load of a wave is 1 KB of contiguous
+// memory.  Read from row-major rows the same operand is 16 pieces of 64
+// bytes, and each piece costs the address path what a whole 128-byte line
+// does: the same kernel over the same bytes took 9.7 us row-major and
+// 5.9 us in fragment order (67 x 2048 x 2048, cold weights, graph-timed).
+//
+// At that rate one workgroup can afford all of K, so there are no K-slice
+// partials to write, flush and read back and no reduce launch.  Graph-timed on
+// cold weights, 67 rows: 2048 x 2048 6.0-6.2 us with any epilogue against 7.3
+// for split-K + the plain reduce, 8.5 for its deferred and 10.0 for its
+// row-wide residual add + RMSNorm; the 6144 x 2048 QKV projection 10.7 against
+// 14.3.  The batch-1 loop went from 11.3 to 9.4 ms.  An empty launch takes
+// 1.65 us, the weights 1.5 us at the rate a large read reaches; with everything
+// in L2 the 2048 x 2048 call takes 4.4 us.
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "sf_act.h"
+#include "sf_device.h"
+#include "sf_hip.h"
+
+namespace sfk {
+
+constexpr int kFragWaves = 4;
+constexpr int kFragMaxRows = 160;
+constexpr int kFragRowTiles = 64;   // tile sums of a deferred row: 16 in each of 4 lane groups
+
+// The epilogue's arguments (the operands' pointers and sizes are scalar kernel
+// arguments of their own, see gemm_frag_kernel).
+struct FragEpi {
+    const float* bias;     // [N] or null
+    const float* w_scale;  // [N] (int8 weights)
+    int N;
+    int act;
+    int c_kind;            // plain: 0 fp32, 1 bf16, 2 fp16
+    int c_frag;            // plain: fragment order (16-bit), else row-major [M][ldc]
+    int accumulate;        // plain: fp32 c += result
+    void* c;               // plain output; the residual of the add + norm
+    int64_t ldc;
+    // residual add + deferred RMSNorm: c (fp32) += result; norm_out (fragment
+    // order) = c * gamma; norm_ss[m][tile] = the tile's sum of c^2
+    const float* norm_gamma;
+    uint16_t* norm_out;
+    float* norm_ss;
+    int norm_f16;
+    // per-head
+    int H, S;
+    float eps;
+    const float* head_gamma[3];
+    uint16_t* head_out[3];
+    int64_t head_sb[3], head_sh[3], head_ss[3];
+};
+
+__device__ __forceinline__ uint2 pack_kind4(f32x4 v, bool f16) {
+    return f16 ? uint2{pack_f16x2_rn(v[0], v[1]), pack_f16x2_rn(v[2], v[3])}
+               : uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+// Sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 that share an MFMA column.
+__device__ __forceinline__ float sum_groups(float x) {
+    auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// One workgroup of 4 waves per (16 NB columns x 16 MB rows) of C over all of
+// K: wave w contracts its quarter of K (whole 64-wide chunks) with both
+// operands loaded straight into registers -- nothing is shared between waves,
+// so nothing is staged -- two groups of U chunks in flight, and the four
+// waves' fp32 accumulators meet in LDS behind one barrier.  C^T = W . A^T, so
+// weight rows are MFMA rows: accumulator [nb][mb] holds column 16 nb + 4 g + i
+// and row 16 mb + r in lane 16 g + r.  Wave w then finishes the row blocks
+// mb = w, w + 4, ...: the four sums in wave order, scale, the deferred norm's
+// row scale, bias, activation and the epilogue, whose operands were loaded
+// ahead of the contraction.
+//
+// What bounds it: the rate at which a CU fetches operands that come from the
+// L2 and the memory-side cache (50-75 GB/s), so the tile is chosen for few
+// bytes per CU (frag_tile) and the row splits of a column tile run on one XCD
+// (workgroup ids congruent mod 8), whose L2 then serves the weights to all but the first.
+//
+// The operands' pointers and the sizes are separate scalar arguments at the
+// front: those are preloaded into SGPRs with the wave
+// (-amdgpu-kernarg-preload-count), so the first loads go out without a
+// scalar-memory round trip; the epilogue's arguments are fetched behind them.
+template <int NB, int MB, int U, bool W8, bool AH, int EPI, bool RS>
+__global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu(1, 2))) void gemm_frag_kernel(
+    const void* A, const void* W, int K, int M, int ntiles, const float* row_ss, int row_tiles, float row_inv_n,
+    float row_eps, const FragEpi e) {
+    static_assert(EPI != SF_EPI_HEADS || NB == 4, "a head is one column tile");
+    constexpr int NW = kFragWaves;
+    constexpr int WL = W8 ? NB : 2 * NB;   // weight loads per 64-wide chunk
+    constexpr bool kAddNorm = EPI == SF_EPI_ADD_NORM, kHeads = EPI == SF_EPI_HEADS, kPlain = EPI == SF_EPI_PLAIN;
+    __shared__ __attribute__((aligned(16))) f32x4 red[NW * NB * MB * 64];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int g4 = lane >> 4, r = lane & 15;
+    const int ms = (int)blockIdx.x >> 3;
+    const int tile = ((int)blockIdx.x & 7) + 8 * (int)blockIdx.y;
+    if (tile >= ntiles) return;   // the last group of 8 tiles is padded
+    const int n0 = tile * 16 * NB, m0 = ms * 16 * MB;
+    const int rows16 = min((M + 15) / 16 - ms * MB, MB) * 16;   // stored rows of this tile
+    const __amdgpu_buffer_rsrc_t ars =
+        make_rsrc(static_cast<const char*>(A) + (int64_t)m0 * K * 2, (uint32_t)(rows16 * K * 2));
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(static_cast<const char*>(W) + (int64_t)n0 * K * (W8 ? 1 : 2),
+                                                 (uint32_t)(16 * NB * K * (W8 ? 1 : 2)));
+    const int nd = K >> 6;                       // 64-wide chunks
+    const int per = (nd + NW - 1) / NW;
+    const int cb = w * per, ce = min(nd, cb + per);
+
+    // RS: the rows' tile sums, row-major so that lane group g4 fetches tiles
+    // 16 q + 4 g4 .. + 3 of row r as 16 bytes (q < 4).  Loaded ahead of the
+    // operands, so the row scale is formed while the weights are under way.
+    auto load_row = [&](int m, bool on, f32x4 (&v)[kFragRowTiles / 16]) {
+        const __amdgpu_buffer_rsrc_t rrs = make_rsrc(row_ss, (uint32_t)(row_tiles * M * 4));
+#pragma unroll
+        for (int q = 0; q < kFragRowTiles / 16; ++q) {
+            const int t = 16 * q + 4 * g4;
+            const uint32_t off = on && t < row_tiles ? (uint32_t)((m * row_tiles + t) * 4) : 0x80000000u;
+            v[q] = __builtin_bit_cast(f32x4, buffer_load16(rrs, off));
+        }
+    };
+    auto row_scale = [&](f32x4 (&v)[kFragRowTiles / 16]) {
+        if (row_tiles & 3) {   // the last quad runs into the next row
+#pragma unroll
+            for (int q = 0; q < kFragRowTiles / 16; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[q][i] = 16 * q + 4 * g4 + i < row_tiles ? v[q][i] : 0.f;
+        }
+        const f32x4 t = (v[0] + v[1]) + (v[2] + v[3]);
+        return deferred_rsqrt(sum_groups((t[0] + t[1]) + (t[2] + t[3])), row_inv_n, row_eps);
+    };
+    const int mrow = m0 + 16 * w + r;      // this lane's row of the wave's first row block
+    f32x4 rss[kFragRowTiles / 16];
+    if constexpr (RS) load_row(mrow, w < MB && mrow < M, rss);
+
+    u32x4 wv[2][U][WL], av[2][U][2 * MB];
+    // One group of U chunks; chunks past ce load zeros (beyond the buffer
+    // range, no traffic).  Always issued, so that the count of loads in
+    // flight is known and each wait covers one operand at a time.
+    auto issue_w = [&](int c0, u32x4 (&ww)[U][WL]) {
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+            const uint32_t off = (uint32_t)(lane * 16) | (c0 + t < ce ? 0u : 0x80000000u);
+            const int c = c0 + t < ce ? c0 + t : 0;
+#pragma unroll
+            for (int i = 0; i < WL; ++i) {
+                const int blk = W8 ? i * nd + c : (i >> 1) * 2 * nd + 2 * c + (i & 1);
+                ww[t][i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, off, blk * 1024, 0);
+            }
+        }
+    };
+    auto issue_a = [&](int c0, u32x4 (&aa)[U][2 * MB]) {
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+            const uint32_t off = (uint32_t)(lane * 16) | (c0 + t < ce ? 0u : 0x80000000u);
+            const int c = c0 + t < ce ? c0 + t : 0;
+#pragma unroll
+            for (int i = 0; i < 2 * MB; ++i)
+                aa[t][i] = __builtin_amdgcn_raw_buffer_load_b128(ars, off, ((i >> 1) * 2 * nd + 2 * c + (i & 1)) * 1024, 0);
+        }
+    };
+    f32x4 acc[NB][MB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mm = [&](const u32x4 (&ww)[U][WL], const u32x4 (&aa)[U][2 * MB]) {
+#pragma unroll
+        for (int t = 0; t < U; ++t)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                u32x4 wf[NB];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    if constexpr (W8) {
+                        const uint2 q = {ww[t][nb][2 * s], ww[t][nb][2 * s + 1]};
+                        if constexpr (AH) wf[nb] = __builtin_bit_cast(u32x4, i8x8_to_f16x8(q));
+                        else wf[nb] = __builtin_bit_cast(u32x4, i8x8_to_bf16x8(q));
+                    } else {
+                        wf[nb] = ww[t][2 * nb + s];
+                    }
+                }
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        if constexpr (AH)
+                            acc[nb][mb] = mfma16x16x32_f16(u32x4_as_f16x8(wf[nb]), u32x4_as_f16x8(aa[t][2 * mb + s]), acc[nb][mb]);
+                        else
+                            acc[nb][mb] = mfma16x16x32(u32x4_as_bf16x8(wf[nb]), u32x4_as_bf16x8(aa[t][2 * mb + s]), acc[nb][mb]);
+                    }
+            }
+    };
+    // Weights first: they come from HBM; the epilogue's operands and the
+    // activations, from the L2 or the memory-side cache, while the weights
+    // are under way.  (The barriers: the compiler would sink the loads next
+    // to their uses.)
+    issue_w(cb, wv[0]);
+    issue_w(cb + U, wv[1]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the epilogue's operands for this wave's first row block
+    f32x4 bias[NB], scale[NB], res[NB], gam[NB];
+    const bool need_res = kAddNorm || (kPlain && e.accumulate);
+    {
+        const __amdgpu_buffer_rsrc_t brs = make_rsrc(e.bias, e.bias ? (uint32_t)(e.N * 4) : 0u);
+        const __amdgpu_buffer_rsrc_t srs = make_rsrc(e.w_scale, W8 ? (uint32_t)(e.N * 4) : 0u);
+        const __amdgpu_buffer_rsrc_t xrs = make_rsrc(static_cast<const char*>(e.c) + (need_res ? (int64_t)m0 * e.ldc * 4 : 0),
+                                                     need_res && w < MB ? (uint32_t)(min(16 * MB, M - m0) * e.ldc * 4) : 0u);
+        const __amdgpu_buffer_rsrc_t grs = make_rsrc(e.norm_gamma, kAddNorm ? (uint32_t)(e.N * 4) : 0u);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int n = n0 + 16 * nb + 4 * g4;
+            bias[nb] = __builtin_bit_cast(f32x4, buffer_load16(brs, (uint32_t)(n * 4)));
+            scale[nb] = W8 ? __builtin_bit_cast(f32x4, buffer_load16(srs, (uint32_t)(n * 4))) : f32x4{1.f, 1.f, 1.f, 1.f};
+            if constexpr (kAddNorm) gam[nb] = __builtin_bit_cast(f32x4, buffer_load16(grs, (uint32_t)(n * 4)));
+            if constexpr (kAddNorm || kPlain)
+                res[nb] = __builtin_bit_cast(f32x4, buffer_load16(xrs, (uint32_t)(((16 * w + r) * e.ldc + n) * 4)));
+        }
+    }
+    issue_a(cb, av[0]);
+    issue_a(cb + U, av[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    float rs = 1.f;
+    if constexpr (RS) rs = row_scale(rss);
+
+    int c0 = cb;
+    for (; c0 + 2 * U < ce; c0 += 2 * U) {
+        mm(wv[0], av[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_w(c0 + 2 * U, wv[0]);
+        issue_a(c0 + 2 * U, av[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(wv[1], av[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_w(c0 + 3 * U, wv[1]);
+        issue_a(c0 + 3 * U, av[1]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    mm(wv[0], av[0]);
+    mm(wv[1], av[1]);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) red[((w * MB + mb) * NB + nb) * 64 + lane] = acc[nb][mb];
+    __syncthreads();
+
+    for (int mb = w; mb < MB; mb += NW) {
+        const int m = m0 + 16 * mb + r;
+        f32x4 v[NB];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            v[nb] = red[(mb * NB + nb) * 64 + lane];
+#pragma unroll
+            for (int s = 1; s < NW; ++s) v[nb] += red[((s * MB + mb) * NB + nb) * 64 + lane];
+        }
+        if (MB > NW && mb != w) {   // a second row block: its residual and row sums
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                if (need_res && m < M)
+                    res[nb] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(e.c) + (int64_t)m * e.ldc + n0 +
+                                                              16 * nb + 4 * g4);
+            if constexpr (RS) {
+                load_row(m, m < M, rss);
+                rs = row_scale(rss);
+            }
+        }
+        if constexpr (RS) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[nb][j] = deferred_affine(v[nb][j], scale[nb][j], rs, bias[nb][j]);
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[nb][j] = v[nb][j] * scale[nb][j] + bias[nb][j];
+        }
+        if constexpr (kHeads) {
+            const int cols = e.H * 64;
+            const int sec = n0 / cols, h = (n0 % cols) / 64;
+            const float* gamma = e.head_gamma[sec];
+            if (gamma) {   // rms_norm_kernel_impl over the 64 head dims (norm.cuh:89-122)
+                float ss = 0.f;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) ss += v[nb][j] * v[nb][j];
+                const float inv_rms = 1.f / sqrtf(sum_groups(ss) / 64.f + e.eps);
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    const f32x4 gq = *reinterpret_cast<const f32x4*>(gamma + 16 * nb + 4 * g4);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[nb][j] = v[nb][j] * inv_rms * gq[j];
+                }
+            }
+            if (m >= M) continue;
+            uint16_t* o = e.head_out[sec] + (int64_t)(m / e.S) * e.head_sb[sec] + h * e.head_sh[sec] +
+                          (int64_t)(m % e.S) * e.head_ss[sec];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                *reinterpret_cast<uint2*>(o + 16 * nb + 4 * g4) = pack_kind4(v[nb], false);
+        } else if constexpr (kAddNorm) {
+            float ss = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                v[nb] += res[nb];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ss += v[nb][j] * v[nb][j];
+            }
+            ss = sum_groups(ss);
+            if (m >= M) continue;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const int n = n0 + 16 * nb + 4 * g4;
+                *reinterpret_cast<f32x4*>(static_cast<float*>(e.c) + (int64_t)m * e.ldc + n) = v[nb];
+                *reinterpret_cast<uint2*>(e.norm_out + frag_off(m, n, e.N)) = pack_kind4(v[nb] * gam[nb], e.norm_f16 != 0);
+            }
+            if (g4 == 0) e.norm_ss[(int64_t)m * ntiles + tile] = ss;
+        } else {
+            if (m >= M) continue;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const int n = n0 + 16 * nb + 4 * g4;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[nb][j] = apply_act(e.act, v[nb][j]);
+                if (e.c_frag) {
+                    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(e.c) + frag_off(m, n, e.N)) = pack_kind4(v[nb], e.c_kind == 2);
+                } else if (e.c_kind == 0) {
+                    *reinterpret_cast<f32x4*>(static_cast<float*>(e.c) + (int64_t)m * e.ldc + n) =
+                        e.accumulate ? res[nb] + v[nb] : v[nb];
+                } else {
+                    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(e.c) + (int64_t)m * e.ldc + n) = pack_kind4(v[nb], e.c_kind == 2);
+                }
+            }
+        }
+    }
+}
+
+// RMSNorm of fp32 rows into fragment order, one workgroup of 256 threads per
+// row (rms_norm_kernel_impl, norm.cuh:89-122).  Thread t owns columns
+// 8 t .. 8 t + 7 (and 2048 further), one 16-byte store each.  ss != null: the
+// deferred form instead -- x * gamma, and ss[row][t] = the sum of x^2 over the
+// 64 columns of tile t.
+constexpr int kNormFragPer = 2;   // cols <= 2 * 256 * 8 = 4096
+__global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t ldx, const float* gamma, uint16_t* out,
+                                                        int f16, float* ss, int cols, float eps) {
+    __shared__ float red[4];
+    const int row = blockIdx.x;
+    f32x4 v[kNormFragPer][2], gq[kNormFragPer][2];
+    float sum[kNormFragPer];
+#pragma unroll
+    for (int i = 0; i < kNormFragPer; ++i) {
+        const int c = 8 * ((int)threadIdx.x + 256 * i);
+        sum[i] = 0.f;
+        if (c < cols) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v[i][h] = *reinterpret_cast<const f32x4*>(x + row * ldx + c + 4 * h);
+                gq[i][h] = *reinterpret_cast<const f32x4*>(gamma + c + 4 * h);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum[i] += v[i][h][j] * v[i][h][j];
+        }
+    }
+    float s = 1.f;
+    if (ss) {   // 8 lanes hold a 64-column tile
+#pragma unroll
+        for (int i = 0; i < kNormFragPer; ++i) {
+            float t = sum[i];
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) t += __shfl_xor(t, off, 64);
+            const int c = 8 * ((int)threadIdx.x + 256 * i);
+            if (c < cols && (threadIdx.x & 7) == 0) ss[(int64_t)row * (cols / 64) + c / 64] = t;
+        }
+    } else {
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < kNormFragPer; ++i) t += sum[i];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+        __syncthreads();
+        s = 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)cols + eps);
+    }
+#pragma unroll
+    for (int i = 0; i < kNormFragPer; ++i) {
+        const int c = 8 * ((int)threadIdx.x + 256 * i);
+        if (c < cols) {
+            const uint2 lo = pack_kind4(v[i][0] * s * gq[i][0], f16 != 0);
+            const uint2 hi = pack_kind4(v[i][1] * s * gq[i][1], f16 != 0);
+            *reinterpret_cast<u32x4*>(out + frag_off(row, c, cols)) = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+    }
+}
+
+// Weight copies in fragment order: 16 bytes of the copy per thread, bf16 kept
+// or rounded to the nearest fp16 (as sf_weights_to_f16 rounds), int8 codes
+// kept.  The reads of 16 rows x 64 bytes are gathered by one wave.
+struct FragJobs {
+    const void* w[SF_CODES_MAX_JOBS];
+    void* out[SF_CODES_MAX_JOBS];
+    int64_t ldw[SF_CODES_MAX_JOBS];
+    int32_t K[SF_CODES_MAX_JOBS];
+    int32_t kind[SF_CODES_MAX_JOBS];   // 0 copy 16-bit, 1 bf16 -> fp16, 2 int8
+    uint32_t start[SF_CODES_MAX_JOBS + 1];
+    int32_t count;
+};
+
+__global__ __launch_bounds__(256) void frag_pack_kernel(const FragJobs J) {
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= J.start[J.count]) return;
+    int j = 0;
+#pragma unroll
+    for (int i = 1; i < SF_CODES_MAX_JOBS; ++i)
+        if (i < J.count && idx >= J.start[i]) j = i;
+    const uint32_t local = idx - J.start[j];
+    const uint32_t lane = local & 63u, blk = local >> 6;
+    const bool i8 = J.kind[j] == 2;
+    const uint32_t kc = (uint32_t)J.K[j] / (i8 ? 64u : 32u);
+    const uint32_t rb = blk / kc, c = blk - rb * kc;
+    const int64_t row = 16 * (int64_t)rb + (lane & 15u);
+    const uint32_t g4 = lane >> 4;
+    u32x4 o;
+    if (i8) {
+        const int8_t* src = static_cast<const int8_t*>(J.w[j]) + row * J.ldw[j] + 64u * c + 8u * g4;
+        const uint2 lo = *reinterpret_cast<const uint2*>(src), hi = *reinterpret_cast<const uint2*>(src + 32);
+        o = u32x4{lo.x, lo.y, hi.x, hi.y};
+    } else {
+        o = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(J.w[j]) + row * J.ldw[j] + 32u * c + 8u * g4);
+        if (J.kind[j] == 1) o = __builtin_bit_cast(u32x4, bf16x8_to_f16x8(o));
+    }
+    *(static_cast<u32x4*>(J.out[j]) + local) = o;
+}
+
+// Tile of a call: NB (16-column blocks: 2 or 4) and MB (16-row blocks: 2, 3
+// or 5).  A CU runs one workgroup at a time and the time follows the operand
+// bytes it fetches, (NB + MB) * 32 K per workgroup, so the smallest
+// rounds-of-256-workgroups * (NB + MB) is taken, on a tie the smaller MB.
+// Graph-timed, cold weights, K = 2048, while the kernel was a probe: 67 x 2048
+// (2, 2) 5.9 us against 7.0 for (2, 3) and 8.5 for (4, 2); 134 x 2048 (2, 3)
+// 7.4 against 9.7 for (2, 2); 67 x 6144 (4, 3) 11.3 against 14.2 for (4, 2)
+// and 14.6 for (4, 5); 134 x 6144 (4, 5) 14.4 against 14.8 for (4, 2) and 19.2
+// for (4, 3).
+struct FragTile {
+    int nb = 0, mb = 0, ntiles = 0, nms = 0;
+};
+FragTile frag_tile(int M, int N, int nb_only) {
+    FragTile best;
+    long cost = 0;
+    for (int nb : {2, 4}) {
+        if ((nb_only && nb != nb_only) || N % (16 * nb)) continue;
+        for (int mb : {2, 3, 5}) {
+            const int nt = N / (16 * nb), nms = (M + 16 * mb - 1) / (16 * mb);
+            const long c = ((long)nt * nms + 255) / 256 * (nb + mb);
+            if (!best.nb || c < cost) {
+                best.nb = nb;
+                best.mb = mb;
+                best.ntiles = nt;
+                best.nms = nms;
+                cost = c;
+            }
+        }
+    }
+    return best;
+}
+
+struct FragOps {
+    const void* a;
+    const void* w;
+    int K, M;
+    bool w8, ah;
+    // the rows of a hold x * gamma of a deferred norm
+    const float* row_ss;
+    int row_tiles;
+    float row_inv_n, row_eps;
+};
+
+template <int NB, int MB, int U, int EPI, bool RS>
+void launch_frag_rs(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
+    const dim3 grid(8u * (unsigned)t.nms, (unsigned)((t.ntiles + 7) / 8)), block(64 * kFragWaves);
+    if (o.w8) {
+        if (o.ah) hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, true, true, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
+        else hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, true, false, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
+    } else {
+        if (o.ah) hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, false, true, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
+        else hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, false, false, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
+    }
+}
+
+template <int NB, int MB, int U, int EPI>
+void launch_frag_tile(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
+    if constexpr (EPI != SF_EPI_ADD_NORM) {
+        if (o.row_ss) {
+            launch_frag_rs<NB, MB, U, EPI, true>(o, t, e, s);
+            return;
+        }
+    }
+    launch_frag_rs<NB, MB, U, EPI, false>(o, t, e, s);
+}
+
+// U chunks per group: the loads of two groups about fill the wave's 63-entry
+// load counter.
+template <int EPI>
+void launch_frag(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
+    if constexpr (EPI != SF_EPI_HEADS) {
+        if (t.nb == 2) {
+            if (t.mb == 2) launch_frag_tile<2, 2, 4, EPI>(o, t, e, s);
+            else if (t.mb == 3) launch_frag_tile<2, 3, 2, EPI>(o, t, e, s);
+            else launch_frag_tile<2, 5, 2, EPI>(o, t, e, s);
+            return;
+        }
+    }
+    if (t.mb == 2) launch_frag_tile<4, 2, 2, EPI>(o, t, e, s);
+    else if (t.mb == 3) launch_frag_tile<4, 3, 2, EPI>(o, t, e, s);
+    else launch_frag_tile<4, 5, 1, EPI>(o, t, e, s);
+}
+
+}  // namespace sfk
+
+namespace {
+bool fal16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Columns per tile sum of the deferred add + norm epilogue: 32, or 64 where
+// 32 would give a row more than kFragRowTiles sums.
+int norm_nb(int N) { return N <= 32 * sfk::kFragRowTiles ? 2 : 4; }
+}  // namespace
+
+extern "C" size_t sf_frag_elems(int64_t rows, int64_t cols) {
+    return rows > 0 && cols > 0 ? (size_t)((rows + 15) / 16 * 16) * (size_t)cols : 0;
+}
+
+extern "C" int32_t sf_gemm_frag_ss_tiles(int32_t N) {
+    if (N <= 0) return 0;
+    const int cols = 16 * norm_nb(N);
+    return N % cols ? 0 : N / cols;
+}
+
+extern "C" int sf_frag_pack(const sf_frag_job* jobs, int32_t count, void* stream) {
+    if (count == 0) return SF_OK;
+    if (!jobs || count < 0 || count > SF_CODES_MAX_JOBS) return SF_EINVAL;
+    sfk::FragJobs J{};
+    J.count = count;
+    uint64_t total = 0;
+    for (int j = 0; j < count; ++j) {
+        const sf_frag_job& b = jobs[j];
+        if (b.N < 0 || b.K < 0) return SF_EINVAL;
+        const bool i8 = b.w_dtype == SF_I8 && b.out_dtype == SF_I8;
+        const bool same = (b.w_dtype == SF_BF16 || b.w_dtype == SF_F16) && b.out_dtype == b.w_dtype;
+        const bool cvt = b.w_dtype == SF_BF16 && b.out_dtype == SF_F16;
+        if (!i8 && !same && !cvt) return SF_ENOTSUP;
+        J.start[j] = (uint32_t)total;
+        if ((int64_t)b.N * b.K == 0) continue;
+        // rows of 16-byte (int8: 8-byte) aligned pieces
+        if (!b.w || !b.out || !fal16(b.w) || !fal16(b.out) || (b.N & 15) || (b.K & 63) || b.ldw < b.K || (b.ldw & 7))
+            return SF_EINVAL;
+        J.w[j] = b.w;
+        J.out[j] = b.out;
+        J.ldw[j] = b.ldw;
+        J.K[j] = b.K;
+        J.kind[j] = i8 ? 2 : (cvt ? 1 : 0);
+        total += (uint64_t)b.N * (uint64_t)b.K / (i8 ? 16 : 8);
+        if (total >= 0x7fffff00ull) return SF_ENOTSUP;   // 32-bit thread indices
+    }
+    J.start[count] = (uint32_t)total;
+    if (total == 0) return SF_OK;
+    hipLaunchKernelGGL(sfk::frag_pack_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), J);
+    return hipGetLastError() == hipSuccess ? SF_OK : SF_ELAUNCH;
+}
+
+extern "C" int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int32_t out_dtype, float* ss,
+                            int32_t rows, int32_t cols, float eps, void* stream) {
+    if (rows < 0 || cols < 0) return SF_EINVAL;
+    if ((long)rows * cols == 0) return SF_OK;
+    if (!x || !gamma || !out || ldx < cols) return SF_EINVAL;
+    if (out_dtype != SF_BF16 && out_dtype != SF_F16) return SF_ENOTSUP;
+    if ((cols & 63) || cols > 2048 * sfk::kNormFragPer) return SF_ENOTSUP;
+    if ((ldx & 3) || !fal16(x) || !fal16(gamma) || !fal16(out)) return SF_EINVAL;
+    hipLaunchKernelGGL(sfk::norm_frag_kernel, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream), x, ldx, gamma,
+                       static_cast<uint16_t*>(out), out_dtype == SF_F16 ? 1 : 0, ss, cols, eps);
+    return hipGetLastError() == hipSuccess ? SF_OK : SF_ELAUNCH;
+}
+
+extern "C" int sf_gemm_frag(const sf_frag_gemm_desc* d, void* stream) {
+    if (!d) return SF_EINVAL;
+    if (d->M < 0 || d->N < 0 || d->K < 0) return SF_EINVAL;
+    if ((long)d->M * d->N == 0) return SF_OK;
+    if (d->M > sfk::kFragMaxRows || d->K == 0 || (d->K & 63) || d->K > (1 << 20) || (d->N & 31)) return SF_ENOTSUP;
+    if (d->a_dtype != SF_BF16 && d->a_dtype != SF_F16) return SF_ENOTSUP;
+    if (d->w_dtype != d->a_dtype && d->w_dtype != SF_I8) return SF_ENOTSUP;
+    if (d->act < 0 || d->act > 2 || (d->act && d->epilogue != SF_EPI_PLAIN)) return SF_EINVAL;
+    if (d->a_row_ss && d->epilogue == SF_EPI_ADD_NORM) return SF_EINVAL;
+    if (!d->A || !d->W || !fal16(d->A) || !fal16(d->W)) return SF_EINVAL;
+    const bool w8 = d->w_dtype == SF_I8;
+    if (w8 && (!d->w_scale || !fal16(d->w_scale))) return SF_EINVAL;
+    if (!fal16(d->bias)) return SF_EINVAL;
+    if ((int64_t)d->N * 4 > 0x7fffffffLL) return SF_ENOTSUP;
+    sfk::FragOps o{d->A, d->W, d->K, d->M, w8, d->a_dtype == SF_F16, nullptr, 0, 0.f, 0.f};
+    sfk::FragEpi a{};
+    a.w_scale = w8 ? d->w_scale : nullptr;
+    a.bias = d->bias;
+    a.N = d->N;
+    a.act = d->act;
+    if (d->a_row_ss) {
+        if (d->a_row_tiles < 1 || d->a_row_tiles > sfk::kFragRowTiles || d->a_row_n <= 0 || !(d->a_row_eps >= 0.f))
+            return SF_EINVAL;
+        o.row_ss = d->a_row_ss;
+        o.row_tiles = d->a_row_tiles;
+        o.row_inv_n = 1.f / (float)d->a_row_n;
+        o.row_eps = d->a_row_eps;
+    }
+    int nb = 0;   // columns per tile where the epilogue fixes them
+    if (d->epilogue == SF_EPI_HEADS) {
+        if (d->H <= 0 || d->S <= 0) return SF_EINVAL;
+        const int cols = d->H * 64;
+        if (d->N % cols || d->N / cols > 3) return SF_EINVAL;
+        for (int j = 0; j < d->N / cols; ++j) {
+            if (!d->head_out[j] || (reinterpret_cast<uintptr_t>(d->head_out[j]) & 7) || !fal16(d->head_gamma[j]))
+                return SF_EINVAL;
+            for (int q = 0; q < 3; ++q)
+                if (d->head_stride[j][q] & 3) return SF_EINVAL;
+            a.head_out[j] = static_cast<uint16_t*>(d->head_out[j]);
+            a.head_gamma[j] = d->head_gamma[j];
+            a.head_sb[j] = d->head_stride[j][0];
+            a.head_sh[j] = d->head_stride[j][1];
+            a.head_ss[j] = d->head_stride[j][2];
+        }
+        a.H = d->H;
+        a.S = d->S;
+        a.eps = d->eps;
+        nb = 4;
+    } else if (d->epilogue == SF_EPI_ADD_NORM) {
+        if (!d->C || !fal16(d->C) || d->ldc < d->N || (d->ldc & 3) || d->c_dtype != SF_F32) return SF_EINVAL;
+        if (!d->norm_gamma || !fal16(d->norm_gamma) || !d->norm_out || !fal16(d->norm_out) || !d->norm_ss) return SF_EINVAL;
+        if (d->norm_dtype != SF_BF16 && d->norm_dtype != SF_F16) return SF_ENOTSUP;
+        const int tiles = sf_gemm_frag_ss_tiles(d->N);
+        if (tiles < 1 || tiles > sfk::kFragRowTiles) return SF_ENOTSUP;
+        a.c = d->C;
+        a.ldc = d->ldc;
+        a.norm_gamma = d->norm_gamma;
+        a.norm_out = static_cast<uint16_t*>(d->norm_out);
+        a.norm_f16 = d->norm_dtype == SF_F16;
+        a.norm_ss = d->norm_ss;
+        nb = norm_nb(d->N);
+    } else if (d->epilogue == SF_EPI_PLAIN) {
+        if (!d->C) return SF_EINVAL;
+        if (d->c_dtype != SF_F32 && d->c_dtype != SF_BF16 && d->c_dtype != SF_F16) return SF_ENOTSUP;
+        if (d->accumulate && (d->c_frag || d->c_dtype != SF_F32)) return SF_EINVAL;
+        if (d->c_frag) {
+            if (d->c_dtype == SF_F32 || !fal16(d->C)) return SF_EINVAL;
+        } else if (d->ldc < d->N || (d->ldc & 3) ||
+                   (reinterpret_cast<uintptr_t>(d->C) & (d->c_dtype == SF_F32 ? 15u : 7u))) {
+            return SF_EINVAL;
+        }
+        a.c = d->C;
+        a.ldc = d->ldc;
+        a.c_kind = d->c_dtype == SF_F32 ? 0 : (d->c_dtype == SF_BF16 ? 1 : 2);
+        a.c_frag = d->c_frag != 0;
+        a.accumulate = d->accumulate != 0;
+    } else {
+        return SF_ENOTSUP;
+    }
+    if (a.c && (int64_t)80 * a.ldc * 4 > 0x7fffffffLL) return SF_ENOTSUP;   // 32-bit residual offsets of a row tile
+    const sfk::FragTile t = sfk::frag_tile(d->M, d->N, nb);
+    if (!t.nb) return SF_ENOTSUP;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (d->epilogue == SF_EPI_HEADS) sfk::launch_frag<SF_EPI_HEADS>(o, t, a, s);
+    else if (d->epilogue == SF_EPI_ADD_NORM) sfk::launch_frag<SF_EPI_ADD_NORM>(o, t, a, s);
+    else sfk::launch_frag<SF_EPI_PLAIN>(o, t, a, s);
+    return hipGetLastError() == hipSuccess ? SF_OK : SF_ELAUNCH;
+}

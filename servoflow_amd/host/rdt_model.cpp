@@ -99,21 +99,18 @@ struct sf_rdt {
     uint16_t* n = nullptr;         // [B*S, D] bf16 norm1 / norm2 / final-norm output
     uint16_t *q = nullptr, *k = nullptr, *v = nullptr;   // [B, H, S, 64]
     // Above 160 rows (the library-path GEMMs) the QKV projection is kept as
-    // its bf16 output [B*S, 3D] and the cross-q projection's as [B*S, D] in
+    // its fp16 output [B*S, 3D] and the cross-q projection's as [B*S, D] in
     // q; the attention reads Q / K / V from those rows and applies q_norm /
-    // k_norm as it loads them (sf_attn_desc.q_gamma / k_gamma) in place of
-    // the per-head epilogue pass.
-    bool rows_qkv = false;
+    // k_norm as it loads them (sf_attn_desc.q_gamma / k_gamma).
     uint16_t* qkv_rows = nullptr;
     uint16_t* a = nullptr;         // [B*S, D] attention output (act16)
     // Element type of the projections' 16-bit inputs.  The FFN's inputs
     // (norm3 output, GELU hidden; ffn_dtype) are fp16 at every batch size
     // (3 more significant bits than bf16 at the same bytes; of the block's
     // 16-bit storage points these two move the block output furthest from
-    // fp32 arithmetic); on the split-K path the fc1 / fc2 weight fragments
-    // are converted to fp16 in registers.  The other inputs -- norm1 /
+    // fp32 arithmetic).  The other inputs -- norm1 /
     // norm2 / final-norm outputs and attention outputs (act16) -- are bf16
-    // while B*S rows fit the split-K regime (<= 160) and fp16 above it,
+    // while B*S rows run fragment-ordered (<= 160) and fp16 above it,
     // where the library path multiplies fp16 activations by fp16 copies of
     // the weights (w16) and keeps its 16-bit products in fp16: with bf16
     // inputs and bf16 products a block sat at 1.6-1.8e-3 from fp32
@@ -124,18 +121,20 @@ struct sf_rdt {
     // long as the model's activations do.
     int32_t ffn_dtype = SF_F16;
     int32_t act16 = SF_BF16;
-    // Deferred RMSNorm (split-K regime, B*S <= 160): the norm1 / norm2
-    // producers -- the entry norm, the fc2 and attention-proj residual adds --
-    // store x * gamma and per-64-column sums of squares (row_ss, [D/64][B*S])
-    // and the consumers (the QKV and cross-q projections, or the language
-    // attention finishing Q from partials) apply the row's 1/rms after their
-    // contraction: every CU takes part in the residual-add kernels, which
-    // otherwise run one workgroup per row.  norm3 and the final norm keep the
-    // row-wide form (their fp16 outputs need the normalised range).
-    // n_deferred: whether n holds deferred rows (set as kernels are enqueued).
-    bool defer = false;
-    bool n_deferred = false;
+    // Fragment-ordered step (B*S <= 160): every block and final-layer
+    // projection is one sf_gemm_frag launch over fragment-ordered weight
+    // copies (frag_of) and activations: n, a, n3 and h are in fragment order.
+    // norm1 / norm2 are deferred: the residual adds before them store
+    // x * gamma and per-tile sums of squares (row_ss, [row_tiles][B*S]), and
+    // the QKV and cross-q projections apply the row's 1/rms after their
+    // contraction.  norm3 and the final norm are row-wide launches of their
+    // own (sf_norm_frag): their fp16 outputs need the normalised range.  The
+    // cross-q projection leaves finished fp32 rows (q32); the attention
+    // applies q_norm as it loads them.
+    bool frag = false;
     float* row_ss = nullptr;
+    int row_tiles = 0;             // tiles of the sums row_ss holds now
+    float* q32 = nullptr;          // [B*S, D] cross-q rows
     void* n3 = nullptr;            // [B*S, D] norm3 output
     void* h = nullptr;             // [B*S, F] FFN hidden
     uint16_t* act_in = nullptr;    // [B*T, 2A]
@@ -174,32 +173,29 @@ struct sf_rdt {
     } kvg[2];
     uint16_t* kv_prod = nullptr;   // [rows][blocks * 2D] bf16 product of a batched group
     size_t kv_prod_bytes = 0;
-    // Language blocks at <= 160 rows: the cross-q projection leaves its
-    // split-K partials (SF_EPI_PARTIALS) and the language attention, on its
-    // query-block grid, finishes Q from them (sum, scale, bias, q_norm) --
-    // one launch less per language block.  cq_splits: the partials' count.
-    int cq_splits = 0;
     void* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
     void* gemm_ws = nullptr;       // split-K partial sums, shared by the stream's GEMMs
     size_t gemm_ws_bytes = 0;
-    // fp16 copies of projection weights (w16_params: above 160 rows every
-    // block's six and the final layer's two; at most 160 rows with bf16
-    // weights the ones multiplying fp16 inputs; int8 codes widened exactly,
-    // bf16 weights rounded to fp16; sf_weights_to_f16, up to eight
-    // matrices per launch), made before the first pass and again before
-    // the first pass after the parameters may have changed (w16_stale), on
+    // Copies of projection weights.  Above 160 rows (w16_params) fp16 copies
+    // of every block's six and the final layer's two (int8 codes widened
+    // exactly, bf16 weights rounded to fp16; sf_weights_to_f16); at most 160
+    // rows (frag_params) fragment-ordered copies of the same matrices in the
+    // type the projection multiplies -- bf16, fp16 for the matrices whose
+    // inputs are fp16 (fc1, fc2, the final fc2), int8 codes (sf_frag_pack).
+    // Up to eight matrices per launch, made before the first pass and again before
+    // the first pass after the parameters may have changed (copies_stale), on
     // the pass's stream and outside any graph capture -- not once per loop:
     // a batch-16 loop refreshing them in its graph took 0.8 ms more.
-    // codes16_of[param] is a weight's copy (fixed at creation).
-    char* codes16 = nullptr;
-    size_t codes16_bytes = 0;
-    std::vector<const void*> codes16_of;
+    // copy_of[param] is a weight's copy (fixed at creation).
+    char* copies = nullptr;
+    size_t copies_bytes = 0;
+    std::vector<void*> copy_of;
     // The copies may no longer match the weights: set by every call that
     // writes parameters or hands out a pointer to them (and by
     // sf_rdt_params_changed), cleared by the refresh at the start of the
     // next pass.
-    bool w16_stale = true;
+    bool copies_stale = true;
 
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -241,7 +237,7 @@ void sf_rdt_set_error(sf_rdt* m, const std::string& msg) {
 void sf_rdt_weights_changed(sf_rdt* m) {
     if (!m) return;
     m->infer_cond_valid = false;
-    m->w16_stale = true;
+    m->copies_stale = true;
 }
 
 extern "C" const char* sf_rdt_last_error(const sf_rdt* m) { return m ? m->last_error.c_str() : ""; }
@@ -382,15 +378,6 @@ bool kv_batched(const sf_rdt* m, int g, int rows) {
            bytes <= m->kv_prod_bytes;
 }
 
-// A as deferred-norm rows (x * gamma with m->row_ss): the output rows get
-// their 1/rms after the product.
-void set_row_scale(const sf_rdt* m, sf_gemm_desc& d) {
-    d.a_row_ss = m->row_ss;
-    d.a_row_tiles = m->cfg.hidden / 64;
-    d.a_row_n = m->cfg.hidden;
-    d.a_row_eps = m->cfg.eps;
-}
-
 int linear(sf_rdt* m, const void* A, int64_t lda, int M, int w_idx, int b_idx, int act, void* C,
            int64_t ldc, int c_dtype, bool accumulate, hipStream_t s, int a_dtype = SF_BF16) {
     const Param& W = m->params[w_idx];
@@ -405,7 +392,7 @@ int linear(sf_rdt* m, const void* A, int64_t lda, int M, int w_idx, int b_idx, i
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->codes16_of[w_idx];
+    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = b_idx >= 0 ? pf(m, b_idx) : nullptr;
     d.act = act;
@@ -424,7 +411,7 @@ int linear(sf_rdt* m, const void* A, int64_t lda, int M, int w_idx, int b_idx, i
 // output is stored in bf16 before the add (round_product), as the
 // reference's projection returns it (dit_block.cu:233, 321, 160).
 int linear_add_norm(sf_rdt* m, const void* A, int a_dtype, int M, int w_idx, int b_idx, int gamma_idx,
-                    void* out, int out_dtype, hipStream_t s, bool deferred = false) {
+                    void* out, int out_dtype, hipStream_t s) {
     const Param& W = m->params[w_idx];
     const int D = m->cfg.hidden;
     sf_gemm_desc d{};
@@ -438,7 +425,7 @@ int linear_add_norm(sf_rdt* m, const void* A, int a_dtype, int M, int w_idx, int
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->codes16_of[w_idx];
+    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = pf(m, b_idx);
     d.epilogue = SF_EPI_ADD_NORM;
@@ -453,7 +440,6 @@ int linear_add_norm(sf_rdt* m, const void* A, int a_dtype, int M, int w_idx, int
     d.workspace = m->gemm_ws;
     d.workspace_bytes = (int64_t)m->gemm_ws_bytes;
     d.round_product = 1;
-    if (deferred) d.norm_ss = m->row_ss;
     return sf_gemm(&d, s);
 }
 
@@ -463,7 +449,7 @@ int linear_add_norm(sf_rdt* m, const void* A, int a_dtype, int M, int w_idx, int
 // (dit_block.cu:207, 284, 291).
 int linear_heads(sf_rdt* m, const void* A, int M, int S, int w_idx, int b_idx,
                  uint16_t* const* outs, const int* gamma_idx, int nsec, hipStream_t s,
-                 int a_dtype = SF_BF16, bool round_product = false, bool a_deferred = false) {
+                 int a_dtype = SF_BF16, bool round_product = false) {
     const Param& W = m->params[w_idx];
     const int H = m->cfg.heads;
     sf_gemm_desc d{};
@@ -477,7 +463,7 @@ int linear_heads(sf_rdt* m, const void* A, int M, int S, int w_idx, int b_idx,
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->codes16_of[w_idx];
+    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = pf(m, b_idx);
     d.epilogue = SF_EPI_HEADS;
@@ -494,21 +480,85 @@ int linear_heads(sf_rdt* m, const void* A, int M, int S, int w_idx, int b_idx,
     d.workspace = m->gemm_ws;
     d.workspace_bytes = (int64_t)m->gemm_ws_bytes;
     d.round_product = round_product ? 1 : 0;
-    if (a_deferred) set_row_scale(m, d);
     return sf_gemm(&d, s);
 }
 
-// Q of a cross-attention given as the cross-q projection's split-K
-// partials (sf_attn_desc.q_partials); row_ss: their input rows were
-// deferred-norm rows.
-struct QPartials {
-    const float* p = nullptr;
-    int splits = 0;
-    const float* bias = nullptr;
-    const float* scale = nullptr;
-    const float* gamma = nullptr;
-    const float* row_ss = nullptr;
-};
+// ---- fragment-ordered projections (m->frag) ----
+
+// A descriptor over the M = B*S rows of A (fragment order, a_dtype) and the
+// fragment-ordered copy of weight w_idx.  deferred: A holds x * gamma of a
+// deferred norm whose sums are in row_ss.
+sf_frag_gemm_desc frag_desc(const sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, bool deferred) {
+    const Param& W = m->params[w_idx];
+    const sf_rdt_config& c = m->cfg;
+    sf_frag_gemm_desc d{};
+    d.M = c.batch * (c.horizon + 3);
+    d.N = (int32_t)W.shape[0];
+    d.K = (int32_t)W.shape[1];
+    d.A = A;
+    d.a_dtype = a_dtype;
+    d.W = m->copy_of[w_idx];
+    d.w_dtype = W.dtype == SF_I8 ? SF_I8 : a_dtype;
+    d.w_scale = W.scale;
+    d.bias = static_cast<const float*>(m->params[b_idx].data);
+    if (deferred) {
+        d.a_row_ss = m->row_ss;
+        d.a_row_tiles = m->row_tiles;
+        d.a_row_n = c.hidden;
+        d.a_row_eps = c.eps;
+    }
+    return d;
+}
+
+// C = act(A W^T + b): fp32 row-major (accumulate: C +=) or, with frag, in
+// fragment order.
+int frag_linear(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, int act, void* C, int c_dtype,
+                bool c_frag, bool accumulate, hipStream_t s, bool deferred = false) {
+    sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, deferred);
+    d.act = act;
+    d.epilogue = SF_EPI_PLAIN;
+    d.C = C;
+    d.ldc = d.N;
+    d.c_dtype = c_dtype;
+    d.c_frag = c_frag ? 1 : 0;
+    d.accumulate = accumulate ? 1 : 0;
+    return sf_gemm_frag(&d, s);
+}
+
+// x += A W^T + b; m->n = x * gamma (bf16, fragment order), row_ss = the sums.
+int frag_add_norm(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, int gamma_idx, hipStream_t s) {
+    sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, false);
+    d.epilogue = SF_EPI_ADD_NORM;
+    d.C = m->x;
+    d.ldc = d.N;
+    d.c_dtype = SF_F32;
+    d.norm_gamma = pf(m, gamma_idx);
+    d.norm_out = m->n;
+    d.norm_dtype = m->act16;
+    d.norm_ss = m->row_ss;
+    m->row_tiles = sf_gemm_frag_ss_tiles(d.N);
+    return sf_gemm_frag(&d, s);
+}
+
+// q, k (with q_norm / k_norm) and v of the deferred rows m->n, per head.
+int frag_qkv(sf_rdt* m, const LayerIdx& L, hipStream_t s) {
+    const int H = m->cfg.heads, S = m->cfg.horizon + 3;
+    sf_frag_gemm_desc d = frag_desc(m, m->n, m->act16, L.qkv_w, L.qkv_b, true);
+    d.epilogue = SF_EPI_HEADS;
+    d.H = H;
+    d.S = S;
+    d.eps = m->cfg.eps;
+    void* const outs[3] = {m->q, m->k, m->v};
+    const float* const gammas[3] = {pf(m, L.q_norm), pf(m, L.k_norm), nullptr};
+    for (int j = 0; j < 3; ++j) {
+        d.head_out[j] = outs[j];
+        d.head_gamma[j] = gammas[j];
+        d.head_stride[j][0] = (int64_t)H * S * 64;
+        d.head_stride[j][1] = (int64_t)S * 64;
+        d.head_stride[j][2] = 64;
+    }
+    return sf_gemm_frag(&d, s);
+}
 
 // Q (and for the self-attention K, V) read from a projection's bf16 output
 // rows instead of [B, H, S, 64]: row b*S + s, row length q_ld / kv_ld
@@ -523,10 +573,12 @@ struct RowsIn {
 };
 
 // Sc: the rows per head of the K/V buffer (its capacity), Sk <= Sc the keys
-// read.  qp: Q from partials instead of q (which is then not read).
+// read.  q32: Q as fp32 projection rows, normalised with q32_gamma, instead
+// of q (which is then not read).
 int attention(sf_rdt* m, const uint16_t* q, const uint16_t* k, const uint16_t* v, int Sk,
               const int32_t* valid_len, void* out, bool exact_pv, hipStream_t s, int Sc = 0,
-              const QPartials* qp = nullptr, const RowsIn* rows = nullptr, bool v_f16 = false) {
+              const RowsIn* rows = nullptr, bool v_f16 = false, const float* q32 = nullptr,
+              const float* q32_gamma = nullptr) {
     const sf_rdt_config& c = m->cfg;
     const int S = c.horizon + 3;
     sf_attn_desc d;
@@ -564,67 +616,25 @@ int attention(sf_rdt* m, const uint16_t* q, const uint16_t* k, const uint16_t* v
     d.kv_valid_len = valid_len;
     d.exact_pv = exact_pv ? 1 : 0;
     d.v_f16 = v_f16 ? 1 : 0;
-    if (qp) {
-        d.q_partials = qp->p;
-        d.q_splits = qp->splits;
-        d.q_bias = qp->bias;
-        d.q_scale = qp->scale;
-        d.q_gamma = qp->gamma;
+    if (q32) {
+        d.q_rows32 = q32;
+        d.q_gamma = q32_gamma;
         d.q_eps = c.eps;
-        if (qp->row_ss) {
-            d.q_row_ss = qp->row_ss;
-            d.q_row_tiles = c.hidden / 64;
-            d.q_row_n = c.hidden;
-            d.q_row_eps = c.eps;
-        }
     }
-    // output straight into [B, S, H*64] (head_to_seq fused away)
+    d.o_frag = m->frag ? 1 : 0;
+    // output straight into [B, S, H*64] (head_to_seq fused away), or its
+    // fragment order
     d.o_stride[0] = (int64_t)S * c.hidden;
     d.o_stride[1] = 64;
     d.o_stride[2] = c.hidden;
     return sf_attn_fwd(&d, q, k, v, out, m->attn_ws, m->attn_ws_bytes, s);
 }
 
-// The cross-q projection of block L over the M rows of m->n, left as its
-// split-K partials in the GEMM workspace (SF_EPI_PARTIALS); *qp describes
-// them for the language attention, which finishes Q (bias, int8 scale,
-// q_norm) as the heads epilogue would (dit_block.cu:282-307).
-int cross_q_partials(sf_rdt* m, const LayerIdx& L, int M, hipStream_t s, QPartials* qp) {
-    const Param& W = m->params[L.cq_w];
-    sf_gemm_desc d{};
-    d.M = M;
-    d.N = (int32_t)W.shape[0];
-    d.K = (int32_t)W.shape[1];
-    d.A = m->n;
-    d.lda = m->cfg.hidden;
-    d.a_dtype = SF_BF16;
-    d.W = W.data;
-    d.ldw = W.shape[1];
-    d.w_dtype = W.dtype;
-    d.w_scale = W.scale;
-    d.epilogue = SF_EPI_PARTIALS;
-    d.workspace = m->gemm_ws;
-    d.workspace_bytes = (int64_t)m->gemm_ws_bytes;
-    SF_TRY(sf_gemm(&d, s));
-    qp->p = static_cast<const float*>(m->gemm_ws);
-    qp->splits = m->cq_splits;
-    qp->bias = pf(m, L.cq_b);
-    qp->scale = W.scale;
-    qp->gamma = pf(m, L.cq_norm);
-    qp->row_ss = m->n_deferred ? m->row_ss : nullptr;
-    return SF_OK;
-}
-
-// The projection weights that get fp16 copies.  Above 160 rows (the
-// library path): every block's six and the final layer's two.  At most 160
-// rows, with bf16 weights: the matrices whose inputs are fp16 there -- each
-// block's fc1 and fc2 and the final layer's fc2 -- so the split-K kernel
-// reads fp16 operands instead of converting every bf16 fragment in
-// registers (the same operands, so the same results); int8 weights keep
-// their 1-byte codes.  Only matrices with K a multiple of 16.  With
-// int8_weights = 2, no copy of the int8 matrices sf_gemm multiplies directly
-// at the block's rows (sf_gemm_int8_direct; every such call the block makes
-// has fp16 activations and a 16-bit fp16 product).
+// The projection weights that get fp16 copies above 160 rows (the library
+// path): every block's six and the final layer's two, where K is a multiple
+// of 16.  With int8_weights = 2, no copy of the int8 matrices sf_gemm
+// multiplies directly at the block's rows (sf_gemm_int8_direct; every such
+// call the block makes has fp16 activations and a 16-bit fp16 product).
 std::vector<int> w16_params(const sf_rdt* m) {
     const sf_rdt_config& c = m->cfg;
     std::vector<int> ws;
@@ -652,17 +662,35 @@ std::vector<int> w16_params(const sf_rdt* m) {
             }
             ws.swap(keep);
         }
-    } else if (!c.int8_weights) {
-        for (const LayerIdx& L : m->layers) {
-            ws.push_back(L.fc1_w);
-            ws.push_back(L.fc2_w);
-        }
-        ws.push_back(m->f2w);
     }
     std::vector<int> out;
     for (int w : ws)
         if (m->params[w].shape[1] % 16 == 0) out.push_back(w);
     return out;
+}
+
+// The weights that get fragment-ordered copies (at most 160 rows) and their
+// copies' types: fp16 where the projection's input is fp16 (fc1, fc2, the
+// final fc2), else bf16; int8 weights keep their codes.  The final fc2 joins
+// when its columns fill 32-wide tiles.
+std::vector<std::pair<int, int32_t>> frag_params(const sf_rdt* m) {
+    std::vector<std::pair<int, int32_t>> out;
+    if (!m->frag) return out;
+    auto add = [&](int w, int32_t dt) {
+        out.emplace_back(w, m->params[w].dtype == SF_I8 ? (int32_t)SF_I8 : dt);
+    };
+    for (const LayerIdx& L : m->layers) {
+        for (int w : {L.qkv_w, L.proj_w, L.cq_w, L.cproj_w}) add(w, SF_BF16);
+        for (int w : {L.fc1_w, L.fc2_w}) add(w, SF_F16);
+    }
+    add(m->f1w, SF_BF16);
+    if (m->cfg.action_dim % 32 == 0) add(m->f2w, SF_F16);
+    return out;
+}
+
+// Bytes of weight w's copy (both kinds hold every element).
+size_t copy_bytes(const sf_rdt* m, int w, int32_t dtype) {
+    return align256((size_t)m->params[w].shape[0] * m->params[w].shape[1] * (dtype == SF_I8 ? 1 : 2));
 }
 
 // Every GEMM the runtime issues: each matrix at each row count it is used
@@ -736,30 +764,29 @@ int next_norm(const sf_rdt* m, int i) {
     return i + 1 < m->cfg.layers ? m->layers[i + 1].norm1 : m->fnorm;
 }
 
-// Refreshes the fp16 weight copies of blocks [first, first + count) and,
-// with final_layer, of the final layer (no-op without copies), up to
-// SF_CODES_MAX_JOBS matrices per launch.
-int widen_codes(sf_rdt* m, int first, int count, hipStream_t s, bool final_layer = false) {
-    if (!m->codes16) return SF_OK;
+// Rewrites every weight copy from the parameters, up to SF_CODES_MAX_JOBS
+// matrices per launch.
+int write_copies(sf_rdt* m, hipStream_t s) {
+    if (m->frag) {
+        sf_frag_job jobs[SF_CODES_MAX_JOBS];
+        int n = 0;
+        for (const auto& f : frag_params(m)) {
+            const Param& P = m->params[f.first];
+            jobs[n++] = sf_frag_job{P.data, P.dtype, P.shape[1], m->copy_of[f.first], f.second,
+                                    (int32_t)P.shape[0], (int32_t)P.shape[1]};
+            if (n == SF_CODES_MAX_JOBS) {
+                SF_TRY(sf_frag_pack(jobs, n, s));
+                n = 0;
+            }
+        }
+        return n ? sf_frag_pack(jobs, n, s) : SF_OK;
+    }
     sf_w16_job jobs[SF_CODES_MAX_JOBS];
     int n = 0;
-    std::vector<int> ws;
-    for (int i = first; i < first + count; ++i)
-        for (int w : block_weights(m->layers[i])) ws.push_back(w);
-    if (final_layer) {
-        ws.push_back(m->f1w);
-        ws.push_back(m->f2w);
-    }
-    for (int w : ws) {
+    for (int w : w16_params(m)) {
         const Param& P = m->params[w];
-        if (!m->codes16_of[w]) continue;
-        jobs[n].w = P.data;
-        jobs[n].w_dtype = P.dtype;
-        jobs[n].ldw = P.shape[1];
-        jobs[n].out = const_cast<void*>(m->codes16_of[w]);
-        jobs[n].N = (int32_t)P.shape[0];
-        jobs[n].K = (int32_t)P.shape[1];
-        if (++n == SF_CODES_MAX_JOBS) {
+        jobs[n++] = sf_w16_job{P.data, P.dtype, P.shape[1], m->copy_of[w], (int32_t)P.shape[0], (int32_t)P.shape[1]};
+        if (n == SF_CODES_MAX_JOBS) {
             SF_TRY(sf_weights_to_f16(jobs, n, s));
             n = 0;
         }
@@ -767,77 +794,78 @@ int widen_codes(sf_rdt* m, int first, int count, hipStream_t s, bool final_layer
     return n ? sf_weights_to_f16(jobs, n, s) : SF_OK;
 }
 
-// RDTBlock::forward (dit_block.cu:349-387) on the fp32 residual m->x, with
-// m->n holding norm1(x) on entry; on exit m->n holds the next norm of x.
-// The fp16 weight copies of the library path (if any) are current
-// (refresh_w16).
-int block_forward(sf_rdt* m, int i, hipStream_t s) {
+// RDTBlock::forward (dit_block.cu:349-387) with fragment-ordered projections:
+// m->n holds the deferred norm1 on entry, and on exit the next block's (after
+// the last block the final norm, normalised).
+int block_forward_frag(sf_rdt* m, int i, hipStream_t s) {
     const sf_rdt_config& c = m->cfg;
     const LayerIdx& L = m->layers[i];
     const int D = c.hidden, S = c.horizon + 3, M = c.batch * S;
     const int fd = m->ffn_dtype, ad = m->act16;
     // self-attention branch
-    if (m->rows_qkv) {
-        // qkv = x W^T + b in fp16 (dit_block.cu:206-207); split_qkv and
-        // apply_qk_norm (:209-220) happen as the attention loads the rows
-        SF_TRY(linear(m, m->n, D, M, L.qkv_w, L.qkv_b, SF_ACT_NONE, m->qkv_rows, 3 * D, ad, false, s, ad));
-        RowsIn r;
-        r.q_ld = r.kv_ld = 3 * D;
-        r.q_gamma = pf(m, L.q_norm);
-        r.k_gamma = pf(m, L.k_norm);
-        r.f16 = ad == SF_F16;
-        SF_TRY(attention(m, m->qkv_rows, m->qkv_rows + D, m->qkv_rows + 2 * D, S, nullptr, m->a, false, s, 0,
-                         nullptr, &r));
-    } else {
-        uint16_t* qkv[3] = {m->q, m->k, m->v};
-        const int qk_g[3] = {L.q_norm, L.k_norm, -1};
-        SF_TRY(linear_heads(m, m->n, M, S, L.qkv_w, L.qkv_b, qkv, qk_g, 3, s, SF_BF16, true, m->n_deferred));
-        SF_TRY(attention(m, m->q, m->k, m->v, S, nullptr, m->a, false, s));
-    }
-    SF_TRY(linear_add_norm(m, m->a, ad, M, L.proj_w, L.proj_b, L.norm2, m->n, ad, s, m->defer));
-    m->n_deferred = m->defer;
+    SF_TRY(frag_qkv(m, L, s));
+    SF_TRY(attention(m, m->q, m->k, m->v, S, nullptr, m->a, false, s));
+    SF_TRY(frag_add_norm(m, m->a, ad, L.proj_w, L.proj_b, L.norm2, s));
+    // cross-attention branch: even blocks attend to language, odd to image
+    // (dit_block.cu:369); the cached V of a layer on the fp16 P.V form is
+    // held in fp16 (sf_bf16_to_f16_below)
+    const bool lang = (i % 2) == 0;
+    const bool exact = m->exact_pv[i] != 0;
+    SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, SF_ACT_NONE, m->q32, SF_F32, false, false, s, true));
+    SF_TRY(attention(m, nullptr, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
+                     lang ? m->lang_len : nullptr, m->a, exact, s, lang ? c.lang_max : c.img_len, nullptr, !exact,
+                     m->q32, pf(m, L.cq_norm)));
+    SF_TRY(frag_linear(m, m->a, ad, L.cproj_w, L.cproj_b, SF_ACT_NONE, m->x, SF_F32, false, true, s));
+    SF_TRY(sf_norm_frag(m->x, D, pf(m, L.norm3), m->n3, fd, nullptr, M, D, c.eps, s));
+    // FFN branch (Mlp::forward, dit_block.cu:143-163)
+    SF_TRY(frag_linear(m, m->n3, fd, L.fc1_w, L.fc1_b, SF_ACT_GELU_TANH, m->h, fd, true, false, s));
+    if (i + 1 < c.layers) return frag_add_norm(m, m->h, fd, L.fc2_w, L.fc2_b, m->layers[i + 1].norm1, s);
+    SF_TRY(frag_linear(m, m->h, fd, L.fc2_w, L.fc2_b, SF_ACT_NONE, m->x, SF_F32, false, true, s));
+    return sf_norm_frag(m->x, D, pf(m, m->fnorm), m->n, ad, nullptr, M, D, c.eps, s);
+}
+
+// RDTBlock::forward (dit_block.cu:349-387) on the fp32 residual m->x, with
+// m->n holding norm1(x) on entry; on exit m->n holds the next norm of x.
+// The weight copies are current (refresh_copies).
+int block_forward(sf_rdt* m, int i, hipStream_t s) {
+    if (m->frag) return block_forward_frag(m, i, s);
+    const sf_rdt_config& c = m->cfg;
+    const LayerIdx& L = m->layers[i];
+    const int D = c.hidden, S = c.horizon + 3, M = c.batch * S;
+    const int fd = m->ffn_dtype, ad = m->act16;
+    // self-attention branch: qkv = x W^T + b in fp16 (dit_block.cu:206-207);
+    // split_qkv and apply_qk_norm (:209-220) happen as the attention loads
+    // the rows
+    SF_TRY(linear(m, m->n, D, M, L.qkv_w, L.qkv_b, SF_ACT_NONE, m->qkv_rows, 3 * D, ad, false, s, ad));
+    RowsIn r;
+    r.q_ld = r.kv_ld = 3 * D;
+    r.q_gamma = pf(m, L.q_norm);
+    r.k_gamma = pf(m, L.k_norm);
+    r.f16 = ad == SF_F16;
+    SF_TRY(attention(m, m->qkv_rows, m->qkv_rows + D, m->qkv_rows + 2 * D, S, nullptr, m->a, false, s, 0, &r));
+    SF_TRY(linear_add_norm(m, m->a, ad, M, L.proj_w, L.proj_b, L.norm2, m->n, ad, s));
     // cross-attention branch: even blocks attend to language, odd to image
     // (dit_block.cu:369)
     const bool lang = (i % 2) == 0;
     // the cached V of a layer on the fp16 P.V form is held in fp16 (converted
     // once when the condition was set, sf_bf16_to_f16_below)
     const bool exact = m->exact_pv[i] != 0;
-    if (lang && m->cq_splits > 0) {   // Q finished inside the attention
-        QPartials qp;
-        SF_TRY(cross_q_partials(m, L, M, s, &qp));
-        SF_TRY(attention(m, nullptr, m->ck[i], m->cv[i], m->cond_lang_rows, m->lang_len, m->a,
-                         exact, s, c.lang_max, &qp, nullptr, !exact));
-    } else if (m->rows_qkv) {
-        // q = x W^T + b in fp16 rows (dit_block.cu:282-284); seq_to_head and
-        // q_norm (:298-307) happen as the attention loads them (rounding Q to
-        // bf16 for the bf16 K/V cache)
-        SF_TRY(linear(m, m->n, D, M, L.cq_w, L.cq_b, SF_ACT_NONE, m->q, D, ad, false, s, ad));
-        RowsIn r;
-        r.q_ld = D;
-        r.q_gamma = pf(m, L.cq_norm);
-        r.f16 = ad == SF_F16;
-        SF_TRY(attention(m, m->q, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
-                         lang ? m->lang_len : nullptr, m->a, exact, s,
-                         lang ? c.lang_max : c.img_len, nullptr, &r, !exact));
-    } else {
-        uint16_t* cq[1] = {m->q};
-        const int cq_g[1] = {L.cq_norm};
-        SF_TRY(linear_heads(m, m->n, M, S, L.cq_w, L.cq_b, cq, cq_g, 1, s, SF_BF16, true, m->n_deferred));
-        SF_TRY(attention(m, m->q, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
-                         lang ? m->lang_len : nullptr, m->a, exact, s,
-                         lang ? c.lang_max : c.img_len, nullptr, nullptr, !exact));
-    }
+    // q = x W^T + b in fp16 rows (dit_block.cu:282-284); seq_to_head and
+    // q_norm (:298-307) happen as the attention loads them (rounding Q to
+    // bf16 for the bf16 K/V cache)
+    SF_TRY(linear(m, m->n, D, M, L.cq_w, L.cq_b, SF_ACT_NONE, m->q, D, ad, false, s, ad));
+    RowsIn cr;
+    cr.q_ld = D;
+    cr.q_gamma = pf(m, L.cq_norm);
+    cr.f16 = ad == SF_F16;
+    SF_TRY(attention(m, m->q, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
+                     lang ? m->lang_len : nullptr, m->a, exact, s, lang ? c.lang_max : c.img_len, &cr, !exact));
     SF_TRY(linear_add_norm(m, m->a, ad, M, L.cproj_w, L.cproj_b, L.norm3, m->n3, fd, s));
     // FFN branch (Mlp::forward, dit_block.cu:143-163); fc2's add + norm
     // writes the next block's norm1 (act16, the QKV input)
     const int F = (int)ffn_dim(c);
     SF_TRY(linear(m, m->n3, D, M, L.fc1_w, L.fc1_b, SF_ACT_GELU_TANH, m->h, F, fd, false, s, fd));
-    // the next block's norm1 deferred; the final norm row-wide (its consumer,
-    // the final layer's fc1, takes normalised rows)
-    const bool defer_next = m->defer && i + 1 < c.layers;
-    SF_TRY(linear_add_norm(m, m->h, fd, M, L.fc2_w, L.fc2_b, next_norm(m, i), m->n, ad, s, defer_next));
-    m->n_deferred = defer_next;
-    return SF_OK;
+    return linear_add_norm(m, m->h, fd, M, L.fc2_w, L.fc2_b, next_norm(m, i), m->n, ad, s);
 }
 
 // m->n = first norm applied to the residual m->x before block `first`.
@@ -845,8 +873,11 @@ int entry_norm(sf_rdt* m, int first, hipStream_t s) {
     const sf_rdt_config& c = m->cfg;
     const int D = c.hidden, M = c.batch * (c.horizon + 3);
     const int g = first < c.layers ? m->layers[first].norm1 : m->fnorm;
-    m->n_deferred = m->defer && first < c.layers;
-    if (m->n_deferred) return sf_rmsnorm_deferred(m->x, D, pf(m, g), m->n, m->act16, D, m->row_ss, M, D, s);
+    if (m->frag) {
+        const bool deferred = first < c.layers;   // the final norm is row-wide
+        if (deferred) m->row_tiles = D / 64;
+        return sf_norm_frag(m->x, D, pf(m, g), m->n, m->act16, deferred ? m->row_ss : nullptr, M, D, c.eps, s);
+    }
     return sf_rmsnorm(m->x, SF_F32, D, pf(m, g), m->n, m->act16, D, M, D, c.eps, s);
 }
 
@@ -882,6 +913,20 @@ int step_forward(sf_rdt* m, const float* x_t, float t, hipStream_t s,
     SF_TRY(entry_norm(m, 0, s));
     for (int i = 0; i < c.layers; ++i) SF_TRY(block_forward(m, i, s));
     // FinalLayer (dit_block.cu:407-412); m->n = norm_final(x) from the last block
+    if (m->frag) {
+        const bool f2 = m->copy_of[m->f2w] != nullptr;   // else row-major into the split-K kernel
+        sf_frag_gemm_desc d = frag_desc(m, m->n, m->act16, m->f1w, m->f1b, false);
+        d.act = SF_ACT_GELU_TANH;
+        d.epilogue = SF_EPI_PLAIN;
+        d.C = m->h;
+        d.ldc = D;
+        d.c_dtype = m->ffn_dtype;
+        d.c_frag = f2 ? 1 : 0;
+        SF_TRY(sf_gemm_frag(&d, s));
+        if (f2)
+            return frag_linear(m, m->h, m->ffn_dtype, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, SF_F32, false, false, s);
+        return linear(m, m->h, D, M, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, A, SF_F32, false, s, m->ffn_dtype);
+    }
     SF_TRY(linear(m, m->n, D, M, m->f1w, m->f1b, SF_ACT_GELU_TANH, m->h, D, m->ffn_dtype, false, s, m->act16));
     return linear(m, m->h, D, M, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, A, SF_F32, false, s,
                   m->ffn_dtype);
@@ -938,12 +983,12 @@ hipStream_t pick_stream(sf_rdt* m, void* stream) {
     return stream ? static_cast<hipStream_t>(stream) : m->own_stream;
 }
 
-// The fp16 weight copies of the library path, brought up to date before a
-// pass (never under capture: every entry point calls this first).
-int refresh_w16(sf_rdt* m, hipStream_t s) {
-    if (!m->codes16 || !m->w16_stale) return SF_OK;
-    SF_TRY(widen_codes(m, 0, m->cfg.layers, s, true));
-    m->w16_stale = false;
+// The weight copies, brought up to date before a pass (never under capture:
+// every entry point calls this first).
+int refresh_copies(sf_rdt* m, hipStream_t s) {
+    if (!m->copies || !m->copies_stale) return SF_OK;
+    SF_TRY(write_copies(m, s));
+    m->copies_stale = false;
     return SF_OK;
 }
 
@@ -988,10 +1033,10 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     sf_rdt* m = new sf_rdt();
     m->cfg = c;
     // fp16 FFN inputs at every batch size; the other projection inputs in
-    // fp16 once the block GEMMs leave the split-K regime (M > 160 rows)
+    // fp16 once the block GEMMs leave the fragment-ordered step (M > 160 rows)
     m->ffn_dtype = SF_F16;
     m->act16 = c.batch * (c.horizon + 3) <= 160 ? SF_BF16 : SF_F16;
-    m->defer = c.batch * (c.horizon + 3) <= 160 && c.hidden % 64 == 0 && c.hidden / 64 <= 64;
+    m->frag = c.batch * (c.horizon + 3) <= 160;
     build_param_table(m);
 
     const int64_t B = c.batch, D = c.hidden, T = c.horizon, S = T + 3, A = c.action_dim;
@@ -1052,13 +1097,13 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     m->cv.assign(c.layers, nullptr);
     std::vector<Buf> bufs = {
         {(void**)&m->x, (size_t)(B * S * D * 4)},
-        {(void**)&m->n, (size_t)(B * S * D * 2)},
+        {(void**)&m->n, sf_frag_elems(B * S, D) * 2},
         {(void**)&m->q, (size_t)(B * H * S * 64 * 2)},
         {(void**)&m->k, (size_t)(B * H * S * 64 * 2)},
         {(void**)&m->v, (size_t)(B * H * S * 64 * 2)},
-        {(void**)&m->a, (size_t)(B * S * D * 2)},
-        {(void**)&m->n3, (size_t)(B * S * D * 2)},
-        {(void**)&m->h, (size_t)(B * S * ffn_dim(c) * 2)},
+        {(void**)&m->a, sf_frag_elems(B * S, D) * 2},
+        {(void**)&m->n3, sf_frag_elems(B * S, D) * 2},
+        {(void**)&m->h, sf_frag_elems(B * S, ffn_dim(c)) * 2},
         {(void**)&m->act_in, (size_t)(B * T * 2 * A * 2)},
         {(void**)&m->sa0, (size_t)(B * T * D * 2)},
         {(void**)&m->sa1, (size_t)(B * T * D * 2)},
@@ -1089,12 +1134,15 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     if (m->kv_prod_bytes) bufs.push_back({(void**)&m->kv_prod, m->kv_prod_bytes});
     m->gemm_ws_bytes = gemm_ws_for(m, false, nullptr);
     bufs.push_back({&m->gemm_ws, std::max<size_t>(m->gemm_ws_bytes, 256)});
-    m->rows_qkv = S * B > 160;
-    if (m->rows_qkv) bufs.push_back({(void**)&m->qkv_rows, (size_t)(B * S * 3 * D * 2)});
-    if (m->defer) bufs.push_back({(void**)&m->row_ss, (size_t)(D / 64) * B * S * 4});
-    for (int w : w16_params(m))   // fp16 weight copies
-        m->codes16_bytes += align256((size_t)m->params[w].shape[0] * m->params[w].shape[1] * 2);
-    if (m->codes16_bytes) bufs.push_back({(void**)&m->codes16, m->codes16_bytes});
+    if (!m->frag) bufs.push_back({(void**)&m->qkv_rows, (size_t)(B * S * 3 * D * 2)});
+    if (m->frag) {
+        bufs.push_back({(void**)&m->row_ss, (size_t)((D + 31) / 32) * B * S * 4});
+        bufs.push_back({(void**)&m->q32, (size_t)(B * S * D * 4)});
+    }
+    std::vector<std::pair<int, int32_t>> copies = frag_params(m);   // weight copies
+    for (int w : w16_params(m)) copies.emplace_back(w, (int32_t)SF_F16);
+    for (const auto& cp : copies) m->copies_bytes += copy_bytes(m, cp.first, cp.second);
+    if (m->copies_bytes) bufs.push_back({(void**)&m->copies, m->copies_bytes});
     std::vector<size_t> boff(bufs.size());
     for (size_t i = 0; i < bufs.size(); ++i) {
         boff[i] = off;
@@ -1117,30 +1165,16 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
         G.scale = G.w_dtype == SF_I8 ? reinterpret_cast<const float*>(m->arena + kv_s_off[g]) : nullptr;
     }
     for (size_t i = 0; i < bufs.size(); ++i) *bufs[i].ptr = m->arena + boff[i];
-    m->codes16_of.assign(m->params.size(), nullptr);
-    if (m->codes16) {
-        char* dst = m->codes16;
-        for (int w : w16_params(m)) {
-            const Param& P = m->params[w];
-            m->codes16_of[w] = dst;
-            dst += align256((size_t)P.shape[0] * P.shape[1] * 2);
+    m->copy_of.assign(m->params.size(), nullptr);
+    if (m->copies) {
+        char* dst = m->copies;
+        for (const auto& cp : copies) {
+            m->copy_of[cp.first] = dst;
+            dst += copy_bytes(m, cp.first, cp.second);
         }
     }
     m->exact_pv.assign(c.layers, 0);
     m->lang_rows = m->cond_lang_rows = c.lang_max;
-    if (c.layers > 0) {   // the fused cross-q finish (see cq_splits)
-        sf_gemm_desc g{};
-        g.M = (int32_t)(B * S);
-        g.N = (int32_t)D;
-        g.K = (int32_t)D;
-        g.a_dtype = SF_BF16;
-        const int splits = sf_gemm_num_splits(&g);
-        sf_attn_desc a;
-        sf_attn_desc_init_bhsd(&a, (int32_t)B, (int32_t)H, (int32_t)S, c.lang_max, 64, SF_BF16, SF_BF16);
-        const bool qblocks = B * H * ((S + 79) / 80) < 256 && c.lang_max <= 1024 && sf_attn_num_splits(&a) == 1;
-        if (splits >= 1 && splits <= 8 && qblocks && (size_t)splits * B * S * D * 4 <= m->gemm_ws_bytes)
-            m->cq_splits = splits;
-    }
     if (hipStreamCreate(&m->own_stream) != hipSuccess) {
         (void)hipFree(m->arena);
         delete m;
@@ -1240,7 +1274,7 @@ extern "C" int sf_rdt_param_info(const sf_rdt* m, int32_t idx, const char** name
 
 extern "C" void* sf_rdt_param_data(sf_rdt* m, int32_t idx) {
     if (!m || idx < 0 || idx >= (int32_t)m->params.size()) return nullptr;
-    m->w16_stale = true;   // the caller may write through it before the next pass
+    m->copies_stale = true;   // the caller may write through it before the next pass
     return m->params[idx].data;
 }
 
@@ -1430,7 +1464,7 @@ extern "C" int sf_rdt_run_blocks(sf_rdt* m, float* x, int32_t first, int32_t cou
     hipStream_t s = pick_stream(m, stream);
     SF_TRY(resolve_pv_forms(m));
     const size_t nbytes = (size_t)c.batch * (c.horizon + 3) * c.hidden * 4;
-    SF_TRY(refresh_w16(m, s));
+    SF_TRY(refresh_copies(m, s));
     SF_HIP(hipMemcpyAsync(m->x, x, nbytes, hipMemcpyDeviceToDevice, s));
     SF_TRY(entry_norm(m, first, s));
     for (int i = first; i < first + count; ++i) SF_TRY(block_forward(m, i, s));
@@ -1444,7 +1478,7 @@ extern "C" int sf_rdt_denoise_step(sf_rdt* m, const float* x_t, float t, float* 
     const sf_rdt_config& c = m->cfg;
     hipStream_t s = pick_stream(m, stream);
     SF_TRY(resolve_pv_forms(m));
-    SF_TRY(refresh_w16(m, s));
+    SF_TRY(refresh_copies(m, s));
     SF_TRY(step_forward(m, x_t, t, s));
     // last T token rows of each batch element (rdt1b.cpp:362-368)
     SF_HIP(hipMemcpy2DAsync(velocity, (size_t)c.horizon * c.action_dim * 4,
@@ -1458,7 +1492,7 @@ extern "C" int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* strea
     const sf_rdt_config& c = m->cfg;
     hipStream_t s = pick_stream(m, stream);
     SF_TRY(resolve_pv_forms(m));
-    SF_TRY(refresh_w16(m, s));
+    SF_TRY(refresh_copies(m, s));
     const size_t nbytes = (size_t)c.batch * c.horizon * c.action_dim * 4;
     // the initial noise is copied in outside the graph (flow_matching.cpp:49-51)
     SF_HIP(hipMemcpyAsync(m->x_state, x, nbytes, hipMemcpyDeviceToDevice, s));

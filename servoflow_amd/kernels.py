@@ -155,6 +155,87 @@ def weights_to_f16(ws):
     return outs
 
 
+def frag_pack(ws, out_dtypes):
+    """Fragment-ordered copies (sf_frag_pack) of row-major matrices, one
+    launch (at most abi.SF_CODES_MAX_JOBS)."""
+    outs = [torch.empty(w.shape[0], w.shape[1], dtype=dt, device=w.device) for w, dt in zip(ws, out_dtypes)]
+    jobs = (abi.FragJob * max(1, len(ws)))()
+    for j, (w, o) in enumerate(zip(ws, outs)):
+        jobs[j].w, jobs[j].w_dtype, jobs[j].ldw = w.data_ptr(), _DT[w.dtype], w.stride(0)
+        jobs[j].out, jobs[j].out_dtype, jobs[j].N, jobs[j].K = o.data_ptr(), _DT[o.dtype], w.shape[0], w.shape[1]
+    abi.check(abi.lib().sf_frag_pack(jobs, len(ws), _stream(ws[0]) if ws else None), "sf_frag_pack")
+    return outs
+
+
+def _frag_desc(M, a, w, bias, act, w_scale, row_ss, row_n, row_eps):
+    d = abi.FragGemmDesc()
+    d.M, d.N, d.K = M, w.shape[0], w.shape[1]
+    d.A, d.a_dtype = a.data_ptr(), _DT[a.dtype]
+    d.W, d.w_dtype = w.data_ptr(), _DT[w.dtype]
+    d.w_scale, d.bias, d.act = _p(w_scale), _p(bias), act
+    if row_ss is not None:
+        d.a_row_ss, d.a_row_tiles, d.a_row_n, d.a_row_eps = row_ss.data_ptr(), row_ss.shape[1], row_n, row_eps
+    return d
+
+
+def _run_frag(d, t):
+    abi.check(abi.lib().sf_gemm_frag(ctypes.byref(d), _stream(t)), "sf_gemm_frag")
+
+
+def gemm_frag(M, a, w, bias=None, act=abi.SF_ACT_NONE, out=None, out_dtype=torch.float32, c_frag=False,
+              accumulate=False, w_scale=None, row_ss=None, row_n=0, row_eps=1e-6):
+    """sf_gemm_frag's plain epilogue on M rows of a (fragment order, padded
+    rows) and w (frag_pack): row-major [M, N], or fragment order with c_frag."""
+    N = w.shape[0]
+    d = _frag_desc(M, a, w, bias, act, w_scale, row_ss, row_n, row_eps)
+    if out is None:
+        out = torch.empty((M + 15) // 16 * 16 if c_frag else M, N, dtype=out_dtype, device=a.device)
+    d.epilogue = abi.SF_EPI_PLAIN
+    d.C, d.ldc, d.c_dtype = out.data_ptr(), N if c_frag else out.stride(0), _DT[out.dtype]
+    d.c_frag, d.accumulate = int(c_frag), int(accumulate)
+    _run_frag(d, a)
+    return out
+
+
+def gemm_frag_heads(M, a, w, bias, S, H, outs, gammas=(None, None, None), eps=1e-6, w_scale=None, row_ss=None,
+                    row_n=0, row_eps=1e-6):
+    """sf_gemm_frag's per-head epilogue (outs: [B,H,S,64] bf16 views)."""
+    d = _frag_desc(M, a, w, bias, abi.SF_ACT_NONE, w_scale, row_ss, row_n, row_eps)
+    d.epilogue, d.H, d.S, d.eps = abi.SF_EPI_HEADS, H, S, eps
+    for j, o in enumerate(outs):
+        d.head_out[j], d.head_gamma[j] = o.data_ptr(), _p(gammas[j])
+        d.head_stride[j][:] = (o.stride(0), o.stride(1), o.stride(2))
+    _run_frag(d, a)
+    return outs
+
+
+def gemm_frag_add_norm(M, a, w, bias, residual, gamma, norm_dtype=torch.bfloat16, w_scale=None):
+    """sf_gemm_frag's residual add + deferred RMSNorm: residual (fp32 [M, N])
+    += a w^T + bias; returns (residual * gamma in fragment order, tile sums
+    of squares)."""
+    N = w.shape[0]
+    d = _frag_desc(M, a, w, bias, abi.SF_ACT_NONE, w_scale, None, 0, 0.0)
+    out = torch.empty((M + 15) // 16 * 16, N, dtype=norm_dtype, device=a.device)
+    ss = torch.empty(M, abi.lib().sf_gemm_frag_ss_tiles(N), dtype=torch.float32, device=a.device)
+    d.epilogue = abi.SF_EPI_ADD_NORM
+    d.C, d.ldc, d.c_dtype = residual.data_ptr(), residual.stride(0), abi.SF_F32
+    d.norm_gamma, d.norm_out, d.norm_dtype, d.norm_ss = gamma.data_ptr(), out.data_ptr(), _DT[norm_dtype], ss.data_ptr()
+    _run_frag(d, a)
+    return out, ss
+
+
+def norm_frag(x, gamma, eps=1e-6, out_dtype=torch.bfloat16, deferred=False):
+    """sf_norm_frag on fp32 rows: (fragment-ordered norm or x * gamma, tile
+    sums or None)."""
+    rows, cols = x.shape
+    out = torch.empty((rows + 15) // 16 * 16, cols, dtype=out_dtype, device=x.device)
+    ss = torch.empty(rows, cols // 64, dtype=torch.float32, device=x.device) if deferred else None
+    st = abi.lib().sf_norm_frag(x.data_ptr(), x.stride(0), gamma.data_ptr(), out.data_ptr(), _DT[out_dtype], _p(ss),
+                                rows, cols, eps, _stream(x))
+    abi.check(st, "sf_norm_frag")
+    return out, ss
+
+
 def rmsnorm_deferred(x, gamma, out_dtype=torch.bfloat16):
     """sf_rmsnorm_deferred on fp32 rows x [rows, cols]: (x * gamma in
     out_dtype, tile sums of squares [cols / 64, rows] fp32)."""
