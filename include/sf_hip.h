@@ -544,7 +544,10 @@ int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int
  *                    norm_ss[m * T + t] = the sum of C[m][n]^2 over tile t's
  *                    columns, T = sf_gemm_frag_ss_tiles(N) <= 64 tiles.
  * a_row_ss (SF_EPI_PLAIN, SF_EPI_HEADS): as sf_gemm_desc's, but row-major,
- * [M][a_row_tiles].  Row m's result depends on
+ * [M][a_row_tiles].  SF_F16 rows from SF_EPI_ADD_NORM need a_x (SF_EPI_PLAIN):
+ * x * gamma can leave fp16's range, which that epilogue marks by an infinite
+ * sum; rows whose mean square is not in [2^-16, inf) are then normalised from
+ * the fp32 rows a_x [M][a_x_ld] with a_x_gamma instead (a_row_n == K).  Row m's result depends on
  * row m, the weights and the summation order that K fixes, not on M. */
 typedef struct sf_frag_gemm_desc {
     int32_t M, N, K;
@@ -574,6 +577,9 @@ typedef struct sf_frag_gemm_desc {
     int32_t a_row_tiles;
     int32_t a_row_n;
     float a_row_eps;
+    const float* a_x;
+    int64_t a_x_ld;
+    const float* a_x_gamma;
 } sf_frag_gemm_desc;
 int sf_gemm_frag(const sf_frag_gemm_desc* desc, void* stream);
 int32_t sf_gemm_frag_ss_tiles(int32_t N);

@@ -133,6 +133,7 @@ class FragGemmDesc(ctypes.Structure):
         ("a_row_tiles", ctypes.c_int32),
         ("a_row_n", ctypes.c_int32),
         ("a_row_eps", ctypes.c_float),
+        ("a_x", ctypes.c_void_p), ("a_x_ld", ctypes.c_int64), ("a_x_gamma", ctypes.c_void_p),
     ]
 
 

@@ -82,10 +82,15 @@ __device__ __forceinline__ u32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_
 // Sum over the 16 lanes of each row (DPP quad permutes, then the row's half
 // mirror and mirror: VALU only, no LDS round trip); every lane of the row
 // gets the sum, added in the order of an xor butterfly over 1, 2, 4, 8.
-__device__ __forceinline__ float row16_sum(float x) {
+// row8_sum: over each half row of 8 lanes only.
+__device__ __forceinline__ float row8_sum(float x) {
     x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true));   // quad_perm 1,0,3,2
     x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, true));   // quad_perm 2,3,0,1
     x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xF, 0xF, true));  // row_half_mirror
+    return x;
+}
+__device__ __forceinline__ float row16_sum(float x) {
+    x = row8_sum(x);
     x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x140, 0xF, 0xF, true));  // row_mirror
     return x;
 }

@@ -42,6 +42,22 @@ constexpr int kFragWaves = 4;
 constexpr int kFragMaxRows = 160;
 constexpr int kFragRowTiles = 64;   // tile sums of a deferred row: 16 in each of 4 lane groups
 
+// What the rows of a are (the RS template argument): finished; x * gamma of a
+// deferred norm; or that in fp16 with the range guard.
+//
+// The guard.  x * gamma, unlike the normalised row, is not bounded by fp16's
+// range.  The add + norm epilogue reports an element beyond it by an infinite
+// tile sum, and the consumer reads each row's sum anyway: a row whose mean
+// square is not in [2^-16, inf) -- out of range above, or so small that fp16's
+// subnormal step (2^-25) is no longer far below the row's own rounding -- is
+// contracted again from the fp32 residual, normalised first, by the wave that
+// finishes it.  Rows in range, every row of a model whose residual is not
+// degenerate, pay one comparison; a row's result does not depend on whether
+// its neighbours are in range.
+enum RowKind { kRowPlain = 0, kRowDeferred = 1, kRowGuarded = 2 };
+constexpr float kGuardMinMeanSq = 1.f / 65536.f;
+constexpr float kF16Max = 65504.f;
+
 // The epilogue's arguments (the operands' pointers and sizes are scalar kernel
 // arguments of their own, see gemm_frag_kernel).
 struct FragEpi {
@@ -60,6 +76,10 @@ struct FragEpi {
     uint16_t* norm_out;
     float* norm_ss;
     int norm_f16;
+    // kRowGuarded: the fp32 rows [M][x_ld] and the norm's gamma
+    const float* x;
+    const float* x_gamma;
+    int64_t x_ld;
     // per-head
     int H, S;
     float eps;
@@ -101,11 +121,12 @@ __device__ __forceinline__ float sum_groups(float x) {
 // front: those are preloaded into SGPRs with the wave
 // (-amdgpu-kernarg-preload-count), so the first loads go out without a
 // scalar-memory round trip; the epilogue's arguments are fetched behind them.
-template <int NB, int MB, int U, bool W8, bool AH, int EPI, bool RS>
+template <int NB, int MB, int U, bool W8, bool AH, int EPI, int RS>
 __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu(1, 2))) void gemm_frag_kernel(
     const void* A, const void* W, int K, int M, int ntiles, const float* row_ss, int row_tiles, float row_inv_n,
     float row_eps, const FragEpi e) {
     static_assert(EPI != SF_EPI_HEADS || NB == 4, "a head is one column tile");
+    static_assert(RS != kRowGuarded || (AH && EPI == SF_EPI_PLAIN), "fp16 rows of the plain epilogue are guarded");
     constexpr int NW = kFragWaves;
     constexpr int WL = W8 ? NB : 2 * NB;   // weight loads per 64-wide chunk
     constexpr bool kAddNorm = EPI == SF_EPI_ADD_NORM, kHeads = EPI == SF_EPI_HEADS, kPlain = EPI == SF_EPI_PLAIN;
@@ -138,7 +159,7 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
             v[q] = __builtin_bit_cast(f32x4, buffer_load16(rrs, off));
         }
     };
-    auto row_scale = [&](f32x4 (&v)[kFragRowTiles / 16]) {
+    auto row_sum = [&](f32x4 (&v)[kFragRowTiles / 16]) {
         if (row_tiles & 3) {   // the last quad runs into the next row
 #pragma unroll
             for (int q = 0; q < kFragRowTiles / 16; ++q)
@@ -146,11 +167,11 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
                 for (int i = 0; i < 4; ++i) v[q][i] = 16 * q + 4 * g4 + i < row_tiles ? v[q][i] : 0.f;
         }
         const f32x4 t = (v[0] + v[1]) + (v[2] + v[3]);
-        return deferred_rsqrt(sum_groups((t[0] + t[1]) + (t[2] + t[3])), row_inv_n, row_eps);
+        return sum_groups((t[0] + t[1]) + (t[2] + t[3]));
     };
     const int mrow = m0 + 16 * w + r;      // this lane's row of the wave's first row block
     f32x4 rss[kFragRowTiles / 16];
-    if constexpr (RS) load_row(mrow, w < MB && mrow < M, rss);
+    if constexpr (RS != kRowPlain) load_row(mrow, w < MB && mrow < M, rss);
 
     u32x4 wv[2][U][WL], av[2][U][2 * MB];
     // One group of U chunks; chunks past ce load zeros (beyond the buffer
@@ -240,8 +261,11 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
     issue_a(cb, av[0]);
     issue_a(cb + U, av[1]);
     __builtin_amdgcn_sched_barrier(0);
-    float rs = 1.f;
-    if constexpr (RS) rs = row_scale(rss);
+    float rs = 1.f, sum = 0.f;
+    if constexpr (RS != kRowPlain) {
+        sum = row_sum(rss);
+        rs = deferred_rsqrt(sum, row_inv_n, row_eps);
+    }
 
     int c0 = cb;
     for (; c0 + 2 * U < ce; c0 += 2 * U) {
@@ -279,12 +303,48 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
                 if (need_res && m < M)
                     res[nb] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(e.c) + (int64_t)m * e.ldc + n0 +
                                                               16 * nb + 4 * g4);
-            if constexpr (RS) {
+            if constexpr (RS != kRowPlain) {
                 load_row(m, m < M, rss);
-                rs = row_scale(rss);
+                sum = row_sum(rss);
+                rs = deferred_rsqrt(sum, row_inv_n, row_eps);
             }
         }
-        if constexpr (RS) {
+        if constexpr (RS == kRowGuarded) {
+            const float mean = sum * row_inv_n;
+            const bool out = m < M && !(mean >= kGuardMinMeanSq && mean < INFINITY);
+            if (__any(out)) {   // lanes r, r + 16, r + 32, r + 48 agree
+                const float* xr = e.x + (int64_t)min(m, M - 1) * e.x_ld;
+                float t = 0.f;
+                for (int k = 8 * g4; k < K; k += 32)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) t += xr[k + j] * xr[k + j];
+                const float inv_rms = 1.f / sqrtf(sum_groups(t) / (float)K + row_eps);
+                f32x4 s[NB];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) s[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int c = 0; c < 2 * nd; ++c) {
+                    const int k = 32 * c + 8 * g4;
+                    f16x8 f;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) f[j] = (_Float16)(xr[k + j] * inv_rms * e.x_gamma[k + j]);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        const int blk = W8 ? nb * nd + (c >> 1) : nb * 2 * nd + c;
+                        const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(wrs, (uint32_t)(lane * 16), blk * 1024, 0);
+                        f16x8 wf;
+                        if constexpr (W8) wf = i8x8_to_f16x8(c & 1 ? uint2{q[2], q[3]} : uint2{q[0], q[1]});
+                        else wf = u32x4_as_f16x8(q);
+                        s[nb] = mfma16x16x32_f16(wf, f, s[nb]);
+                    }
+                }
+                if (out) {
+                    rs = 1.f;
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) v[nb] = s[nb];
+                }
+            }
+        }
+        if constexpr (RS != kRowPlain) {
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -320,20 +380,26 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
             for (int nb = 0; nb < NB; ++nb)
                 *reinterpret_cast<uint2*>(o + 16 * nb + 4 * g4) = pack_kind4(v[nb], false);
         } else if constexpr (kAddNorm) {
-            float ss = 0.f;
+            float ss = 0.f, top = 0.f;
+            f32x4 u[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 v[nb] += res[nb];
+                u[nb] = v[nb] * gam[nb];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) ss += v[nb][j] * v[nb][j];
+                for (int j = 0; j < 4; ++j) {
+                    ss += v[nb][j] * v[nb][j];
+                    top = fmaxf(top, fabsf(u[nb][j]));
+                }
             }
+            if (e.norm_f16 && top > kF16Max) ss = INFINITY;   // the consumer's guard takes the row
             ss = sum_groups(ss);
             if (m >= M) continue;
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 const int n = n0 + 16 * nb + 4 * g4;
                 *reinterpret_cast<f32x4*>(static_cast<float*>(e.c) + (int64_t)m * e.ldc + n) = v[nb];
-                *reinterpret_cast<uint2*>(e.norm_out + frag_off(m, n, e.N)) = pack_kind4(v[nb] * gam[nb], e.norm_f16 != 0);
+                *reinterpret_cast<uint2*>(e.norm_out + frag_off(m, n, e.N)) = pack_kind4(u[nb], e.norm_f16 != 0);
             }
             if (g4 == 0) e.norm_ss[(int64_t)m * ntiles + tile] = ss;
         } else {
@@ -388,9 +454,7 @@ __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t 
     if (ss) {   // 8 lanes hold a 64-column tile
 #pragma unroll
         for (int i = 0; i < kNormFragPer; ++i) {
-            float t = sum[i];
-#pragma unroll
-            for (int off = 1; off < 8; off <<= 1) t += __shfl_xor(t, off, 64);
+            const float t = row8_sum(sum[i]);
             const int c = 8 * ((int)threadIdx.x + 256 * i);
             if (c < cols && (threadIdx.x & 7) == 0) ss[(int64_t)row * (cols / 64) + c / 64] = t;
         }
@@ -398,8 +462,7 @@ __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t 
         float t = 0.f;
 #pragma unroll
         for (int i = 0; i < kNormFragPer; ++i) t += sum[i];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off, 64);
+        t = sum_groups(row16_sum(t));
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
         __syncthreads();
         s = 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)cols + eps);
@@ -497,27 +560,39 @@ struct FragOps {
     float row_inv_n, row_eps;
 };
 
-template <int NB, int MB, int U, int EPI, bool RS>
-void launch_frag_rs(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
-    const dim3 grid(8u * (unsigned)t.nms, (unsigned)((t.ntiles + 7) / 8)), block(64 * kFragWaves);
-    if (o.w8) {
-        if (o.ah) hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, true, true, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
-        else hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, true, false, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
-    } else {
-        if (o.ah) hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, false, true, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
-        else hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, false, false, EPI, RS>), grid, block, 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n, o.row_eps, e);
+template <int NB, int MB, int U, bool W8, bool AH, int EPI, int RS>
+void launch_frag_one(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_frag_kernel<NB, MB, U, W8, AH, EPI, RS>), dim3(8u * (unsigned)t.nms, (unsigned)((t.ntiles + 7) / 8)),
+                       dim3(64 * kFragWaves), 0, s, o.a, o.w, o.K, o.M, t.ntiles, o.row_ss, o.row_tiles, o.row_inv_n,
+                       o.row_eps, e);
+}
+
+template <int NB, int MB, int U, bool W8, bool AH, int EPI>
+void launch_frag_rows(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
+    if constexpr (AH && EPI == SF_EPI_PLAIN) {
+        if (o.row_ss && e.x) {
+            launch_frag_one<NB, MB, U, W8, AH, EPI, kRowGuarded>(o, t, e, s);
+            return;
+        }
     }
+    if constexpr (EPI != SF_EPI_ADD_NORM) {
+        if (o.row_ss) {
+            launch_frag_one<NB, MB, U, W8, AH, EPI, kRowDeferred>(o, t, e, s);
+            return;
+        }
+    }
+    launch_frag_one<NB, MB, U, W8, AH, EPI, kRowPlain>(o, t, e, s);
 }
 
 template <int NB, int MB, int U, int EPI>
 void launch_frag_tile(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
-    if constexpr (EPI != SF_EPI_ADD_NORM) {
-        if (o.row_ss) {
-            launch_frag_rs<NB, MB, U, EPI, true>(o, t, e, s);
-            return;
-        }
+    if (o.w8) {
+        if (o.ah) launch_frag_rows<NB, MB, U, true, true, EPI>(o, t, e, s);
+        else launch_frag_rows<NB, MB, U, true, false, EPI>(o, t, e, s);
+    } else {
+        if (o.ah) launch_frag_rows<NB, MB, U, false, true, EPI>(o, t, e, s);
+        else launch_frag_rows<NB, MB, U, false, false, EPI>(o, t, e, s);
     }
-    launch_frag_rs<NB, MB, U, EPI, false>(o, t, e, s);
 }
 
 // U chunks per group: the loads of two groups about fill the wave's 63-entry
@@ -630,6 +705,15 @@ extern "C" int sf_gemm_frag(const sf_frag_gemm_desc* d, void* stream) {
         o.row_tiles = d->a_row_tiles;
         o.row_inv_n = 1.f / (float)d->a_row_n;
         o.row_eps = d->a_row_eps;
+        if (d->a_x) {   // fp16 rows with the range guard
+            if (d->a_dtype != SF_F16 || d->epilogue != SF_EPI_PLAIN || d->a_row_n != d->K) return SF_ENOTSUP;
+            if (!d->a_x_gamma || d->a_x_ld < d->K) return SF_EINVAL;
+            a.x = d->a_x;
+            a.x_gamma = d->a_x_gamma;
+            a.x_ld = d->a_x_ld;
+        }
+    } else if (d->a_x) {
+        return SF_EINVAL;
     }
     int nb = 0;   // columns per tile where the epilogue fixes them
     if (d->epilogue == SF_EPI_HEADS) {

@@ -124,12 +124,13 @@ struct sf_rdt {
     // Fragment-ordered step (B*S <= 160): every block and final-layer
     // projection is one sf_gemm_frag launch over fragment-ordered weight
     // copies (frag_of) and activations: n, a, n3 and h are in fragment order.
-    // norm1 / norm2 are deferred: the residual adds before them store
-    // x * gamma and per-tile sums of squares (row_ss, [row_tiles][B*S]), and
-    // the QKV and cross-q projections apply the row's 1/rms after their
-    // contraction.  norm3 and the final norm are row-wide launches of their
-    // own (sf_norm_frag): their fp16 outputs need the normalised range.  The
-    // cross-q projection leaves finished fp32 rows (q32); the attention
+    // The blocks' norms are deferred: the residual adds before them store x * gamma
+    // and per-tile sums of squares (row_ss, [B*S][row_tiles]), and the
+    // projection that follows applies the row's 1/rms after its contraction
+    // (fc1, whose fp16 rows can leave fp16's range, with the range guard of
+    // sf_gemm_frag: such rows are normalised from x).  The final norm is a
+    // row-wide launch of its own (sf_norm_frag): its bf16 rounding then falls
+    // on the normalised values, one layer ahead of the output.  The cross-q projection leaves finished fp32 rows (q32); the attention
     // applies q_norm as it loads them.
     bool frag = false;
     float* row_ss = nullptr;
@@ -510,31 +511,27 @@ sf_frag_gemm_desc frag_desc(const sf_rdt* m, const void* A, int a_dtype, int w_i
     return d;
 }
 
-// C = act(A W^T + b): fp32 row-major (accumulate: C +=) or, with frag, in
-// fragment order.
-int frag_linear(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, int act, void* C, int c_dtype,
-                bool c_frag, bool accumulate, hipStream_t s, bool deferred = false) {
+// C = A W^T + b in fp32 rows.
+int frag_linear(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, float* C, hipStream_t s, bool deferred) {
     sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, deferred);
-    d.act = act;
     d.epilogue = SF_EPI_PLAIN;
     d.C = C;
     d.ldc = d.N;
-    d.c_dtype = c_dtype;
-    d.c_frag = c_frag ? 1 : 0;
-    d.accumulate = accumulate ? 1 : 0;
+    d.c_dtype = SF_F32;
     return sf_gemm_frag(&d, s);
 }
 
-// x += A W^T + b; m->n = x * gamma (bf16, fragment order), row_ss = the sums.
-int frag_add_norm(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, int gamma_idx, hipStream_t s) {
+// x += A W^T + b; out = x * gamma (out_dtype, fragment order), row_ss = the sums.
+int frag_add_norm(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, int gamma_idx, void* out,
+                  int out_dtype, hipStream_t s) {
     sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, false);
     d.epilogue = SF_EPI_ADD_NORM;
     d.C = m->x;
     d.ldc = d.N;
     d.c_dtype = SF_F32;
     d.norm_gamma = pf(m, gamma_idx);
-    d.norm_out = m->n;
-    d.norm_dtype = m->act16;
+    d.norm_out = out;
+    d.norm_dtype = out_dtype;
     d.norm_ss = m->row_ss;
     m->row_tiles = sf_gemm_frag_ss_tiles(d.N);
     return sf_gemm_frag(&d, s);
@@ -800,28 +797,42 @@ int write_copies(sf_rdt* m, hipStream_t s) {
 int block_forward_frag(sf_rdt* m, int i, hipStream_t s) {
     const sf_rdt_config& c = m->cfg;
     const LayerIdx& L = m->layers[i];
-    const int D = c.hidden, S = c.horizon + 3, M = c.batch * S;
+    const int D = c.hidden, S = c.horizon + 3;
     const int fd = m->ffn_dtype, ad = m->act16;
     // self-attention branch
     SF_TRY(frag_qkv(m, L, s));
     SF_TRY(attention(m, m->q, m->k, m->v, S, nullptr, m->a, false, s));
-    SF_TRY(frag_add_norm(m, m->a, ad, L.proj_w, L.proj_b, L.norm2, s));
+    SF_TRY(frag_add_norm(m, m->a, ad, L.proj_w, L.proj_b, L.norm2, m->n, ad, s));
     // cross-attention branch: even blocks attend to language, odd to image
     // (dit_block.cu:369); the cached V of a layer on the fp16 P.V form is
     // held in fp16 (sf_bf16_to_f16_below)
     const bool lang = (i % 2) == 0;
     const bool exact = m->exact_pv[i] != 0;
-    SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, SF_ACT_NONE, m->q32, SF_F32, false, false, s, true));
+    SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, m->q32, s, true));
     SF_TRY(attention(m, nullptr, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
                      lang ? m->lang_len : nullptr, m->a, exact, s, lang ? c.lang_max : c.img_len, nullptr, !exact,
                      m->q32, pf(m, L.cq_norm)));
-    SF_TRY(frag_linear(m, m->a, ad, L.cproj_w, L.cproj_b, SF_ACT_NONE, m->x, SF_F32, false, true, s));
-    SF_TRY(sf_norm_frag(m->x, D, pf(m, L.norm3), m->n3, fd, nullptr, M, D, c.eps, s));
+    SF_TRY(frag_add_norm(m, m->a, ad, L.cproj_w, L.cproj_b, L.norm3, m->n3, fd, s));
     // FFN branch (Mlp::forward, dit_block.cu:143-163)
-    SF_TRY(frag_linear(m, m->n3, fd, L.fc1_w, L.fc1_b, SF_ACT_GELU_TANH, m->h, fd, true, false, s));
-    if (i + 1 < c.layers) return frag_add_norm(m, m->h, fd, L.fc2_w, L.fc2_b, m->layers[i + 1].norm1, s);
-    SF_TRY(frag_linear(m, m->h, fd, L.fc2_w, L.fc2_b, SF_ACT_NONE, m->x, SF_F32, false, true, s));
-    return sf_norm_frag(m->x, D, pf(m, m->fnorm), m->n, ad, nullptr, M, D, c.eps, s);
+    sf_frag_gemm_desc d = frag_desc(m, m->n3, fd, L.fc1_w, L.fc1_b, true);
+    d.act = SF_ACT_GELU_TANH;
+    d.epilogue = SF_EPI_PLAIN;
+    d.C = m->h;
+    d.c_dtype = fd;
+    d.c_frag = 1;
+    d.a_x = m->x;
+    d.a_x_ld = D;
+    d.a_x_gamma = pf(m, L.norm3);
+    SF_TRY(sf_gemm_frag(&d, s));
+    if (i + 1 < c.layers) return frag_add_norm(m, m->h, fd, L.fc2_w, L.fc2_b, m->layers[i + 1].norm1, m->n, ad, s);
+    d = frag_desc(m, m->h, fd, L.fc2_w, L.fc2_b, false);
+    d.epilogue = SF_EPI_PLAIN;
+    d.C = m->x;
+    d.ldc = D;
+    d.c_dtype = SF_F32;
+    d.accumulate = 1;
+    SF_TRY(sf_gemm_frag(&d, s));
+    return sf_norm_frag(m->x, D, pf(m, m->fnorm), m->n, ad, nullptr, c.batch * S, D, c.eps, s);
 }
 
 // RDTBlock::forward (dit_block.cu:349-387) on the fp32 residual m->x, with
@@ -874,9 +885,8 @@ int entry_norm(sf_rdt* m, int first, hipStream_t s) {
     const int D = c.hidden, M = c.batch * (c.horizon + 3);
     const int g = first < c.layers ? m->layers[first].norm1 : m->fnorm;
     if (m->frag) {
-        const bool deferred = first < c.layers;   // the final norm is row-wide
-        if (deferred) m->row_tiles = D / 64;
-        return sf_norm_frag(m->x, D, pf(m, g), m->n, m->act16, deferred ? m->row_ss : nullptr, M, D, c.eps, s);
+        m->row_tiles = D / 64;
+        return sf_norm_frag(m->x, D, pf(m, g), m->n, m->act16, m->row_ss, M, D, c.eps, s);
     }
     return sf_rmsnorm(m->x, SF_F32, D, pf(m, g), m->n, m->act16, D, M, D, c.eps, s);
 }
@@ -924,7 +934,7 @@ int step_forward(sf_rdt* m, const float* x_t, float t, hipStream_t s,
         d.c_frag = f2 ? 1 : 0;
         SF_TRY(sf_gemm_frag(&d, s));
         if (f2)
-            return frag_linear(m, m->h, m->ffn_dtype, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, SF_F32, false, false, s);
+            return frag_linear(m, m->h, m->ffn_dtype, m->f2w, m->f2b, m->vel_rows, s, false);
         return linear(m, m->h, D, M, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, A, SF_F32, false, s, m->ffn_dtype);
     }
     SF_TRY(linear(m, m->n, D, M, m->f1w, m->f1b, SF_ACT_GELU_TANH, m->h, D, m->ffn_dtype, false, s, m->act16));

@@ -183,9 +183,10 @@ def _run_frag(d, t):
 
 
 def gemm_frag(M, a, w, bias=None, act=abi.SF_ACT_NONE, out=None, out_dtype=torch.float32, c_frag=False,
-              accumulate=False, w_scale=None, row_ss=None, row_n=0, row_eps=1e-6):
+              accumulate=False, w_scale=None, row_ss=None, row_n=0, row_eps=1e-6, x=None, x_gamma=None):
     """sf_gemm_frag's plain epilogue on M rows of a (fragment order, padded
-    rows) and w (frag_pack): row-major [M, N], or fragment order with c_frag."""
+    rows) and w (frag_pack): row-major [M, N], or fragment order with c_frag.
+    x, x_gamma: the fp32 rows and gamma behind deferred fp16 rows."""
     N = w.shape[0]
     d = _frag_desc(M, a, w, bias, act, w_scale, row_ss, row_n, row_eps)
     if out is None:
@@ -193,6 +194,8 @@ def gemm_frag(M, a, w, bias=None, act=abi.SF_ACT_NONE, out=None, out_dtype=torch
     d.epilogue = abi.SF_EPI_PLAIN
     d.C, d.ldc, d.c_dtype = out.data_ptr(), N if c_frag else out.stride(0), _DT[out.dtype]
     d.c_frag, d.accumulate = int(c_frag), int(accumulate)
+    if x is not None:
+        d.a_x, d.a_x_ld, d.a_x_gamma = x.data_ptr(), x.stride(0), x_gamma.data_ptr()
     _run_frag(d, a)
     return out
 

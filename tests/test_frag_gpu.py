@@ -149,6 +149,31 @@ def test_norm_frag(rows, cols, dt):
     assert rel(ss, x.double().view(rows, -1, 64).square().sum(-1)) < 1e-6
 
 
+@pytest.mark.parametrize("M,N,kind", [(67, 2048, "w16"), (134, 256, "int8"), (81, 4096, "w16"), (160, 2048, "int8")])
+def test_fp16_rows_out_of_range(M, N, kind):
+    """Deferred fp16 rows whose x * gamma leaves fp16's range, is far below
+    it, or is zero: those rows come from the fp32 residual, normalised first;
+    the others are bit for bit what they are without such neighbours."""
+    zero, small, big = 0, 7, M - 1
+    a = torch.zeros(M, 64, dtype=torch.bfloat16, device=DEV)
+    wz = K.frag_pack([torch.zeros(N, 64, dtype=torch.bfloat16, device=DEV)], [torch.bfloat16])[0]
+    gamma, x = 1 + randn(40, N, std=0.1), randn(41, M, N)
+    plain = x.clone()
+    x[zero], x[small], x[big] = 0, x[small] * 1e-6, x[big] * 1e5
+    wf, s, w64 = weights(42, 512, N, kind, torch.float16)
+    b = randn(43, 512)
+    got = []
+    for rows in (x, plain):
+        n, ss = K.gemm_frag_add_norm(M, to_frag(a), wz, None, rows, gamma, norm_dtype=torch.float16)
+        got.append(K.gemm_frag(M, n, wf, b, w_scale=s, row_ss=ss, row_n=N, x=rows, x_gamma=gamma))
+        assert (not torch.isfinite(ss[big].sum())) == (rows is x)
+    ref = (x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-6) * gamma.double()) @ w64.t() + b.double()
+    for r in (zero, small, big, 1):
+        assert rel(got[0][r], ref[r]) < _ROUND[torch.float16]
+    same = [r for r in range(M) if r not in (zero, small, big)]
+    assert torch.equal(got[0][same], got[1][same])
+
+
 # the one-wave and grouped short-key kernels, the query-block grid, key splits
 # with the merge, the unsplit 80-row grid, and fp32 inputs
 @pytest.mark.parametrize("B,H,Sq,Sk,dt", [(1, 32, 67, 67, torch.bfloat16), (8, 32, 67, 67, torch.float16),
