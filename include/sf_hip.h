@@ -492,7 +492,7 @@ typedef struct sf_w16_job {
 int sf_weights_to_f16(const sf_w16_job* jobs, int32_t count, void* stream);
 
 /* ---------------------------------------------------------------------------
- * Fragment-ordered projections: one launch per projection for few rows.
+ * Fragment-ordered projections: one launch per projection.
  *
  * Fragment order of X[R][K] in 16 bits: blocks of 16 rows x 32 columns, block
  * (r / 16, k / 32) at index (r / 16) * (K / 32) + k / 32, 512 elements each;
@@ -508,8 +508,8 @@ size_t sf_frag_elems(int64_t rows, int64_t cols);
 
 /* Row-major weights w [N][ldw] -> out in fragment order, up to
  * SF_CODES_MAX_JOBS matrices per launch: bf16 -> bf16, bf16 -> fp16 (rounded
- * as sf_weights_to_f16 does), fp16 -> fp16, int8 -> int8.  N a multiple of
- * 16, K of 64, ldw of 8, pointers 16-byte aligned. */
+ * as sf_weights_to_f16 does), fp16 -> fp16, int8 -> int8, int8 -> fp16
+ * (exact, the row scale stays with the GEMM).  N a multiple of 16, K of 64, ldw of 8, pointers 16-byte aligned. */
 typedef struct sf_frag_job {
     const void* w;
     int32_t w_dtype;
@@ -532,8 +532,8 @@ int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int
  * the row scale not with SF_EPI_ADD_NORM) with A and W in fragment
  * order, one launch, no workspace: sf_gemm's arithmetic (gemm_bias_act,
  * cuda_backend.cu:337-467) and epilogues over all of K in one workgroup.
- * M <= 160, N a multiple of 32, K of 64.  a_dtype SF_BF16 or SF_F16; w_dtype
- * the same, or SF_I8 with w_scale.  Epilogues:
+ * N a multiple of 32, K of 64.  a_dtype SF_BF16 or SF_F16; w_dtype the same, or
+ * SF_I8; w_scale [N] required for SF_I8, optional else.  Epilogues:
  *   SF_EPI_PLAIN     C row-major (ldc a multiple of 4) in c_dtype, with
  *                    accumulate for SF_F32; or, with c_frag, in fragment
  *                    order (SF_BF16 / SF_F16).
@@ -542,7 +542,7 @@ int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int
  *   SF_EPI_ADD_NORM  the deferred form only: C (fp32) += result, norm_out
  *                    (fragment order, norm_dtype) = C * norm_gamma, and
  *                    norm_ss[m * T + t] = the sum of C[m][n]^2 over tile t's
- *                    columns, T = sf_gemm_frag_ss_tiles(N) <= 64 tiles.
+ *                    columns, T = sf_gemm_frag_ss_tiles(desc) <= 64 tiles.
  * a_row_ss (SF_EPI_PLAIN, SF_EPI_HEADS): as sf_gemm_desc's, but row-major,
  * [M][a_row_tiles].  SF_F16 rows from SF_EPI_ADD_NORM need a_x (SF_EPI_PLAIN):
  * x * gamma can leave fp16's range, which that epilogue marks by an infinite
@@ -582,7 +582,9 @@ typedef struct sf_frag_gemm_desc {
     const float* a_x_gamma;
 } sf_frag_gemm_desc;
 int sf_gemm_frag(const sf_frag_gemm_desc* desc, void* stream);
-int32_t sf_gemm_frag_ss_tiles(int32_t N);
+/* Tile sums per row that SF_EPI_ADD_NORM writes for this call (M, N, a_dtype,
+ * w_dtype are read). */
+int32_t sf_gemm_frag_ss_tiles(const sf_frag_gemm_desc* desc);
 
 /* Static text for a status code. */
 const char* sf_strerror(int status);

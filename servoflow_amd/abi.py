@@ -232,7 +232,7 @@ def lib() -> ctypes.CDLL:
     L.sf_norm_frag.restype = ctypes.c_int
     L.sf_gemm_frag.argtypes = [ctypes.POINTER(FragGemmDesc), vp]
     L.sf_gemm_frag.restype = ctypes.c_int
-    L.sf_gemm_frag_ss_tiles.argtypes = [i32]
+    L.sf_gemm_frag_ss_tiles.argtypes = [ctypes.POINTER(FragGemmDesc)]
     L.sf_gemm_frag_ss_tiles.restype = i32
     L.sf_gemm_num_splits.argtypes = [ctypes.POINTER(GemmDesc)]
     L.sf_gemm_num_splits.restype = ctypes.c_int32

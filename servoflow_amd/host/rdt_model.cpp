@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <array>
 #include <cstring>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -76,6 +77,17 @@ struct LayerIdx {
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// Rows of a step up to which the projections run fragment-ordered; above, the
+// library path (sf_gemm).  Per block of hidden 2048, graph-timed on cold
+// weights, against hipBLASLt with its residual add + RMSNorm launches: 402
+// rows 69 vs 98 us, 536 rows 82 vs 117.  The line lies where the QKV product's
+// 128 x 128 tiles need a second round of workgroups (hidden 2048: 5 x 48 = 240
+// up to 640 rows): five steps of 4 layers take 3.34 vs 3.64 ms at 536 rows,
+// 3.70 vs 4.00 at 603, 4.15 vs 4.14 at 670, 4.48 vs 4.39 at 804.
+// int8_weights = 2 above 160 rows keeps no 16-bit copies and stays with sf_gemm.
+constexpr int64_t kFragStepRows = 640;
+constexpr int64_t kSmallStepRows = 160;   // bf16 projection inputs, per-head QKV epilogue
+
 // The projection weights a block's forward multiplies by.
 std::array<int, 6> block_weights(const LayerIdx& L) {
     return {L.qkv_w, L.proj_w, L.cq_w, L.cproj_w, L.fc1_w, L.fc2_w};
@@ -98,7 +110,7 @@ struct sf_rdt {
     float* x = nullptr;            // [B*S, D] fp32 residual stream
     uint16_t* n = nullptr;         // [B*S, D] bf16 norm1 / norm2 / final-norm output
     uint16_t *q = nullptr, *k = nullptr, *v = nullptr;   // [B, H, S, 64]
-    // Above 160 rows (the library-path GEMMs) the QKV projection is kept as
+    // Above 160 rows the QKV projection is kept as
     // its fp16 output [B*S, 3D] and the cross-q projection's as [B*S, D] in
     // q; the attention reads Q / K / V from those rows and applies q_norm /
     // k_norm as it loads them (sf_attn_desc.q_gamma / k_gamma).
@@ -110,9 +122,9 @@ struct sf_rdt {
     // 16-bit storage points these two move the block output furthest from
     // fp32 arithmetic).  The other inputs -- norm1 /
     // norm2 / final-norm outputs and attention outputs (act16) -- are bf16
-    // while B*S rows run fragment-ordered (<= 160) and fp16 above it,
-    // where the library path multiplies fp16 activations by fp16 copies of
-    // the weights (w16) and keeps its 16-bit products in fp16: with bf16
+    // while there are at most 160 rows and fp16 above, where fp16 activations
+    // are multiplied by fp16 copies of the weights and 16-bit products are
+    // kept in fp16: with bf16
     // inputs and bf16 products a block sat at 1.6-1.8e-3 from fp32
     // arithmetic, with fp16 ones at 0.6-0.8e-3.  fp16 holds magnitudes below
     // 65504: norm outputs stay below sqrt(hidden) * max|gamma|, attention
@@ -121,17 +133,18 @@ struct sf_rdt {
     // long as the model's activations do.
     int32_t ffn_dtype = SF_F16;
     int32_t act16 = SF_BF16;
-    // Fragment-ordered step (B*S <= 160): every block and final-layer
+    // Fragment-ordered step (B*S <= kFragStepRows): every block and final-layer
     // projection is one sf_gemm_frag launch over fragment-ordered weight
-    // copies (frag_of) and activations: n, a, n3 and h are in fragment order.
+    // copies and activations: n, a, n3 and h are in fragment order.
     // The blocks' norms are deferred: the residual adds before them store x * gamma
     // and per-tile sums of squares (row_ss, [B*S][row_tiles]), and the
     // projection that follows applies the row's 1/rms after its contraction
-    // (fc1, whose fp16 rows can leave fp16's range, with the range guard of
+    // (fp16 rows, which can leave fp16's range, with the range guard of
     // sf_gemm_frag: such rows are normalised from x).  The final norm is a
     // row-wide launch of its own (sf_norm_frag): its bf16 rounding then falls
-    // on the normalised values, one layer ahead of the output.  The cross-q projection leaves finished fp32 rows (q32); the attention
-    // applies q_norm as it loads them.
+    // on the normalised values, one layer ahead of the output.  The cross-q projection leaves finished fp32 rows (q32), above 160 rows fp16
+    // ones as the QKV projection does there; the attention applies the
+    // per-head norms as it loads them.
     bool frag = false;
     float* row_ss = nullptr;
     int row_tiles = 0;             // tiles of the sums row_ss holds now
@@ -178,12 +191,13 @@ struct sf_rdt {
     size_t attn_ws_bytes = 0;
     void* gemm_ws = nullptr;       // split-K partial sums, shared by the stream's GEMMs
     size_t gemm_ws_bytes = 0;
-    // Copies of projection weights.  Above 160 rows (w16_params) fp16 copies
-    // of every block's six and the final layer's two (int8 codes widened
-    // exactly, bf16 weights rounded to fp16; sf_weights_to_f16); at most 160
-    // rows (frag_params) fragment-ordered copies of the same matrices in the
-    // type the projection multiplies -- bf16, fp16 for the matrices whose
-    // inputs are fp16 (fc1, fc2, the final fc2), int8 codes (sf_frag_pack).
+    // Copies of projection weights.  Fragment-ordered step (frag_params): every
+    // block's six and the final layer's two in the type the projection
+    // multiplies -- above 160 rows fp16 (int8 codes widened exactly, bf16
+    // weights rounded), at most 160 rows bf16, fp16 for the matrices whose
+    // inputs are fp16 (fc1, fc2, the final fc2), or the int8 codes
+    // (sf_frag_pack).  Otherwise (w16_params) row-major fp16 copies of the same
+    // matrices (sf_weights_to_f16).
     // Up to eight matrices per launch, made before the first pass and again before
     // the first pass after the parameters may have changed (copies_stale), on
     // the pass's stream and outside any graph capture -- not once per loop:
@@ -192,6 +206,8 @@ struct sf_rdt {
     char* copies = nullptr;
     size_t copies_bytes = 0;
     std::vector<void*> copy_of;
+    std::vector<int32_t> copy_dtype;
+    std::vector<char> copy_frag;   // in fragment order (else row-major fp16)
     // The copies may no longer match the weights: set by every call that
     // writes parameters or hands out a pointer to them (and by
     // sf_rdt_params_changed), cleared by the refresh at the start of the
@@ -393,7 +409,7 @@ int linear(sf_rdt* m, const void* A, int64_t lda, int M, int w_idx, int b_idx, i
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
+    d.w_codes16 = m->copy_frag[w_idx] ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = b_idx >= 0 ? pf(m, b_idx) : nullptr;
     d.act = act;
@@ -426,7 +442,7 @@ int linear_add_norm(sf_rdt* m, const void* A, int a_dtype, int M, int w_idx, int
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
+    d.w_codes16 = m->copy_frag[w_idx] ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = pf(m, b_idx);
     d.epilogue = SF_EPI_ADD_NORM;
@@ -464,7 +480,7 @@ int linear_heads(sf_rdt* m, const void* A, int M, int S, int w_idx, int b_idx,
     d.ldw = W.shape[1];
     d.w_dtype = W.dtype;
     d.w_scale = W.scale;
-    d.w_codes16 = m->frag ? nullptr : m->copy_of[w_idx];
+    d.w_codes16 = m->copy_frag[w_idx] ? nullptr : m->copy_of[w_idx];
     d.w16_f16 = d.w_codes16 ? 1 : 0;
     d.bias = pf(m, b_idx);
     d.epilogue = SF_EPI_HEADS;
@@ -499,7 +515,7 @@ sf_frag_gemm_desc frag_desc(const sf_rdt* m, const void* A, int a_dtype, int w_i
     d.A = A;
     d.a_dtype = a_dtype;
     d.W = m->copy_of[w_idx];
-    d.w_dtype = W.dtype == SF_I8 ? SF_I8 : a_dtype;
+    d.w_dtype = m->copy_dtype[w_idx];
     d.w_scale = W.scale;
     d.bias = static_cast<const float*>(m->params[b_idx].data);
     if (deferred) {
@@ -511,13 +527,24 @@ sf_frag_gemm_desc frag_desc(const sf_rdt* m, const void* A, int a_dtype, int w_i
     return d;
 }
 
-// C = A W^T + b in fp32 rows.
-int frag_linear(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, float* C, hipStream_t s, bool deferred) {
-    sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, deferred);
+// The range guard of deferred fp16 rows (bf16 rows need none).
+void set_guard(const sf_rdt* m, sf_frag_gemm_desc& d, int gamma_idx) {
+    if (d.a_dtype != SF_F16) return;
+    d.a_x = m->x;
+    d.a_x_ld = m->cfg.hidden;
+    d.a_x_gamma = static_cast<const float*>(m->params[gamma_idx].data);
+}
+
+// C = A W^T + b in row-major rows (c_dtype); gamma_idx >= 0: A holds the
+// deferred rows of the norm with that gamma.
+int frag_linear(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, void* C, int c_dtype, hipStream_t s,
+                int gamma_idx = -1) {
+    sf_frag_gemm_desc d = frag_desc(m, A, a_dtype, w_idx, b_idx, gamma_idx >= 0);
     d.epilogue = SF_EPI_PLAIN;
     d.C = C;
     d.ldc = d.N;
-    d.c_dtype = SF_F32;
+    d.c_dtype = c_dtype;
+    if (gamma_idx >= 0) set_guard(m, d, gamma_idx);
     return sf_gemm_frag(&d, s);
 }
 
@@ -533,7 +560,7 @@ int frag_add_norm(sf_rdt* m, const void* A, int a_dtype, int w_idx, int b_idx, i
     d.norm_out = out;
     d.norm_dtype = out_dtype;
     d.norm_ss = m->row_ss;
-    m->row_tiles = sf_gemm_frag_ss_tiles(d.N);
+    m->row_tiles = sf_gemm_frag_ss_tiles(&d);
     return sf_gemm_frag(&d, s);
 }
 
@@ -568,6 +595,23 @@ struct RowsIn {
     const float* k_gamma = nullptr;
     bool f16 = false;    // rows in fp16: with kv_ld, Q, K and V (an fp16 attention); else Q only
 };
+
+// The QKV projection's rows (self-attention), and the cross-q projection's.
+RowsIn qkv_rows_in(const sf_rdt* m, const LayerIdx& L) {
+    RowsIn r;
+    r.q_ld = r.kv_ld = 3 * m->cfg.hidden;
+    r.q_gamma = static_cast<const float*>(m->params[L.q_norm].data);
+    r.k_gamma = static_cast<const float*>(m->params[L.k_norm].data);
+    r.f16 = m->act16 == SF_F16;
+    return r;
+}
+RowsIn cross_rows_in(const sf_rdt* m, const LayerIdx& L) {
+    RowsIn r;
+    r.q_ld = m->cfg.hidden;
+    r.q_gamma = static_cast<const float*>(m->params[L.cq_norm].data);
+    r.f16 = m->act16 == SF_F16;
+    return r;
+}
 
 // Sc: the rows per head of the K/V buffer (its capacity), Sk <= Sc the keys
 // read.  q32: Q as fp32 projection rows, normalised with q32_gamma, instead
@@ -627,8 +671,8 @@ int attention(sf_rdt* m, const uint16_t* q, const uint16_t* k, const uint16_t* v
     return sf_attn_fwd(&d, q, k, v, out, m->attn_ws, m->attn_ws_bytes, s);
 }
 
-// The projection weights that get fp16 copies above 160 rows (the library
-// path): every block's six and the final layer's two, where K is a multiple
+// The projection weights that get row-major fp16 copies, for calls of sf_gemm
+// with fp16 activations: outside the fragment-ordered step every block's six and the final layer's two, where K is a multiple
 // of 16.  With int8_weights = 2, no copy of the int8 matrices sf_gemm
 // multiplies directly at the block's rows (sf_gemm_int8_direct; every such
 // call the block makes has fp16 activations and a 16-bit fp16 product).
@@ -636,7 +680,9 @@ std::vector<int> w16_params(const sf_rdt* m) {
     const sf_rdt_config& c = m->cfg;
     std::vector<int> ws;
     const int rows = c.batch * (c.horizon + 3);
-    if (rows > 160) {
+    if (m->frag) {   // the final fc2 when its columns do not fill the fragment tiles
+        if (c.action_dim % 32) ws.push_back(m->f2w);
+    } else {
         for (const LayerIdx& L : m->layers)
             for (int w : block_weights(L)) ws.push_back(w);
         ws.push_back(m->f1w);
@@ -666,21 +712,23 @@ std::vector<int> w16_params(const sf_rdt* m) {
     return out;
 }
 
-// The weights that get fragment-ordered copies (at most 160 rows) and their
-// copies' types: fp16 where the projection's input is fp16 (fc1, fc2, the
-// final fc2), else bf16; int8 weights keep their codes.  The final fc2 joins
-// when its columns fill 32-wide tiles.
+// The weights that get fragment-ordered copies and their copies' types: fp16
+// where the projection's input is fp16 (fc1, fc2, the final fc2; all above 160
+// rows), else bf16; at most 160 rows int8 weights keep their codes (above, the
+// widening would cost each row tile).  The final fc2 joins when its columns
+// fill 32-wide tiles.
 std::vector<std::pair<int, int32_t>> frag_params(const sf_rdt* m) {
     std::vector<std::pair<int, int32_t>> out;
     if (!m->frag) return out;
     auto add = [&](int w, int32_t dt) {
-        out.emplace_back(w, m->params[w].dtype == SF_I8 ? (int32_t)SF_I8 : dt);
+        const bool codes = m->params[w].dtype == SF_I8 && m->act16 == SF_BF16;
+        out.emplace_back(w, codes ? (int32_t)SF_I8 : dt);
     };
     for (const LayerIdx& L : m->layers) {
-        for (int w : {L.qkv_w, L.proj_w, L.cq_w, L.cproj_w}) add(w, SF_BF16);
+        for (int w : {L.qkv_w, L.proj_w, L.cq_w, L.cproj_w}) add(w, m->act16);
         for (int w : {L.fc1_w, L.fc2_w}) add(w, SF_F16);
     }
-    add(m->f1w, SF_BF16);
+    add(m->f1w, m->act16);
     if (m->cfg.action_dim % 32 == 0) add(m->f2w, SF_F16);
     return out;
 }
@@ -700,14 +748,14 @@ size_t gemm_ws_for(const sf_rdt* m, bool prepare, int* status) {
                          c.batch * c.lang_max, c.batch * c.img_len,
                          std::min(160, c.lang_max)};   // largest split-K M (language rows at batch 1)
     size_t best = 0;
-    // weights with an fp16 copy (above 160 rows) multiply fp16 activations
-    // in fp16 on the library path
-    std::vector<char> w16(m->params.size(), 0);
-    if (c.batch * (c.horizon + 3) > 160)
-        for (int w : w16_params(m)) w16[w] = 1;
+    // weights with a row-major fp16 copy multiply fp16 activations in fp16 on
+    // the library path; those with a fragment-ordered copy never reach sf_gemm
+    std::vector<char> w16(m->params.size(), 0), frag(m->params.size(), 0);
+    for (int w : w16_params(m)) w16[w] = 1;
+    for (const auto& f : frag_params(m)) frag[f.first] = 1;
     for (size_t pi = 0; pi < m->params.size(); ++pi) {
         const Param& p = m->params[pi];
-        if (p.shape.size() != 2 || p.dtype == SF_F32) continue;
+        if (p.shape.size() != 2 || p.dtype == SF_F32 || frag[pi]) continue;
         for (int M : rows) {
             for (int ad : {SF_BF16, SF_F16}) {
                 sf_gemm_desc d{};
@@ -764,7 +812,7 @@ int next_norm(const sf_rdt* m, int i) {
 // Rewrites every weight copy from the parameters, up to SF_CODES_MAX_JOBS
 // matrices per launch.
 int write_copies(sf_rdt* m, hipStream_t s) {
-    if (m->frag) {
+    {
         sf_frag_job jobs[SF_CODES_MAX_JOBS];
         int n = 0;
         for (const auto& f : frag_params(m)) {
@@ -776,7 +824,7 @@ int write_copies(sf_rdt* m, hipStream_t s) {
                 n = 0;
             }
         }
-        return n ? sf_frag_pack(jobs, n, s) : SF_OK;
+        if (n) SF_TRY(sf_frag_pack(jobs, n, s));
     }
     sf_w16_job jobs[SF_CODES_MAX_JOBS];
     int n = 0;
@@ -799,19 +847,33 @@ int block_forward_frag(sf_rdt* m, int i, hipStream_t s) {
     const LayerIdx& L = m->layers[i];
     const int D = c.hidden, S = c.horizon + 3;
     const int fd = m->ffn_dtype, ad = m->act16;
+    const bool rows16 = ad == SF_F16;   // more than 160 rows: fp16 q / k / v rows, normed as they are loaded
     // self-attention branch
-    SF_TRY(frag_qkv(m, L, s));
-    SF_TRY(attention(m, m->q, m->k, m->v, S, nullptr, m->a, false, s));
+    if (rows16) {
+        SF_TRY(frag_linear(m, m->n, ad, L.qkv_w, L.qkv_b, m->qkv_rows, ad, s, L.norm1));
+        const RowsIn r = qkv_rows_in(m, L);
+        SF_TRY(attention(m, m->qkv_rows, m->qkv_rows + D, m->qkv_rows + 2 * D, S, nullptr, m->a, false, s, 0, &r));
+    } else {
+        SF_TRY(frag_qkv(m, L, s));
+        SF_TRY(attention(m, m->q, m->k, m->v, S, nullptr, m->a, false, s));
+    }
     SF_TRY(frag_add_norm(m, m->a, ad, L.proj_w, L.proj_b, L.norm2, m->n, ad, s));
     // cross-attention branch: even blocks attend to language, odd to image
     // (dit_block.cu:369); the cached V of a layer on the fp16 P.V form is
     // held in fp16 (sf_bf16_to_f16_below)
     const bool lang = (i % 2) == 0;
     const bool exact = m->exact_pv[i] != 0;
-    SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, m->q32, s, true));
-    SF_TRY(attention(m, nullptr, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
-                     lang ? m->lang_len : nullptr, m->a, exact, s, lang ? c.lang_max : c.img_len, nullptr, !exact,
-                     m->q32, pf(m, L.cq_norm)));
+    const int keys = lang ? m->cond_lang_rows : c.img_len, cap = lang ? c.lang_max : c.img_len;
+    const int32_t* valid = lang ? m->lang_len : nullptr;
+    if (rows16) {
+        SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, m->q, ad, s, L.norm2));
+        const RowsIn r = cross_rows_in(m, L);
+        SF_TRY(attention(m, m->q, m->ck[i], m->cv[i], keys, valid, m->a, exact, s, cap, &r, !exact));
+    } else {
+        SF_TRY(frag_linear(m, m->n, ad, L.cq_w, L.cq_b, m->q32, SF_F32, s, L.norm2));
+        SF_TRY(attention(m, nullptr, m->ck[i], m->cv[i], keys, valid, m->a, exact, s, cap, nullptr, !exact, m->q32,
+                         pf(m, L.cq_norm)));
+    }
     SF_TRY(frag_add_norm(m, m->a, ad, L.cproj_w, L.cproj_b, L.norm3, m->n3, fd, s));
     // FFN branch (Mlp::forward, dit_block.cu:143-163)
     sf_frag_gemm_desc d = frag_desc(m, m->n3, fd, L.fc1_w, L.fc1_b, true);
@@ -820,9 +882,7 @@ int block_forward_frag(sf_rdt* m, int i, hipStream_t s) {
     d.C = m->h;
     d.c_dtype = fd;
     d.c_frag = 1;
-    d.a_x = m->x;
-    d.a_x_ld = D;
-    d.a_x_gamma = pf(m, L.norm3);
+    set_guard(m, d, L.norm3);
     SF_TRY(sf_gemm_frag(&d, s));
     if (i + 1 < c.layers) return frag_add_norm(m, m->h, fd, L.fc2_w, L.fc2_b, m->layers[i + 1].norm1, m->n, ad, s);
     d = frag_desc(m, m->h, fd, L.fc2_w, L.fc2_b, false);
@@ -848,11 +908,7 @@ int block_forward(sf_rdt* m, int i, hipStream_t s) {
     // split_qkv and apply_qk_norm (:209-220) happen as the attention loads
     // the rows
     SF_TRY(linear(m, m->n, D, M, L.qkv_w, L.qkv_b, SF_ACT_NONE, m->qkv_rows, 3 * D, ad, false, s, ad));
-    RowsIn r;
-    r.q_ld = r.kv_ld = 3 * D;
-    r.q_gamma = pf(m, L.q_norm);
-    r.k_gamma = pf(m, L.k_norm);
-    r.f16 = ad == SF_F16;
+    const RowsIn r = qkv_rows_in(m, L);
     SF_TRY(attention(m, m->qkv_rows, m->qkv_rows + D, m->qkv_rows + 2 * D, S, nullptr, m->a, false, s, 0, &r));
     SF_TRY(linear_add_norm(m, m->a, ad, M, L.proj_w, L.proj_b, L.norm2, m->n, ad, s));
     // cross-attention branch: even blocks attend to language, odd to image
@@ -865,10 +921,7 @@ int block_forward(sf_rdt* m, int i, hipStream_t s) {
     // q_norm (:298-307) happen as the attention loads them (rounding Q to
     // bf16 for the bf16 K/V cache)
     SF_TRY(linear(m, m->n, D, M, L.cq_w, L.cq_b, SF_ACT_NONE, m->q, D, ad, false, s, ad));
-    RowsIn cr;
-    cr.q_ld = D;
-    cr.q_gamma = pf(m, L.cq_norm);
-    cr.f16 = ad == SF_F16;
+    const RowsIn cr = cross_rows_in(m, L);
     SF_TRY(attention(m, m->q, m->ck[i], m->cv[i], lang ? m->cond_lang_rows : c.img_len,
                      lang ? m->lang_len : nullptr, m->a, exact, s, lang ? c.lang_max : c.img_len, &cr, !exact));
     SF_TRY(linear_add_norm(m, m->a, ad, M, L.cproj_w, L.cproj_b, L.norm3, m->n3, fd, s));
@@ -924,7 +977,7 @@ int step_forward(sf_rdt* m, const float* x_t, float t, hipStream_t s,
     for (int i = 0; i < c.layers; ++i) SF_TRY(block_forward(m, i, s));
     // FinalLayer (dit_block.cu:407-412); m->n = norm_final(x) from the last block
     if (m->frag) {
-        const bool f2 = m->copy_of[m->f2w] != nullptr;   // else row-major into the split-K kernel
+        const bool f2 = m->copy_frag[m->f2w] != 0;   // else row-major into sf_gemm
         sf_frag_gemm_desc d = frag_desc(m, m->n, m->act16, m->f1w, m->f1b, false);
         d.act = SF_ACT_GELU_TANH;
         d.epilogue = SF_EPI_PLAIN;
@@ -934,7 +987,7 @@ int step_forward(sf_rdt* m, const float* x_t, float t, hipStream_t s,
         d.c_frag = f2 ? 1 : 0;
         SF_TRY(sf_gemm_frag(&d, s));
         if (f2)
-            return frag_linear(m, m->h, m->ffn_dtype, m->f2w, m->f2b, m->vel_rows, s, false);
+            return frag_linear(m, m->h, m->ffn_dtype, m->f2w, m->f2b, m->vel_rows, SF_F32, s);
         return linear(m, m->h, D, M, m->f2w, m->f2b, SF_ACT_NONE, m->vel_rows, A, SF_F32, false, s, m->ffn_dtype);
     }
     SF_TRY(linear(m, m->n, D, M, m->f1w, m->f1b, SF_ACT_GELU_TANH, m->h, D, m->ffn_dtype, false, s, m->act16));
@@ -1045,8 +1098,9 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     // fp16 FFN inputs at every batch size; the other projection inputs in
     // fp16 once the block GEMMs leave the fragment-ordered step (M > 160 rows)
     m->ffn_dtype = SF_F16;
-    m->act16 = c.batch * (c.horizon + 3) <= 160 ? SF_BF16 : SF_F16;
-    m->frag = c.batch * (c.horizon + 3) <= 160;
+    const int64_t step_rows = (int64_t)c.batch * (c.horizon + 3);
+    m->act16 = step_rows <= kSmallStepRows ? SF_BF16 : SF_F16;
+    m->frag = step_rows <= (c.int8_weights == 2 ? kSmallStepRows : kFragStepRows);
     build_param_table(m);
 
     const int64_t B = c.batch, D = c.hidden, T = c.horizon, S = T + 3, A = c.action_dim;
@@ -1144,12 +1198,14 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     if (m->kv_prod_bytes) bufs.push_back({(void**)&m->kv_prod, m->kv_prod_bytes});
     m->gemm_ws_bytes = gemm_ws_for(m, false, nullptr);
     bufs.push_back({&m->gemm_ws, std::max<size_t>(m->gemm_ws_bytes, 256)});
-    if (!m->frag) bufs.push_back({(void**)&m->qkv_rows, (size_t)(B * S * 3 * D * 2)});
+    if (m->act16 == SF_F16) bufs.push_back({(void**)&m->qkv_rows, (size_t)(B * S * 3 * D * 2)});
     if (m->frag) {
         bufs.push_back({(void**)&m->row_ss, (size_t)((D + 31) / 32) * B * S * 4});
-        bufs.push_back({(void**)&m->q32, (size_t)(B * S * D * 4)});
+        if (m->act16 == SF_BF16) bufs.push_back({(void**)&m->q32, (size_t)(B * S * D * 4)});
     }
     std::vector<std::pair<int, int32_t>> copies = frag_params(m);   // weight copies
+    std::set<int> frag;
+    for (const auto& f : copies) frag.insert(f.first);
     for (int w : w16_params(m)) copies.emplace_back(w, (int32_t)SF_F16);
     for (const auto& cp : copies) m->copies_bytes += copy_bytes(m, cp.first, cp.second);
     if (m->copies_bytes) bufs.push_back({(void**)&m->copies, m->copies_bytes});
@@ -1176,10 +1232,14 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     }
     for (size_t i = 0; i < bufs.size(); ++i) *bufs[i].ptr = m->arena + boff[i];
     m->copy_of.assign(m->params.size(), nullptr);
+    m->copy_dtype.assign(m->params.size(), SF_F32);
+    m->copy_frag.assign(m->params.size(), 0);
     if (m->copies) {
         char* dst = m->copies;
         for (const auto& cp : copies) {
             m->copy_of[cp.first] = dst;
+            m->copy_dtype[cp.first] = cp.second;
+            m->copy_frag[cp.first] = frag.count(cp.first) ? 1 : 0;
             dst += copy_bytes(m, cp.first, cp.second);
         }
     }

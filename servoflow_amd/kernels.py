@@ -219,7 +219,7 @@ def gemm_frag_add_norm(M, a, w, bias, residual, gamma, norm_dtype=torch.bfloat16
     N = w.shape[0]
     d = _frag_desc(M, a, w, bias, abi.SF_ACT_NONE, w_scale, None, 0, 0.0)
     out = torch.empty((M + 15) // 16 * 16, N, dtype=norm_dtype, device=a.device)
-    ss = torch.empty(M, abi.lib().sf_gemm_frag_ss_tiles(N), dtype=torch.float32, device=a.device)
+    ss = torch.empty(M, abi.lib().sf_gemm_frag_ss_tiles(ctypes.byref(d)), dtype=torch.float32, device=a.device)
     d.epilogue = abi.SF_EPI_ADD_NORM
     d.C, d.ldc, d.c_dtype = residual.data_ptr(), residual.stride(0), abi.SF_F32
     d.norm_gamma, d.norm_out, d.norm_dtype, d.norm_ss = gamma.data_ptr(), out.data_ptr(), _DT[norm_dtype], ss.data_ptr()

@@ -65,16 +65,22 @@ def test_pack_layouts():
     w = randn(1, 48, 192, dtype=torch.bfloat16)
     wide = randn(2, 32, 264, dtype=torch.bfloat16)[:, :256]           # row stride 264
     q = torch.randint(-128, 128, (16, 128), dtype=torch.int8, device=DEV)
-    a, b, c, d = K.frag_pack([w, w, wide, q], [torch.bfloat16, torch.float16, torch.bfloat16, torch.int8])
+    a, b, c, d, e = K.frag_pack([w, w, wide, q, q], [torch.bfloat16, torch.float16, torch.bfloat16, torch.int8,
+                                                     torch.float16])
+    assert torch.equal(e, to_frag(q.to(torch.float16)))
     assert torch.equal(a, to_frag(w)) and torch.equal(b, to_frag(w.to(torch.float16)))
     assert torch.equal(c, to_frag(wide.contiguous())) and torch.equal(d, i8_frag(q))
 
 
-# row tiles of 2, 3 and 5 blocks, partial last blocks, one row, the largest M;
-# column tiles of 32 and 64, more than 256 of them; K of one chunk, of fewer
-# chunks than waves x groups, and ragged over the waves
+# every tile of the rule -- row tiles of 2 to 9 blocks with partial last
+# blocks, one row; column tiles of 32, 64 and 128, more than 256 of them, a
+# count that is no multiple of 8 -- and K of one chunk, of fewer chunks than
+# waves x groups, and ragged over the waves
 @pytest.mark.parametrize("M,N,Kd", [(67, 2048, 2048), (1, 64, 64), (16, 128, 2048), (134, 2048, 2048), (160, 6144, 192),
-                                    (67, 6144, 1088), (81, 96, 320), (33, 32, 4096), (134, 8192, 576), (67, 2048, 8192)])
+                                    (67, 6144, 1088), (81, 96, 320), (33, 32, 4096), (134, 8192, 576), (67, 2048, 8192),
+                                    (402, 2048, 320), (539, 2048, 192), (640, 2048, 256), (603, 6144, 2048),
+                                    (500, 6144, 448), (1072, 2048, 64), (1000, 2048, 704), (450, 6144, 128),
+                                    (700, 4096, 128), (999, 384, 192)])
 @pytest.mark.parametrize("kind,adt", [("w16", torch.bfloat16), ("w16", torch.float16), ("int8", torch.bfloat16),
                                       ("int8", torch.float16)])
 def test_plain(M, N, Kd, kind, adt):
@@ -94,19 +100,23 @@ def test_plain(M, N, Kd, kind, adt):
     assert rel(from_frag(h, M), href) < _ROUND[torch.float16]
 
 
-def test_row_does_not_depend_on_the_batch():
-    a, (wf, _, _) = randn(7, 160, 2048, dtype=torch.bfloat16), weights(8, 2048, 2048, "w16", torch.bfloat16)
-    full = K.gemm_frag(160, to_frag(a), wf)
-    for M in (1, 17, 67, 134):
-        assert torch.equal(K.gemm_frag(M, to_frag(a[:M].contiguous()), wf), full[:M])
+@pytest.mark.parametrize("kind,dt,full", [("w16", torch.bfloat16, 160), ("int8", torch.float16, 160),
+                                          ("w16", torch.float16, 1072)])
+def test_row_does_not_depend_on_the_batch(kind, dt, full):
+    a, (wf, s, _) = randn(7, full, 2048, dtype=dt), weights(8, 2048, 2048, kind, dt)
+    whole = K.gemm_frag(full, to_frag(a), wf, w_scale=s)
+    for M in (1, 17, 67, 134, 402, 804, 1072):
+        if M < full:
+            assert torch.equal(K.gemm_frag(M, to_frag(a[:M].contiguous()), wf, w_scale=s), whole[:M])
 
 
-@pytest.mark.parametrize("M,N", [(67, 2048), (134, 2048), (5, 64), (97, 4096)])
-@pytest.mark.parametrize("kind,ndt", [("w16", torch.bfloat16), ("int8", torch.float16)])
-def test_add_norm_and_its_consumer(M, N, kind, ndt):
+@pytest.mark.parametrize("M,N", [(67, 2048), (134, 2048), (5, 64), (97, 4096), (640, 2048), (1072, 2048), (402, 1024)])
+@pytest.mark.parametrize("kind,adt,ndt", [("w16", torch.bfloat16, torch.bfloat16), ("int8", torch.bfloat16, torch.float16),
+                                          ("w16", torch.float16, torch.float16)])
+def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
     """The deferred pair: x * gamma and tile sums out of one projection, the
     row scale applied by the next, against the normalised rows' product."""
-    a, (wf, s, w64) = randn(9, M, 512, dtype=torch.bfloat16), weights(10, N, 512, kind, torch.bfloat16)
+    a, (wf, s, w64) = randn(9, M, 512, dtype=adt), weights(10, N, 512, kind, adt)
     b, gamma, x = randn(11, N), 1 + randn(12, N, std=0.1), randn(13, M, N)
     xr = x.double() + a.double() @ w64.t() + b.double()
     n, ss = K.gemm_frag_add_norm(M, to_frag(a), wf, b, x, gamma, norm_dtype=ndt, w_scale=s)
@@ -149,7 +159,8 @@ def test_norm_frag(rows, cols, dt):
     assert rel(ss, x.double().view(rows, -1, 64).square().sum(-1)) < 1e-6
 
 
-@pytest.mark.parametrize("M,N,kind", [(67, 2048, "w16"), (134, 256, "int8"), (81, 4096, "w16"), (160, 2048, "int8")])
+@pytest.mark.parametrize("M,N,kind", [(67, 2048, "w16"), (134, 256, "int8"), (81, 4096, "w16"), (160, 2048, "int8"),
+                                      (640, 2048, "w16"), (1072, 512, "w16")])
 def test_fp16_rows_out_of_range(M, N, kind):
     """Deferred fp16 rows whose x * gamma leaves fp16's range, is far below
     it, or is zero: those rows come from the fp32 residual, normalised first;
@@ -236,7 +247,7 @@ def test_refused():
 
     assert call() == abi.SF_OK
     torch.cuda.synchronize()
-    for kw, st in [({"M": 161}, abi.SF_ENOTSUP), ({"K": 32}, abi.SF_ENOTSUP), ({"N": 16}, abi.SF_ENOTSUP),
+    for kw, st in [({"K": 32}, abi.SF_ENOTSUP), ({"N": 16}, abi.SF_ENOTSUP),
                    ({"a_dtype": abi.SF_F32}, abi.SF_ENOTSUP), ({"w_dtype": abi.SF_F16}, abi.SF_ENOTSUP),
                    ({"w_dtype": abi.SF_I8}, abi.SF_EINVAL), ({"ldc": 62}, abi.SF_EINVAL), ({"C": out.data_ptr() + 4}, abi.SF_EINVAL),
                    ({"c_frag": 1}, abi.SF_EINVAL), ({"epilogue": abi.SF_EPI_PARTIALS}, abi.SF_ENOTSUP),
