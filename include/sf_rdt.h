@@ -195,7 +195,9 @@ int sf_rdt_denoise_step(sf_rdt* m, const float* x_t, float t, float* velocity, v
 
 /* x[B, T, A] (fp32, device) <- num_steps Euler steps from t = 1 to 0.
  * use_graph != 0 captures the loop into a hipGraph on the first call and
- * replays it afterwards (inputs are copied in and out around the graph). */
+ * replays it afterwards (inputs are copied in and out around the graph).
+ * Like every entry point here it works on the stream it is given, NULL being
+ * the device's default stream. */
 int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* stream);
 
 /* InferenceEngine::infer (src/engine/inference_engine.cpp:99-175) on this

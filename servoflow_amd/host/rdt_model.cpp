@@ -104,7 +104,12 @@ struct sf_rdt {
 
     char* arena = nullptr;
     size_t arena_bytes = 0;
-    hipStream_t own_stream = nullptr;
+    // Records the sampler's graph for callers on the NULL stream, which cannot
+    // capture.  Nothing else runs on it: work for the NULL stream moved to a
+    // stream of the model's own made the device wait at both ends of every
+    // pass, about 100 us of an eager two-block pass.  Non-blocking, so a
+    // capture in progress stays apart from NULL-stream work of other threads.
+    hipStream_t capture_stream = nullptr;
 
     // activations (batch B, sequence S = horizon + 3)
     float* x = nullptr;            // [B*S, D] fp32 residual stream
@@ -217,6 +222,7 @@ struct sf_rdt {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     hipStream_t graph_stream = nullptr;
+    hipEvent_t graph_event = nullptr;   // after the last launch
 
     // P.V form of each block's cross-attention.  The fast fp16 form holds a
     // cached V element only below 65504 in magnitude; sf_rdt_set_condition
@@ -1017,8 +1023,12 @@ int sample_body(sf_rdt* m, hipStream_t s) {
     return SF_OK;
 }
 
+// The graph is taken down once its last launch is through.
 void release_graph(sf_rdt* m) {
-    if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
+    if (m->graph_exec) {
+        (void)hipEventSynchronize(m->graph_event);   // never recorded: returns at once
+        (void)hipGraphExecDestroy(m->graph_exec);
+    }
     if (m->graph) (void)hipGraphDestroy(m->graph);
     m->graph_exec = nullptr;
     m->graph = nullptr;
@@ -1040,10 +1050,6 @@ int resolve_pv_forms(sf_rdt* m) {
     if (changed) release_graph(m);
     m->forms_gen = m->cond_gen;
     return SF_OK;
-}
-
-hipStream_t pick_stream(sf_rdt* m, void* stream) {
-    return stream ? static_cast<hipStream_t>(stream) : m->own_stream;
 }
 
 // The weight copies, brought up to date before a pass (never under capture:
@@ -1245,12 +1251,13 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     }
     m->exact_pv.assign(c.layers, 0);
     m->lang_rows = m->cond_lang_rows = c.lang_max;
-    if (hipStreamCreate(&m->own_stream) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&m->capture_stream, hipStreamNonBlocking) != hipSuccess) {
         (void)hipFree(m->arena);
         delete m;
         return SF_EDEVICE;
     }
     if (hipEventCreateWithFlags(&m->cond_event, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&m->graph_event, hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc((void**)&m->v_absmax_host, (size_t)std::max(c.layers, 1) * 4) != hipSuccess) {
         sf_rdt_destroy(m);
         return SF_EDEVICE;
@@ -1302,15 +1309,16 @@ extern "C" void sf_rdt_destroy(sf_rdt* m) {
     if (!m) return;
     release_graph(m);
     if (m->cond_event) (void)hipEventDestroy(m->cond_event);
+    if (m->graph_event) (void)hipEventDestroy(m->graph_event);
     if (m->v_absmax_host) (void)hipHostFree(m->v_absmax_host);
-    if (m->own_stream) (void)hipStreamDestroy(m->own_stream);
+    if (m->capture_stream) (void)hipStreamDestroy(m->capture_stream);
     if (m->arena) (void)hipFree(m->arena);
     delete m;
 }
 
 extern "C" int sf_rdt_init_random(sf_rdt* m, uint64_t seed, float std, void* stream) {
     if (!m) return SF_EINVAL;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     for (size_t i = 0; i < m->params.size(); ++i) {
         Param& p = m->params[i];
         const uint64_t ps = seed * 0x100000001B3ull + 0x9E37ull * (i + 1);
@@ -1376,7 +1384,7 @@ extern "C" int sf_rdt_set_condition(sf_rdt* m, const void* lang_c, const int32_t
     if (!m || !lang_c || !lang_len || !img_c || !state_tok) return SF_EINVAL;
     m->infer_cond_valid = false;   // sf_rdt_infer re-encodes after a condition set here
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     const int D = c.hidden, B = c.batch;
     if (lang_len != m->lang_len)
         SF_HIP(hipMemcpyAsync(m->lang_len, lang_len, B * 4, hipMemcpyDeviceToDevice, s));
@@ -1499,7 +1507,7 @@ extern "C" int sf_rdt_encode_condition(sf_rdt* m, const void* lang_tokens, const
                                        const void* img_tokens, const void* state, void* stream) {
     if (!m || !lang_tokens || !lang_len || !img_tokens || !state) return SF_EINVAL;
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     const int D = c.hidden, B = c.batch;
     // lang_adaptor: mlp2x_gelu 4096 -> D -> D (rdt1b.cpp:118-120, 185), over
     // the L token rows at batch 1
@@ -1531,7 +1539,7 @@ extern "C" int sf_rdt_encode_condition(sf_rdt* m, const void* lang_tokens, const
 extern "C" int sf_rdt_run_blocks(sf_rdt* m, float* x, int32_t first, int32_t count, void* stream) {
     if (!m || !x || first < 0 || count < 0 || first + count > m->cfg.layers) return SF_EINVAL;
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     SF_TRY(resolve_pv_forms(m));
     const size_t nbytes = (size_t)c.batch * (c.horizon + 3) * c.hidden * 4;
     SF_TRY(refresh_copies(m, s));
@@ -1546,7 +1554,7 @@ extern "C" int sf_rdt_denoise_step(sf_rdt* m, const float* x_t, float t, float* 
                                    void* stream) {
     if (!m || !x_t || !velocity) return SF_EINVAL;
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     SF_TRY(resolve_pv_forms(m));
     SF_TRY(refresh_copies(m, s));
     SF_TRY(step_forward(m, x_t, t, s));
@@ -1560,7 +1568,7 @@ extern "C" int sf_rdt_denoise_step(sf_rdt* m, const float* x_t, float t, float* 
 extern "C" int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* stream) {
     if (!m || !x) return SF_EINVAL;
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     SF_TRY(resolve_pv_forms(m));
     SF_TRY(refresh_copies(m, s));
     const size_t nbytes = (size_t)c.batch * c.horizon * c.action_dim * 4;
@@ -1569,10 +1577,11 @@ extern "C" int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* strea
     if (use_graph) {
         if (m->graph_exec && m->graph_stream != s) release_graph(m);
         if (!m->graph_exec) {
-            SF_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            const int st = sample_body(m, s);
+            const hipStream_t cs = s ? s : m->capture_stream;
+            SF_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+            const int st = sample_body(m, cs);
             hipGraph_t g = nullptr;
-            const hipError_t e = hipStreamEndCapture(s, &g);
+            const hipError_t e = hipStreamEndCapture(cs, &g);
             if (st != SF_OK) {
                 if (g) (void)hipGraphDestroy(g);
                 return st;
@@ -1586,6 +1595,7 @@ extern "C" int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* strea
             m->graph_stream = s;
         }
         SF_HIP(hipGraphLaunch(m->graph_exec, s));
+        SF_HIP(hipEventRecord(m->graph_event, s));
     } else {
         SF_TRY(sample_body(m, s));
     }
@@ -1603,7 +1613,7 @@ extern "C" int sf_rdt_infer(sf_rdt* m, uint64_t frame_id, const void* lang_token
                             float* action_out, int32_t* encoded, void* stream) {
     if (!m || !action_out) return SF_EINVAL;
     const sf_rdt_config& c = m->cfg;
-    hipStream_t s = pick_stream(m, stream);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     const bool need_encode = !m->infer_cond_valid || m->infer_cond_frame != frame_id;
     if (need_encode) {
         SF_TRY(sf_rdt_encode_condition(m, lang_tokens, lang_len, img_tokens, state, stream));
