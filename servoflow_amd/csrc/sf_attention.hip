@@ -1248,9 +1248,10 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // attention.cu:90-139, 183-197): fp32 products on the fp32 MFMA
 // (v_mfma_f32_16x16x4_f32), so nothing is rounded below fp32.
 //
-// One wave per (b, h, 16-query block, key split), K and V read straight from
-// global memory (L2 serves the five query blocks of a head).  Per 16-key
-// block: S^T = K.Q^T in 16 steps of 4 head dims, where step s takes dims
+// One workgroup of 4 waves per (b, h, 16-query block, key split), wave w on
+// every fourth 16-key block, K and V read straight from global memory (L2
+// serves the five query blocks of a head), the waves' shares merged in LDS.
+// Per 16-key block: S^T = K.Q^T in 16 steps of 4 head dims, where step s takes dims
 // 16g + s from lane group g, so each lane reads 16 contiguous dims of its
 // key row and of its query row; then O^T += V^T.P^T in 4 steps, where step i
 // contracts keys {4g + i}: exactly the keys whose scores the S^T accumulator
@@ -1258,13 +1259,27 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // (key 4g + i, dim 16db + r) comes from 16 consecutive floats per lane group.
 // Online softmax in log2 units as in the other kernels; multi-split partials
 // go to the same workspace layout and merge kernel.
+//
+// Bound by the fp32 MFMA (32 of 32 cycles each per 16 keys: 36 us for image
+// keys at B = 2) and the chain load -> S^T -> softmax -> O^T of each wave, which
+// only other waves hide.  One wave per workgroup left 1.25 waves a SIMD there,
+// so that some SIMDs had two rounds; four waves make it 5.  67 queries, graph-
+// timed on cold K/V: B = 2 x 4374 keys 115.3 -> 83.3 us, B = 1 72.4 -> 61.7,
+// 517 keys 20.4 -> 13.8, 67 keys 8.2 -> 6.1, B = 8 with ragged keys <= 1024
+// 87.8 -> 64.5.  One wave with four key blocks fetched ahead instead: 114.7,
+// 74.3, 20.2, 8.5, 86.6.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ f32x4 mfma16x16x4_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(64) void attn_f32_kernel(const AttnArgs a) {
-    const int lane = threadIdx.x;
+constexpr int kF32Waves = 4;
+
+__global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) f32x4 wave_o[kF32Waves * 4 * 64];
+    __shared__ float2 wave_ml[kF32Waves * 16];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int g = lane >> 4;
     const int r = lane & 15;
     const int nsplit = a.nsplit;
@@ -1308,7 +1323,7 @@ __global__ __launch_bounds__(64) void attn_f32_kernel(const AttnArgs a) {
     for (int db = 0; db < 4; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY;   // running row max, log2 units
     float l = 0.f;         // this lane's share of the row sum
-    for (int kt = kbeg; kt < kend; kt += 16) {
+    for (int kt = kbeg + 16 * w; kt < kend; kt += 16 * kF32Waves) {
         float kv[16], vv[16];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -1353,19 +1368,36 @@ __global__ __launch_bounds__(64) void attn_f32_kernel(const AttnArgs a) {
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    // The waves' shares meet in LDS; wave w finishes head dims 16w .. 16w + 15.
+#pragma unroll
+    for (int db = 0; db < 4; ++db) wave_o[(w * 4 + db) * 64 + lane] = acc[db];
+    if (g == 0) wave_ml[w * 16 + r] = float2{m, l};
+    __syncthreads();
     if (qrow >= a.Sq) return;
-    // O^T lane layout: head dims 16db + 4g + i of query qrow
+    float2 ml[kF32Waves];
+    m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kF32Waves; ++j) {
+        ml[j] = wave_ml[j * 16 + r];
+        m = fmaxf(m, ml[j].x);
+    }
+    const float muse = m == -INFINITY ? 0.f : m;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    l = 0.f;
+#pragma unroll
+    for (int j = 0; j < kF32Waves; ++j) {
+        const float f = fast_exp2(ml[j].x - muse);
+        l += ml[j].y * f;
+        o += wave_o[(j * 4 + w) * 64 + lane] * f;
+    }
+    // O^T lane layout: head dims 16w + 4g + i of query qrow
     if (nsplit == 1) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-            store_out4(a, out_off(a, b, h, qrow, 16 * db + 4 * g), acc[db] * inv);
+        store_out4(a, out_off(a, b, h, qrow, 16 * w + 4 * g), o * inv);
     } else {
         const size_t row = (((size_t)b * a.H + h) * nsplit + split) * (size_t)a.Sq + qrow;
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-            *reinterpret_cast<f32x4*>(a.part_o + row * kD + 16 * db + 4 * g) = acc[db];
-        if (g == 0) *reinterpret_cast<float2*>(a.part_ml + row * 2) = float2{m, l};
+        *reinterpret_cast<f32x4*>(a.part_o + row * kD + 16 * w + 4 * g) = o;
+        if (w == 0 && g == 0) *reinterpret_cast<float2*>(a.part_ml + row * 2) = float2{m, l};
     }
 }
 
@@ -1681,7 +1713,8 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
     if (d->in_dtype == SF_F32) {
         const long qblocks = (d->Sq + 15) / 16;
         if ((long)ns * qblocks > 0x7fffffffL) return SF_ENOTSUP;
-        hipLaunchKernelGGL(sfk::attn_f32_kernel, dim3((unsigned)(ns * qblocks), d->H, d->B), dim3(64), 0, s, a);
+        hipLaunchKernelGGL(sfk::attn_f32_kernel, dim3((unsigned)(ns * qblocks), d->H, d->B),
+                           dim3(64 * sfk::kF32Waves), 0, s, a);
     } else if (short_keys) {
         const int qb = (d->Sq + 15) / 16;
         const int kb = ((d->Sk + 31) / 32) * 2;

@@ -147,9 +147,10 @@ struct sf_rdt {
     // (fp16 rows, which can leave fp16's range, with the range guard of
     // sf_gemm_frag: such rows are normalised from x).  The final norm is a
     // row-wide launch of its own (sf_norm_frag): its bf16 rounding then falls
-    // on the normalised values, one layer ahead of the output.  The cross-q projection leaves finished fp32 rows (q32), above 160 rows fp16
-    // ones as the QKV projection does there; the attention applies the
-    // per-head norms as it loads them.
+    // on the normalised values, one layer ahead of the output.  The cross-q
+    // projection leaves finished fp32 rows (q32), above 160 rows fp16 ones as
+    // the QKV projection does there; the attention applies the per-head norms
+    // as it loads them.
     bool frag = false;
     float* row_ss = nullptr;
     int row_tiles = 0;             // tiles of the sums row_ss holds now

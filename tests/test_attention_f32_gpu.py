@@ -1,0 +1,40 @@
+"""The fp32 attention kernel deals 16-key blocks to four waves and merges their
+shares: key counts around the block and the round of four (waves without a
+key), split or not, with length and causal masks, against float64.
+
+Bound: a score is a 64-term fp32 dot product of N(0, 1) rows, scaled by 1/8:
+error below 64 * 2^-24 * sum|q_i k_i| / 8 < 64 * 2^-24 * 64 / 8 * 2 (rows of
+64 with mean |q k| 0.64, twice that for the largest) = 6.1e-5 relative on a
+weight, and on outputs of at most 5: 1e-4 for rounding that does not all add
+up the same way."""
+import pytest
+import torch
+
+from servoflow_amd.attention import attention
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def reference(q, k, v, keep):
+    s = (q.double() @ k.double().transpose(-1, -2)) / 8.0
+    s = s.masked_fill(~keep, float("-inf"))
+    p = torch.softmax(s, -1).nan_to_num(0.0)   # no key kept: zeros
+    return p @ v.double()
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("Sk", [1, 15, 16, 17, 48, 63, 64, 65, 80, 129, 300])
+def test_key_counts_and_masks(Sk, splits):
+    B, H, Sq = 2, 3, 37
+    g = torch.Generator(device=DEV).manual_seed(Sk)
+    q, k, v = (torch.randn(B, H, n, 64, device=DEV, generator=g) for n in (Sq, Sk, Sk))
+    vl = torch.tensor([max(1, Sk - 1), (Sk + 1) // 2], device=DEV, dtype=torch.int32)
+    keep = torch.ones(B, 1, Sq, Sk, dtype=torch.bool, device=DEV)
+    cols = torch.arange(Sk, device=DEV)
+    lens = cols[None, None, None, :] < vl[:, None, None, None]
+    print("fp32 attention", Sk, splits, flush=True)
+    for kw, kp in (({}, keep), ({"valid_len": vl}, keep & lens),
+                   ({"is_causal": True}, keep & (cols[None, :] <= torch.arange(Sq, device=DEV)[:, None]))):
+        got = attention(q, k, v, out_dtype=torch.float32, num_splits=splits, **kw).double()
+        assert (got - reference(q, k, v, kp)).abs().max().item() <= 1e-4, kw
