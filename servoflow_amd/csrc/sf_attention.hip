@@ -1249,14 +1249,14 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // (v_mfma_f32_16x16x4_f32), so nothing is rounded below fp32.
 //
 // One workgroup of 4 waves per (b, h, 16-query block, key split), wave w on
-// every fourth 16-key block, K and V read straight from global memory (L2
-// serves the five query blocks of a head), the waves' shares merged in LDS.
-// Per 16-key block: S^T = K.Q^T in 16 steps of 4 head dims, where step s takes dims
-// 16g + s from lane group g, so each lane reads 16 contiguous dims of its
-// key row and of its query row; then O^T += V^T.P^T in 4 steps, where step i
-// contracts keys {4g + i}: exactly the keys whose scores the S^T accumulator
-// holds in element i of lane group g, so P^T needs no shuffle, and V element
-// (key 4g + i, dim 16db + r) comes from 16 consecutive floats per lane group.
+// every fourth 16-key block, K and V read straight from global memory (one
+// XCD's L2 serves the query blocks of a head), the waves' shares merged in LDS.
+// Per 16-key block: S^T = K.Q^T in 16 steps of 4 head dims, where step 4c + e
+// takes dim 16c + 4g + e from lane group g, so load c is 64 contiguous bytes of
+// each key row; then O^T += V^T.P^T in 4 steps, where step i contracts keys
+// {4g + i}: exactly the keys whose scores the S^T accumulator holds in element i
+// of lane group g, so P^T needs no shuffle.  Accumulator db takes dims 4r + db,
+// so a lane's V operands of step i are 16 bytes and the load four whole rows.
 // Online softmax in log2 units as in the other kernels; multi-split partials
 // go to the same workspace layout and merge kernel.
 //
@@ -1268,6 +1268,10 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // 517 keys 20.4 -> 13.8, 67 keys 8.2 -> 6.1, B = 8 with ragged keys <= 1024
 // 87.8 -> 64.5.  One wave with four key blocks fetched ahead instead: 114.7,
 // 74.3, 20.2, 8.5, 86.6.
+// The query blocks on one XCD and these operand orders, against query blocks
+// spread over up to five XCDs, K loads of 16-byte pieces and 4-byte V loads (same
+// timing, another box): B = 2 x 4374 keys 76.7 -> 72.8, B = 1 60.3 -> 45.3, B = 8
+// 379 -> 247, 517 keys 13.4 -> 12.5, 67 keys 5.8 -> 5.2, B = 8 ragged 63.7 -> 46.1.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ f32x4 mfma16x16x4_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -1283,10 +1287,27 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     const int g = lane >> 4;
     const int r = lane & 15;
     const int nsplit = a.nsplit;
-    const int split = blockIdx.x % nsplit;
-    const int q0 = 16 * (int)(blockIdx.x / nsplit);
-    const int h = blockIdx.y;
-    const int b = blockIdx.z;
+    // Workgroup n runs on XCD n mod 8: the query blocks of a (b, h, split) take
+    // ids 8 apart, so one XCD's L2 fetches its keys once (the remainder of
+    // groups by 8 as it comes).
+    const uint32_t nqb = gridDim.x / (uint32_t)nsplit, groups = (uint32_t)nsplit * gridDim.y * gridDim.z;
+    const uint32_t id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const uint32_t whole = (groups & ~7u) * nqb;
+    uint32_t grp, qb;
+    if (id < whole) {
+        grp = (id >> 3) / nqb;
+        qb = (id >> 3) - grp * nqb;
+        grp = grp * 8 + (id & 7);
+    } else {
+        grp = (id - whole) / nqb;
+        qb = id - whole - grp * nqb;
+        grp += groups & ~7u;
+    }
+    const int split = grp % (uint32_t)nsplit;
+    const uint32_t bh = grp / (uint32_t)nsplit;
+    const int h = bh % gridDim.y;
+    const int b = bh / gridDim.y;
+    const int q0 = 16 * (int)qb;
     const int qrow = q0 + r;
 
     int valid = a.Sk;
@@ -1314,7 +1335,7 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     float qv[16];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const u32x4 w = buffer_load16(qrs, (uint32_t)((qrow * a.q_ss + 16 * g + 4 * c) * 4));
+        const u32x4 w = buffer_load16(qrs, (uint32_t)((qrow * a.q_ss + 16 * c + 4 * g) * 4));
 #pragma unroll
         for (int e = 0; e < 4; ++e) qv[4 * c + e] = __uint_as_float(w[e]);
     }
@@ -1324,19 +1345,17 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     float m = -INFINITY;   // running row max, log2 units
     float l = 0.f;         // this lane's share of the row sum
     for (int kt = kbeg + 16 * w; kt < kend; kt += 16 * kF32Waves) {
-        float kv[16], vv[16];
+        float kv[16];
+        f32x4 vv[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const u32x4 w = buffer_load16(krs, (uint32_t)(((kt + r) * a.k_ss + 16 * g + 4 * c) * 4));
+            const u32x4 w = buffer_load16(krs, (uint32_t)(((kt + r) * a.k_ss + 16 * c + 4 * g) * 4));
 #pragma unroll
             for (int e = 0; e < 4; ++e) kv[4 * c + e] = __uint_as_float(w[e]);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int db = 0; db < 4; ++db)
-                vv[4 * i + db] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    vrs, (uint32_t)(((kt + 4 * g + i) * a.v_ss + 16 * db + r) * 4), 0, 0));
+            vv[i] = __builtin_bit_cast(f32x4, buffer_load16(vrs, (uint32_t)(((kt + 4 * g + i) * a.v_ss + 4 * r) * 4)));
         const uint32_t mw = a.kv_mask ? mask_word(mrs, kt + 4 * g) : 0xffffffffu;
         f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1363,14 +1382,16 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
             const float p = fast_exp2(sc[i] - muse);
             l += p;
 #pragma unroll
-            for (int db = 0; db < 4; ++db) acc[db] = mfma16x16x4_f32(vv[4 * i + db], p, acc[db]);
+            for (int db = 0; db < 4; ++db) acc[db] = mfma16x16x4_f32(vv[i][db], p, acc[db]);
         }
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    // The waves' shares meet in LDS; wave w finishes head dims 16w .. 16w + 15.
+    // The waves' shares meet in LDS; element i of a lane's four accumulators is
+    // head dims 16g + 4i .. + 3.  Wave w finishes dims 16w .. 16w + 15.
 #pragma unroll
-    for (int db = 0; db < 4; ++db) wave_o[(w * 4 + db) * 64 + lane] = acc[db];
+    for (int i = 0; i < 4; ++i)
+        wave_o[(w * 4 + i) * 64 + lane] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
     if (g == 0) wave_ml[w * 16 + r] = float2{m, l};
     __syncthreads();
     if (qrow >= a.Sq) return;
@@ -1388,9 +1409,8 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     for (int j = 0; j < kF32Waves; ++j) {
         const float f = fast_exp2(ml[j].x - muse);
         l += ml[j].y * f;
-        o += wave_o[(j * 4 + w) * 64 + lane] * f;
+        o += wave_o[(j * 4 + g) * 64 + 16 * w + r] * f;
     }
-    // O^T lane layout: head dims 16w + 4g + i of query qrow
     if (nsplit == 1) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
         store_out4(a, out_off(a, b, h, qrow, 16 * w + 4 * g), o * inv);

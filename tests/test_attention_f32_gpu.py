@@ -38,3 +38,20 @@ def test_key_counts_and_masks(Sk, splits):
                    ({"is_causal": True}, keep & (cols[None, :] <= torch.arange(Sq, device=DEV)[:, None]))):
         got = attention(q, k, v, out_dtype=torch.float32, num_splits=splits, **kw).double()
         assert (got - reference(q, k, v, kp)).abs().max().item() <= 1e-4, kw
+
+
+@pytest.mark.parametrize("B,H,Sq,splits", [(1, 1, 1, 1), (1, 7, 67, 1), (1, 8, 16, 1), (2, 8, 67, 2), (3, 5, 33, 3),
+                                           (1, 9, 131, 4)])
+def test_every_query_block_is_computed_once(B, H, Sq, splits):
+    """Groups of (b, h, split) below, at and past multiples of 8, the unit in
+    which workgroups are dealt; keys of their own strides in half the cases."""
+    Sk = 150
+    g = torch.Generator(device=DEV).manual_seed(100 * H + Sq)
+    q = torch.randn(B, H, Sq, 64, device=DEV, generator=g)
+    k, v = (torch.randn(B, H, Sk, 64, device=DEV, generator=g) for _ in range(2))
+    if H % 2:   # [B, S, H, 64] storage
+        q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    keep = torch.ones(B, 1, Sq, Sk, dtype=torch.bool, device=DEV)
+    print("fp32 attention grid", B, H, Sq, splits, flush=True)
+    got = attention(q, k, v, out_dtype=torch.float32, num_splits=splits).double()
+    assert (got - reference(q, k, v, keep)).abs().max().item() <= 1e-4
