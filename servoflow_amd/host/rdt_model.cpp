@@ -939,14 +939,16 @@ int block_forward(sf_rdt* m, int i, hipStream_t s) {
     return linear_add_norm(m, m->h, fd, M, L.fc2_w, L.fc2_b, next_norm(m, i), m->n, ad, s);
 }
 
-// m->n = first norm applied to the residual m->x before block `first`.
+// m->n = first norm applied to the residual m->x before block `first`.  The
+// blocks take a deferred norm, the final layer (a model of no blocks) a
+// finished one.
 int entry_norm(sf_rdt* m, int first, hipStream_t s) {
     const sf_rdt_config& c = m->cfg;
     const int D = c.hidden, M = c.batch * (c.horizon + 3);
     const int g = first < c.layers ? m->layers[first].norm1 : m->fnorm;
     if (m->frag) {
         m->row_tiles = D / 64;
-        return sf_norm_frag(m->x, D, pf(m, g), m->n, m->act16, m->row_ss, M, D, c.eps, s);
+        return sf_norm_frag(m->x, D, pf(m, g), m->n, m->act16, first < c.layers ? m->row_ss : nullptr, M, D, c.eps, s);
     }
     return sf_rmsnorm(m->x, SF_F32, D, pf(m, g), m->n, m->act16, D, M, D, c.eps, s);
 }

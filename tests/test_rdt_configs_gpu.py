@@ -121,6 +121,24 @@ def test_block_vs_fp32_oracle_large_batch(batch, int8, blk):
     assert mr_b <= 1e-3
 
 
+@pytest.mark.parametrize("batch", [1, 3, 10])   # bf16 and fp16 fragment-ordered steps, library step
+def test_denoise_step_without_blocks(batch):
+    """A model of no blocks is its embeddings and the final layer: the final
+    norm directly follows the tokens.  One bf16 rounding is at most 2^-9 of a
+    value; the velocity's mean error stays below one rounding of every value
+    (rows left without their norm are off by the row's rms)."""
+    print(f"denoise step without blocks, batch {batch}", flush=True)
+    c = small_cfg(layers=0, batch=batch)
+    m = build(c)
+    lang, ll, img, state = make_condition(c)
+    set_cond(m, lang, ll, img, state)
+    x_t = O.randn(98, (batch, c.horizon, c.action_dim))
+    ref = OR.denoise_step(m.state_dict(), x_t, 0.8, state, [], ll, oracle_cfg(c), rb=rb_of(c))
+    for _ in range(2):
+        got = m.denoise_step(torch.from_numpy(x_t).to(DEV), 0.8).cpu().numpy()
+        assert mean_rel(got, ref) <= 2.0 ** -9
+
+
 @pytest.mark.parametrize("batch,int8", [(16, 0), (32, 1)], ids=["b16", "int8_b32"])
 def test_denoise_step_large_batch(batch, int8):
     """Config 4 at batch 16 and config 5 (int8 weights) at batch 32: every
