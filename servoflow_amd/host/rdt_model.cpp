@@ -1055,12 +1055,15 @@ int resolve_pv_forms(sf_rdt* m) {
     return SF_OK;
 }
 
-// The weight copies, brought up to date before a pass (never under capture:
-// every entry point calls this first).
+// The weight copies, brought up to date before a pass; every entry point calls
+// this first, before it captures anything itself.  In a caller's own capture
+// the copies are written by each replay, so they stay stale for eager passes.
 int refresh_copies(sf_rdt* m, hipStream_t s) {
     if (!m->copies || !m->copies_stale) return SF_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (s) SF_HIP(hipStreamIsCapturing(s, &cs));   // the NULL stream cannot capture
     SF_TRY(write_copies(m, s));
-    m->copies_stale = false;
+    m->copies_stale = cs != hipStreamCaptureStatusNone;
     return SF_OK;
 }
 

@@ -14,8 +14,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-def build(batch, seed=7):
-    c = R.default_config(layers=2, lang_max=40, img_len=72, batch=batch)
+def build(batch, seed=7, int8=0):
+    c = R.default_config(layers=2, lang_max=40, img_len=72, batch=batch, int8_weights=int8)
     m = R.RdtModel(c)
     m.init_random(seed, 0.02)
     g = torch.Generator(device=DEV).manual_seed(seed)
@@ -69,3 +69,27 @@ def test_two_threads_on_the_default_stream():
         assert res[i] is not None
         for got in res[i]:
             assert torch.equal(got, want[i])
+
+
+@pytest.mark.parametrize("batch,int8", [(1, 0), (1, 1), (3, 0), (10, 0)])
+def test_first_pass_recorded_by_the_caller(batch, int8):
+    """A caller may record a model's first pass into a graph of its own.  The
+    weight copies that this pass writes exist only once the graph has run: an
+    eager pass before that, and one in between the replays, gives the model's
+    result, and so does every replay."""
+    print("first pass recorded", batch, int8, flush=True)
+    m, noise = build(batch, int8=int8)
+    ref, _ = build(batch, int8=int8)
+    want = ref.denoise_step(noise, 0.5)
+    m.pv_exact(0)   # the condition's P.V forms are known: nothing left to wait for
+    torch.cuda.synchronize()
+    graph, v = torch.cuda.CUDAGraph(), torch.zeros_like(noise)
+    with torch.cuda.graph(graph):
+        m.denoise_step(noise, 0.5, out=v)
+    assert torch.equal(m.denoise_step(noise, 0.5), want)
+    for _ in range(3):
+        v.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(v, want)
+        assert torch.equal(m.denoise_step(noise, 0.5), want)
