@@ -524,7 +524,8 @@ int sf_frag_pack(const sf_frag_job* jobs, int32_t count, void* stream);
  * 16-byte aligned) into fragment order in SF_BF16 or SF_F16
  * (rms_norm_kernel_impl, norm.cuh:89-122).  ss != NULL: the deferred form of
  * sf_rmsnorm_deferred instead: x * gamma, and ss [rows][cols / 64] (row-major
- * here) the sums of squares of 64 columns. */
+ * here) the sums of squares of 64 columns; for SF_F16 with the marks of
+ * sf_gemm_frag's SF_EPI_ADD_NORM. */
 int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int32_t out_dtype, float* ss,
                  int32_t rows, int32_t cols, float eps, void* stream);
 
@@ -543,12 +544,16 @@ int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int
  *                    (fragment order, norm_dtype) = C * norm_gamma, and
  *                    norm_ss[m * T + t] = the sum of C[m][n]^2 over tile t's
  *                    columns, T = sf_gemm_frag_ss_tiles(desc) <= 64 tiles.
+ *                    SF_F16 marks: infinite where an element leaves fp16's
+ *                    range, negated where the tile has no element of at least
+ *                    sqrt(N) 2^-11 in magnitude.
  * a_row_ss (SF_EPI_PLAIN, SF_EPI_HEADS): as sf_gemm_desc's, but row-major,
  * [M][a_row_tiles].  SF_F16 rows from SF_EPI_ADD_NORM need a_x (SF_EPI_PLAIN):
- * x * gamma can leave fp16's range, which that epilogue marks by an infinite
- * sum; rows whose mean square is not in [2^-16, inf) are then normalised from
- * the fp32 rows a_x [M][a_x_ld] with a_x_gamma instead (a_row_n == K).  Row m's result depends on
- * row m, the weights and the summation order that K fixes, not on M. */
+ * x * gamma can leave fp16's range or lie in its subnormals.  Rows with an
+ * infinite sum, and rows of a mean square below 1 whose sums are all negative,
+ * are normalised from the fp32 rows a_x [M][a_x_ld] with a_x_gamma instead
+ * (a_row_n == K).  Row m's result depends on row m, the weights and the
+ * summation order that K fixes, not on M. */
 typedef struct sf_frag_gemm_desc {
     int32_t M, N, K;
     const void* A;

@@ -44,17 +44,22 @@ constexpr int kFragRowTiles = 64;   // tile sums of a deferred row: 16 in each o
 // What the rows of a are (the RS template argument): finished; x * gamma of a
 // deferred norm; or that in fp16 with the range guard.
 //
-// The guard.  x * gamma, unlike the normalised row, is not bounded by fp16's
-// range.  The add + norm epilogue reports an element beyond it by an infinite
-// tile sum, and the consumer reads each row's sum anyway: a row whose mean
-// square is not in [2^-16, inf) -- out of range above, or so small that fp16's
-// subnormal step (2^-25) is no longer far below the row's own rounding -- is
-// contracted again from the fp32 residual, normalised first, by the wave that
-// finishes it.  Rows in range, every row of a model whose residual is not
-// degenerate, pay one comparison; a row's result does not depend on whether
+// The guard.  x * gamma, unlike the normalised row, is neither bounded by
+// fp16's range nor kept out of its subnormals.  The producer of the row marks
+// both in the tile sums that the consumer reads anyway: an element beyond the
+// range by an infinite sum, and a tile without an element of at least
+// sqrt(N) 2^-11 by a negative one.  A row is contracted again from the fp32
+// residual, normalised first, by the wave that finishes it, if its sum is
+// infinite, or if all its tiles are negative and its mean square is below 1.
+// Any other row is stored no worse than a normalised one: with an element of
+// sqrt(N) 2^-11 its rms is at least 2^-11, of which the half step of a
+// subnormal, 2^-25, is an eighth of the error that an 11-bit rounding may make;
+// with a mean square of at least 1 each x * gamma is at least as large as the
+// normalised element.  Rows in range, every row of a model whose residual is
+// not degenerate, pay the comparison; a row's result does not depend on whether
 // its neighbours are in range.
 enum RowKind { kRowPlain = 0, kRowDeferred = 1, kRowGuarded = 2 };
-constexpr float kGuardMinMeanSq = 1.f / 65536.f;
+constexpr float kGuardTopSq = 1.f / 4194304.f;   // times N: the mark's square
 constexpr float kF16Max = 65504.f;
 
 // The epilogue's arguments (the operands' pointers and sizes are scalar kernel
@@ -98,6 +103,11 @@ __device__ __forceinline__ float sum_groups(float x) {
     x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
     s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// Whether x holds in any of those four lanes.
+__device__ __forceinline__ bool any_groups(bool x) {
+    return ((__ballot(x) >> (threadIdx.x & 15)) & 0x0001000100010001ull) != 0;
 }
 
 // One workgroup of 4 waves per (16 NB columns x 16 MB rows) of C over all of
@@ -168,12 +178,23 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
             v[q] = __builtin_bit_cast(f32x4, buffer_load16(rrs, off));
         }
     };
-    auto row_sum = [&](f32x4 (&v)[kFragRowTiles / 16]) {
+    auto row_sum = [&](f32x4 (&v)[kFragRowTiles / 16], bool& marked) {
         if (row_tiles & 3) {   // the last quad runs into the next row
 #pragma unroll
             for (int q = 0; q < kFragRowTiles / 16; ++q)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[q][i] = 16 * q + 4 * g4 + i < row_tiles ? v[q][i] : 0.f;
+        }
+        if constexpr (RS == kRowGuarded) {   // marked: every tile's sum is negative (or zero)
+            float top = 0.f;
+#pragma unroll
+            for (int q = 0; q < kFragRowTiles / 16; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    top = fmaxf(top, v[q][i]);
+                    v[q][i] = fabsf(v[q][i]);
+                }
+            marked = !any_groups(top > 0.f);
         }
         const f32x4 t = (v[0] + v[1]) + (v[2] + v[3]);
         return sum_groups((t[0] + t[1]) + (t[2] + t[3]));
@@ -215,10 +236,11 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
         for (int k = 0; k < NI; ++k) load_row(item_mb(p0, k) < MB ? m0 + 16 * item_mb(p0, k) + r : M, rss[k]);
     };
     float sum[NI], rs[NI];
+    bool marked[NI];
     auto row_scales = [&] {
 #pragma unroll
         for (int k = 0; k < NI; ++k) {
-            sum[k] = row_sum(rss[k]);
+            sum[k] = row_sum(rss[k], marked[k]);
             rs[k] = deferred_rsqrt(sum[k], row_inv_n, row_eps);
         }
     };
@@ -363,7 +385,7 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
         }
         if constexpr (RS == kRowGuarded) {
             const float mean = sum[k] * row_inv_n;
-            const bool out = m < M && !(mean >= kGuardMinMeanSq && mean < INFINITY);
+            const bool out = m < M && !(mean < INFINITY && (mean >= 1.f || !marked[k]));
             if (__any(out)) {   // lanes r, r + 16, r + 32, r + 48 agree
                 const float* xr = e.x + (int64_t)min(m, M - 1) * e.x_ld;
                 float t = 0.f;
@@ -443,8 +465,9 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
                     top = fmaxf(top, fabsf(u[j][q]));
                 }
             }
-            if (e.norm_f16 && top > kF16Max) ss = INFINITY;   // the consumer's guard takes the row
+            if (e.norm_f16 && top > kF16Max) ss = INFINITY;   // the guard's marks
             ss = sum_groups(ss);
+            if (e.norm_f16 && !any_groups(top * top >= kGuardTopSq * (float)e.N)) ss = -ss;
             if (m >= M) continue;
 #pragma unroll
             for (int j = 0; j < EN; ++j) {
@@ -506,6 +529,7 @@ __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t 
     if (ss) {   // 8 lanes hold a 64-column tile
 #pragma unroll
         for (int i = 0; i < kNormFragPer; ++i) {
+            bool small = false;
             if (f16) {   // as the add + norm epilogue marks it
                 float top = 0.f;
 #pragma unroll
@@ -513,8 +537,9 @@ __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t 
 #pragma unroll
                     for (int j = 0; j < 4; ++j) top = fmaxf(top, fabsf(v[i][h][j] * gq[i][h][j]));
                 if (top > kF16Max) sum[i] = INFINITY;
+                small = !((__ballot(top * top >= kGuardTopSq * (float)cols) >> (threadIdx.x & 56)) & 255);
             }
-            const float t = row8_sum(sum[i]);
+            const float t = row8_sum(sum[i]) * (small ? -1.f : 1.f);
             const int c = 8 * ((int)threadIdx.x + 256 * i);
             if (c < cols && (threadIdx.x & 7) == 0) ss[(int64_t)row * (cols / 64) + c / 64] = t;
         }

@@ -185,6 +185,41 @@ def test_fp16_rows_out_of_range(M, N, kind):
     assert torch.equal(got[0][same], got[1][same])
 
 
+# (x's scale, gamma's scale): x * gamma deep in fp16's subnormals, just above
+# and below the mark, x of ordinary size (no better off normalised), and large
+@pytest.mark.parametrize("xs,gs", [(0.0042, 0.03), (0.0042, 1e-3), (0.0078, 3e-3), (0.3, 1e-3), (0.9, 2e-4), (0.03, 0.1),
+                                   (3.0, 1e-3), (300.0, 3e-3), (1e-4, 40.0)])
+@pytest.mark.parametrize("M,N", [(67, 2048), (402, 512)])
+@pytest.mark.parametrize("entry", [False, True])
+def test_fp16_rows_of_small_products(M, N, entry, xs, gs):
+    """Deferred fp16 rows whose x * gamma is small keep the precision of rows
+    normalised before their rounding to fp16, from both producers.  A rounding
+    to nearest of 11 bits has a relative error below 2^-11, uniformly spread
+    below 2^-11 / sqrt(3) of the value; the product's share is that of its
+    terms.  The second half of the columns has gamma's scale a hundredth: its x
+    is a hundred times larger in every third row, and the first half's zero."""
+    gamma, x = (1 + randn(50, N, std=0.1)) * gs, randn(51, M, N) * xs
+    gamma[N // 2:] *= 0.01
+    x[::3, N // 2:] *= 100
+    x[::3, :N // 2] = 0
+    wf, s, w64 = weights(52, 512, N, "w16", torch.float16)
+    if entry:
+        n, ss = K.norm_frag(x, gamma, out_dtype=torch.float16, deferred=True)
+    else:
+        a = torch.zeros(M, 64, dtype=torch.bfloat16, device=DEV)
+        wz = K.frag_pack([torch.zeros(N, 64, dtype=torch.bfloat16, device=DEV)], [torch.bfloat16])[0]
+        n, ss = K.gemm_frag_add_norm(M, to_frag(a), wz, None, x, gamma, norm_dtype=torch.float16)
+    got = K.gemm_frag(M, n, wf, None, row_ss=ss, row_n=N, x=x, x_gamma=gamma)
+    norm = x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-6) * gamma.double()
+    ref = norm @ w64.t()
+    # what a normalised row's own subnormals (half a step of 2^-24) add
+    sub = 2.0 ** -25 / norm.square().mean(1).sqrt()
+    err = (got.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    bound = 2.0 ** -11 / 3 ** 0.5 + sub
+    print("small products", M, N, entry, xs, gs, (err / bound).max().item(), flush=True)
+    assert (err < bound).all()
+
+
 # the one-wave and grouped short-key kernels, the query-block grid, key splits
 # with the merge, the unsplit 80-row grid, and fp32 inputs
 @pytest.mark.parametrize("B,H,Sq,Sk,dt", [(1, 32, 67, 67, torch.bfloat16), (8, 32, 67, 67, torch.float16),
