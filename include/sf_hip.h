@@ -548,10 +548,11 @@ int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, void* out, int
  *                    range, negated where the tile has no element of at least
  *                    sqrt(N) 2^-11 in magnitude.
  * a_row_ss (SF_EPI_PLAIN, SF_EPI_HEADS): as sf_gemm_desc's, but row-major,
- * [M][a_row_tiles].  SF_F16 rows from SF_EPI_ADD_NORM need a_x (SF_EPI_PLAIN):
- * x * gamma can leave fp16's range or lie in its subnormals.  Rows with an
- * infinite sum, and rows of a mean square below 1 whose sums are all negative,
- * are normalised from the fp32 rows a_x [M][a_x_ld] with a_x_gamma instead
+ * [M][a_row_tiles].  SF_F16 rows need a_x (SF_EINVAL without) and are taken by
+ * SF_EPI_PLAIN only (SF_ENOTSUP else): x * gamma can leave fp16's range or lie
+ * in its subnormals.  Rows with an infinite sum, and rows of a mean square below
+ * 1 whose sums are all negative, are normalised from the fp32 rows
+ * a_x [M][a_x_ld] with a_x_gamma instead
  * (a_row_n == K).  Row m's result depends on row m, the weights and the
  * summation order that K fixes, not on M. */
 typedef struct sf_frag_gemm_desc {

@@ -42,7 +42,7 @@ constexpr size_t kFragLds = 160 * 1024;
 constexpr int kFragRowTiles = 64;   // tile sums of a deferred row: 16 in each of 4 lane groups
 
 // What the rows of a are (the RS template argument): finished; x * gamma of a
-// deferred norm; or that in fp16 with the range guard.
+// deferred norm in bf16; or that in fp16 with the range guard.
 //
 // The guard.  x * gamma, unlike the normalised row, is neither bounded by
 // fp16's range nor kept out of its subnormals.  The producer of the row marks
@@ -137,7 +137,8 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
     const void* A, const void* W, int K, int M, int ntiles, const float* row_ss, int row_tiles, float row_inv_n,
     float row_eps, const FragEpi e) {
     static_assert(EPI != SF_EPI_HEADS || NB == 4, "a head is one column tile");
-    static_assert(RS != kRowGuarded || (AH && EPI == SF_EPI_PLAIN), "fp16 rows of the plain epilogue are guarded");
+    static_assert(RS == kRowPlain || (AH ? RS == kRowGuarded && EPI == SF_EPI_PLAIN : RS == kRowDeferred),
+                  "deferred fp16 rows are guarded, and taken by the plain epilogue only");
     constexpr int NW = kFragWaves;
     constexpr int ST = W8 ? 2 : 1;         // MFMA steps per unit: 16 bytes of codes are two steps
     constexpr bool kAddNorm = EPI == SF_EPI_ADD_NORM, kHeads = EPI == SF_EPI_HEADS, kPlain = EPI == SF_EPI_PLAIN;
@@ -660,12 +661,12 @@ void launch_frag_one(const FragOps& o, const FragTile& t, const FragEpi& e, hipS
 template <int NB, int MB, int U, int NG, bool W8, bool AH, int EPI>
 void launch_frag_rows(const FragOps& o, const FragTile& t, const FragEpi& e, hipStream_t s) {
     if constexpr (AH && EPI == SF_EPI_PLAIN) {
-        if (o.row_ss && e.x) {
+        if (o.row_ss) {
             launch_frag_one<NB, MB, U, NG, W8, AH, EPI, kRowGuarded>(o, t, e, s);
             return;
         }
     }
-    if constexpr (EPI != SF_EPI_ADD_NORM) {
+    if constexpr (!AH && EPI != SF_EPI_ADD_NORM) {
         if (o.row_ss) {
             launch_frag_one<NB, MB, U, NG, W8, AH, EPI, kRowDeferred>(o, t, e, s);
             return;
@@ -819,12 +820,14 @@ extern "C" int sf_gemm_frag(const sf_frag_gemm_desc* d, void* stream) {
         o.row_tiles = d->a_row_tiles;
         o.row_inv_n = 1.f / (float)d->a_row_n;
         o.row_eps = d->a_row_eps;
-        if (d->a_x) {   // fp16 rows with the range guard
-            if (d->a_dtype != SF_F16 || d->epilogue != SF_EPI_PLAIN || d->a_row_n != d->K) return SF_ENOTSUP;
-            if (!d->a_x_gamma || d->a_x_ld < d->K) return SF_EINVAL;
+        if (d->a_dtype == SF_F16) {   // with the range guard
+            if (d->epilogue != SF_EPI_PLAIN || d->a_row_n != d->K) return SF_ENOTSUP;
+            if (!d->a_x || !d->a_x_gamma || d->a_x_ld < d->K) return SF_EINVAL;
             a.x = d->a_x;
             a.x_gamma = d->a_x_gamma;
             a.x_ld = d->a_x_ld;
+        } else if (d->a_x) {
+            return SF_ENOTSUP;
         }
     } else if (d->a_x) {
         return SF_EINVAL;

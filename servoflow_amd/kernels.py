@@ -186,7 +186,7 @@ def gemm_frag(M, a, w, bias=None, act=abi.SF_ACT_NONE, out=None, out_dtype=torch
               accumulate=False, w_scale=None, row_ss=None, row_n=0, row_eps=1e-6, x=None, x_gamma=None):
     """sf_gemm_frag's plain epilogue on M rows of a (fragment order, padded
     rows) and w (frag_pack): row-major [M, N], or fragment order with c_frag.
-    x, x_gamma: the fp32 rows and gamma behind deferred fp16 rows."""
+    x, x_gamma: the fp32 rows and gamma behind deferred fp16 rows (required)."""
     N = w.shape[0]
     d = _frag_desc(M, a, w, bias, act, w_scale, row_ss, row_n, row_eps)
     if out is None:

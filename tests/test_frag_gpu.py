@@ -124,7 +124,8 @@ def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
     assert rel(ss.sum(1), xr.square().sum(1)) < 2e-6
     assert torch.equal(from_frag(n, M), (x * gamma).to(ndt))
     wf2, _, w2 = weights(14, 256, N, "w16", ndt)
-    got = K.gemm_frag(M, n, wf2, b[:256] if N >= 256 else None, row_ss=ss, row_n=N)
+    guard = {"x": x, "x_gamma": gamma} if ndt == torch.float16 else {}
+    got = K.gemm_frag(M, n, wf2, b[:256] if N >= 256 else None, row_ss=ss, row_n=N, **guard)
     ref = (from_frag(n, M).double() @ w2.t()) * torch.rsqrt(xr.square().mean(1, keepdim=True) + 1e-6)
     ref = ref + (b[:256].double() if N >= 256 else 0)
     assert rel(got, ref) < 2e-5
@@ -289,3 +290,18 @@ def test_refused():
                    ({"a_row_ss": out.data_ptr(), "a_row_tiles": 65, "a_row_n": 64}, abi.SF_EINVAL), ({"act": 3}, abi.SF_EINVAL)]:
         assert call(**kw) == st, kw
     assert call(M=0) == abi.SF_OK
+
+
+def test_unguarded_fp16_rows_refused():
+    """Deferred fp16 rows may have left fp16's range, so they need the fp32
+    rows behind them; the per-head epilogue has no guard and takes none."""
+    a, w = torch.zeros(16, 64, dtype=torch.float16, device=DEV), torch.zeros(192, 64, dtype=torch.float16, device=DEV)
+    ss, x, gamma = torch.ones(16, 1, device=DEV), torch.ones(16, 64, device=DEV), torch.ones(64, device=DEV)
+    with pytest.raises(abi.SfError) as e:
+        K.gemm_frag(16, a, w, row_ss=ss, row_n=64)
+    assert e.value.status == abi.SF_EINVAL
+    assert torch.equal(K.gemm_frag(16, a, w, row_ss=ss, row_n=64, x=x, x_gamma=gamma), torch.zeros(16, 192, device=DEV))
+    outs = [torch.empty(1, 1, 16, 64, dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+    with pytest.raises(abi.SfError) as e:
+        K.gemm_frag_heads(16, a, w, None, 16, 1, outs, row_ss=ss, row_n=64)
+    assert e.value.status == abi.SF_ENOTSUP
