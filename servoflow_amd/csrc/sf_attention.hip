@@ -1248,8 +1248,8 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // attention.cu:90-139, 183-197): fp32 products on the fp32 MFMA
 // (v_mfma_f32_16x16x4_f32), so nothing is rounded below fp32.
 //
-// One workgroup of 4 waves per (b, h, 16-query block, key split), wave w on
-// every fourth 16-key block, K and V read straight from global memory (one
+// One workgroup of NW waves per (b, h, 16-query block, key split), wave w on
+// every NW-th 16-key block, K and V read straight from global memory (one
 // XCD's L2 serves the query blocks of a head), the waves' shares merged in LDS.
 // Per 16-key block: S^T = K.Q^T in 16 steps of 4 head dims, where step 4c + e
 // takes dim 16c + 4g + e from lane group g, so load c is 64 contiguous bytes of
@@ -1267,67 +1267,63 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // timed on cold K/V: B = 2 x 4374 keys 115.3 -> 83.3 us, B = 1 72.4 -> 61.7,
 // 517 keys 20.4 -> 13.8, 67 keys 8.2 -> 6.1, B = 8 with ragged keys <= 1024
 // 87.8 -> 64.5.  One wave with four key blocks fetched ahead instead: 114.7,
-// 74.3, 20.2, 8.5, 86.6.
+// 74.3, 20.2, 8.5, 86.6.  Few keys and large grids take fewer (f32_waves).
 // The query blocks on one XCD and these operand orders, against query blocks
 // spread over up to five XCDs, K loads of 16-byte pieces and 4-byte V loads (same
 // timing, another box): B = 2 x 4374 keys 76.7 -> 72.8, B = 1 60.3 -> 45.3, B = 8
 // 379 -> 247, 517 keys 13.4 -> 12.5, 67 keys 5.8 -> 5.2, B = 8 ragged 63.7 -> 46.1.
+// The call of 11 keys took 4.04 us with the XCD's group found by three divisions
+// and the arguments fetched in three rounds, 3.57 with neither.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ f32x4 mfma16x16x4_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-constexpr int kF32Waves = 4;
-
-__global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) f32x4 wave_o[kF32Waves * 4 * 64];
-    __shared__ float2 wave_ml[kF32Waves * 16];
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void attn_f32_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(16))) f32x4 wave_o[NW > 1 ? NW * 4 * 64 : 1];
+    __shared__ float2 wave_ml[NW > 1 ? NW * 16 : 1];
     const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int w = NW > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
     const int g = lane >> 4;
     const int r = lane & 15;
-    const int nsplit = a.nsplit;
-    // Workgroup n runs on XCD n mod 8: the query blocks of a (b, h, split) take
-    // ids 8 apart, so one XCD's L2 fetches its keys once (the remainder of
-    // groups by 8 as it comes).
-    const uint32_t nqb = gridDim.x / (uint32_t)nsplit, groups = (uint32_t)nsplit * gridDim.y * gridDim.z;
-    const uint32_t id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const uint32_t whole = (groups & ~7u) * nqb;
-    uint32_t grp, qb;
-    if (id < whole) {
-        grp = (id >> 3) / nqb;
-        qb = (id >> 3) - grp * nqb;
-        grp = grp * 8 + (id & 7);
-    } else {
-        grp = (id - whole) / nqb;
-        qb = id - whole - grp * nqb;
-        grp += groups & ~7u;
-    }
-    const int split = grp % (uint32_t)nsplit;
-    const uint32_t bh = grp / (uint32_t)nsplit;
-    const int h = bh % gridDim.y;
-    const int b = bh / gridDim.y;
-    const int q0 = 16 * (int)qb;
-    const int qrow = q0 + r;
-
+    // one wait for every argument, not one at each first use
+    int nsplit = a.nsplit, causal = a.causal;
+    int64_t q_sb = a.q_sb, v_ss = a.v_ss, o_ss = a.o_ss;
+    asm("" : "+s"(nsplit), "+s"(causal), "+s"(q_sb), "+s"(v_ss), "+s"(o_ss) : "s"(a.q));
+    // Workgroup n runs on XCD n mod 8.  H a multiple of 8: a (8 query blocks x
+    // splits, H / 8, B) grid, so that the query blocks of a (b, h, split) take ids
+    // 8 apart and one XCD's L2 fetches its keys once.  Else a (query blocks x
+    // splits, H, B) grid.
+    const bool xcd = (a.H & 7) == 0;
+    const int h = xcd ? 8 * blockIdx.y + (blockIdx.x & 7) : blockIdx.y;
+    const int b = blockIdx.z;
     int valid = a.Sk;
     if (a.valid_len) {
         const int vl = a.valid_len[b];
         valid = vl < 0 ? 0 : (vl > a.Sk ? a.Sk : vl);
     }
-    int per = (valid + nsplit - 1) / nsplit;
+    int qb = xcd ? blockIdx.x >> 3 : blockIdx.x, split = 0, per = valid;
+    if (nsplit > 1) {   // query blocks of a split together
+        const int nqb = (a.Sq + 15) >> 4;
+        split = qb / nqb;
+        qb -= split * nqb;
+        per = (valid + nsplit - 1) / nsplit;
+    }
     per = (per + 15) & ~15;
+    const int q0 = 16 * qb;
+    const int qrow = q0 + r;
     const int kbeg = split * per;
     int kend = min(valid, kbeg + per);
-    if (a.causal) kend = min(kend, min(a.Sq, q0 + 16));
+    if (causal) kend = min(kend, min(a.Sq, q0 + 16));
 
-    const float* qp = reinterpret_cast<const float*>(a.q) + b * a.q_sb + h * a.q_sh;
+    const float* qp = reinterpret_cast<const float*>(a.q) + b * q_sb + h * a.q_sh;
     const float* kp = reinterpret_cast<const float*>(a.k) + b * a.k_sb + h * a.k_sh;
     const float* vp = reinterpret_cast<const float*>(a.v) + b * a.v_sb + h * a.v_sh;
     // rows outside [0, Sq) and keys outside [0, kend) read as zeros
     const __amdgpu_buffer_rsrc_t qrs = make_rsrc(qp, (uint32_t)(a.Sq * a.q_ss * 4));
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(kp, (uint32_t)(max(kend, 0) * a.k_ss * 4));
-    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vp, (uint32_t)(max(kend, 0) * a.v_ss * 4));
+    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vp, (uint32_t)(max(kend, 0) * v_ss * 4));
     const __amdgpu_buffer_rsrc_t mrs =
         make_rsrc(a.kv_mask ? static_cast<const void*>(a.kv_mask + b * a.kv_mask_stride) : static_cast<const void*>(a.q),
                   a.kv_mask ? (uint32_t)((a.Sk + 3) & ~3) : 0u);
@@ -1344,7 +1340,7 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     for (int db = 0; db < 4; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY;   // running row max, log2 units
     float l = 0.f;         // this lane's share of the row sum
-    for (int kt = kbeg + 16 * w; kt < kend; kt += 16 * kF32Waves) {
+    for (int kt = kbeg + 16 * w; kt < kend; kt += 16 * NW) {
         float kv[16];
         f32x4 vv[4];
 #pragma unroll
@@ -1355,7 +1351,7 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            vv[i] = __builtin_bit_cast(f32x4, buffer_load16(vrs, (uint32_t)(((kt + 4 * g + i) * a.v_ss + 4 * r) * 4)));
+            vv[i] = __builtin_bit_cast(f32x4, buffer_load16(vrs, (uint32_t)(((kt + 4 * g + i) * v_ss + 4 * r) * 4)));
         const uint32_t mw = a.kv_mask ? mask_word(mrs, kt + 4 * g) : 0xffffffffu;
         f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1387,38 +1383,51 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_kernel(const AttnArgs
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    // The waves' shares meet in LDS; element i of a lane's four accumulators is
-    // head dims 16g + 4i .. + 3.  Wave w finishes dims 16w .. 16w + 15.
+    // Element i of a lane's four accumulators is head dims 16g + 4i .. + 3.
+    // Dims d .. d + 3 of query qrow; fp32, the usual type, is never in fragment order.
+    const size_t row = (((size_t)b * a.H + h) * nsplit + split) * (size_t)a.Sq + qrow;
+    float* const rows32 = nsplit > 1 ? a.part_o + row * kD : static_cast<float*>(a.o) + (b * a.o_sb + h * a.o_sh + qrow * o_ss);
+    auto store = [&](int d, f32x4 o) {
+        if (nsplit > 1 || a.out_kind == kOutF32) *reinterpret_cast<f32x4*>(rows32 + d) = o;
+        else store_out4(a, out_off(a, b, h, qrow, d), o);
+    };
+    auto finish = [&] { return nsplit > 1 ? 1.f : (l > 0.f ? 1.f / l : 0.f); };
+    if constexpr (NW == 1) {
+        if (qrow >= a.Sq) return;
+        const float inv = finish();
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        wave_o[(w * 4 + i) * 64 + lane] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
-    if (g == 0) wave_ml[w * 16 + r] = float2{m, l};
-    __syncthreads();
-    if (qrow >= a.Sq) return;
-    float2 ml[kF32Waves];
-    m = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < kF32Waves; ++j) {
-        ml[j] = wave_ml[j * 16 + r];
-        m = fmaxf(m, ml[j].x);
-    }
-    const float muse = m == -INFINITY ? 0.f : m;
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    l = 0.f;
-#pragma unroll
-    for (int j = 0; j < kF32Waves; ++j) {
-        const float f = fast_exp2(ml[j].x - muse);
-        l += ml[j].y * f;
-        o += wave_o[(j * 4 + g) * 64 + 16 * w + r] * f;
-    }
-    if (nsplit == 1) {
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        store_out4(a, out_off(a, b, h, qrow, 16 * w + 4 * g), o * inv);
+        for (int i = 0; i < 4; ++i) store(16 * g + 4 * i, f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]} * inv);
     } else {
-        const size_t row = (((size_t)b * a.H + h) * nsplit + split) * (size_t)a.Sq + qrow;
-        *reinterpret_cast<f32x4*>(a.part_o + row * kD + 16 * w + 4 * g) = o;
-        if (w == 0 && g == 0) *reinterpret_cast<float2*>(a.part_ml + row * 2) = float2{m, l};
+        // the waves' shares meet in LDS; wave w finishes dims 16w + (0 .. 15), and
+        // every 16 NW further
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            wave_o[(w * 4 + i) * 64 + lane] = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+        if (g == 0) wave_ml[w * 16 + r] = float2{m, l};
+        __syncthreads();
+        if (qrow >= a.Sq) return;
+        float f[NW];
+        m = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < NW; ++j) m = fmaxf(m, wave_ml[j * 16 + r].x);
+        const float muse = m == -INFINITY ? 0.f : m;
+        l = 0.f;
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+            const float2 ml = wave_ml[j * 16 + r];
+            f[j] = fast_exp2(ml.x - muse);
+            l += ml.y * f[j];
+        }
+        const float inv = finish();
+#pragma unroll
+        for (int p = w; p < 4; p += NW) {
+            f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NW; ++j) o += wave_o[(j * 4 + g) * 64 + 16 * p + r] * f[j];
+            store(16 * p + 4 * g, o * inv);
+        }
     }
+    if (nsplit > 1 && w == 0 && g == 0) *reinterpret_cast<float2*>(a.part_ml + row * 2) = float2{m, l};
 }
 
 }  // namespace sfk
@@ -1466,6 +1475,23 @@ int choose_splits(const sf_attn_desc* d) {
     ns = (tiles + longest - 1) / longest;
     if (ns > kMaxSplits) ns = kMaxSplits;
     return (int)ns;
+}
+
+// Waves per workgroup of the fp32 kernel: no more than 16-key blocks, and fewer
+// where the grid is large.  From 1024 workgroups each SIMD has a wave of its own,
+// from 4096 four of them, which hide each other's chains; up to 16 key blocks
+// more waves then only add their merge.  Graph-timed with 1 / 2 / 4 waves:
+// 11 keys, 8 workgroups 3.6 / 3.8 / 3.8 us; 17 keys, 160 workgroups 4.4 / 4.0 /
+// 4.0; 67 keys, 640 workgroups 8.0 / 7.6 / 7.5, 1280 10.7 / 10.2 / 10.7, 2560
+// 15.6 / 15.4 / 17.8; 64 keys, 10240 37.0 / 38.7 / 46.2; 131 keys, 4608 35.1 /
+// 37.2 / 39.1; 256 keys, 2560 36.2 / 32.4 / 33.7; 1024 keys, 1280 92.8 / 66.4 /
+// 56.2, 2560 132.7 / 109.9 / 109.8, 4608 207.6 / 200.0 / 187.7.
+int f32_waves(const sf_attn_desc* d, int nsplit) {
+    const long blocks = ((d->Sk + nsplit - 1) / nsplit + 15) / 16;
+    const long groups = (long)d->B * d->H * ((d->Sq + 15) / 16) * nsplit;
+    if (blocks <= 1 || (blocks <= 16 && groups >= 4096)) return 1;
+    if (blocks <= 2 || (blocks <= 16 && groups >= 1024)) return 2;
+    return 4;
 }
 
 // Key sets of the short-key kernel.
@@ -1732,9 +1758,13 @@ extern "C" int sf_attn_fwd(const sf_attn_desc* d, const void* q, const void* k, 
     const bool vh = d->v_f16 != 0;
     if (d->in_dtype == SF_F32) {
         const long qblocks = (d->Sq + 15) / 16;
-        if ((long)ns * qblocks > 0x7fffffffL) return SF_ENOTSUP;
-        hipLaunchKernelGGL(sfk::attn_f32_kernel, dim3((unsigned)(ns * qblocks), d->H, d->B),
-                           dim3(64 * sfk::kF32Waves), 0, s, a);
+        const bool xcd = (d->H & 7) == 0;
+        if ((xcd ? 8L : 1L) * ns * qblocks > 0x7fffffffL) return SF_ENOTSUP;
+        const dim3 grid((unsigned)((xcd ? 8 : 1) * ns * qblocks), xcd ? d->H / 8 : d->H, d->B);
+        const int nw = f32_waves(d, ns);
+        if (nw == 1) hipLaunchKernelGGL(sfk::attn_f32_kernel<1>, grid, dim3(64), 0, s, a);
+        else if (nw == 2) hipLaunchKernelGGL(sfk::attn_f32_kernel<2>, grid, dim3(128), 0, s, a);
+        else hipLaunchKernelGGL(sfk::attn_f32_kernel<4>, grid, dim3(256), 0, s, a);
     } else if (short_keys) {
         const int qb = (d->Sq + 15) / 16;
         const int kb = ((d->Sk + 31) / 32) * 2;

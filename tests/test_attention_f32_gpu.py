@@ -55,3 +55,24 @@ def test_every_query_block_is_computed_once(B, H, Sq, splits):
     print("fp32 attention grid", B, H, Sq, splits, flush=True)
     got = attention(q, k, v, out_dtype=torch.float32, num_splits=splits).double()
     assert (got - reference(q, k, v, keep)).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 8, 11, 11), (1, 8, 40, 17), (26, 8, 67, 33), (26, 8, 67, 67), (26, 8, 67, 256), (26, 8, 67, 257),
+                                       (103, 8, 67, 17), (103, 8, 67, 256), (103, 8, 67, 257), (147, 7, 67, 50)])
+def test_waves_per_workgroup(B, H, Sq, Sk):
+    """Both sides of the rule for one, two and four waves: one key block and
+    two, 1040 and 4120 workgroups with 16 key blocks and with 17; a full and a
+    ragged set of keys, a batch element without a key among them."""
+    g = torch.Generator(device=DEV).manual_seed(1000 * B + Sk)
+    q, k, v = (torch.randn(B, H, n, 64, device=DEV, generator=g) for n in (Sq, Sk, Sk))
+    vl = torch.randint(0, Sk + 1, (B,), device=DEV, generator=g, dtype=torch.int32)
+    vl[0] = 0
+    keep = torch.ones(B, 1, Sq, Sk, dtype=torch.bool, device=DEV)
+    lens = torch.arange(Sk, device=DEV)[None, None, None, :] < vl[:, None, None, None]
+    print("fp32 attention waves", B, H, Sq, Sk, flush=True)
+    for kw, kp in (({}, keep), ({"valid_len": vl}, keep & lens)):
+        ref = reference(q, k, v, kp)
+        # a rounding to bf16's 8 bits, to nearest, is at most 2^-8 of the value
+        for odt, step in ((torch.float32, 0.0), (torch.bfloat16, 2.0 ** -8)):
+            got = attention(q, k, v, out_dtype=odt, **kw).double()
+            assert ((got - ref).abs() <= 1e-4 + step * ref.abs()).all(), (odt, list(kw))
