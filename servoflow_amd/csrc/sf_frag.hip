@@ -614,11 +614,15 @@ __global__ __launch_bounds__(256) void frag_pack_kernel(const FragJobs J) {
 // (2, 3) and 8.5 for (4, 2); 134 x 2048 (2, 3) 7.4 against 9.7 for (2, 2); 402 x
 // 2048 (4, 4) 10.2 against 11.4 for (4, 5); 1072 x 2048 (8, 5) 16.5 against
 // 22.1 for (4, 5) and 17.8 for (8, 6); 67 x 6144 (4, 3) 11.3 against 14.2 for
-// (4, 2); 1072 x 6144 (8, 8) 40.6 against 45.1 for (8, 5).
+// (4, 2); 1072 x 6144 (8, 8) 40.6 against 45.1 for (8, 5).  The one-block tiles
+// are for few rows or columns, where (2, 2) leaves half the CUs idle: two Euler
+// steps of 4 layers at hidden 2048 take 484 us against 535 without them at 19
+// rows (514 on split-K GEMMs), 500 against 537 (572) at 35; 67 rows at hidden
+// 1024 410 against 446 (518).
 struct FragTile {
     int nb = 0, mb = 0, ntiles = 0, nms = 0;
 };
-constexpr int kFragTiles[][2] = {{2, 2}, {2, 3}, {2, 5}, {4, 2}, {4, 3}, {4, 4}, {4, 5}, {4, 8}, {8, 4}, {8, 5}, {8, 6}, {8, 8}};
+constexpr int kFragTiles[][2] = {{2, 1}, {2, 2}, {2, 3}, {2, 5}, {4, 1}, {4, 2}, {4, 3}, {4, 4}, {4, 5}, {4, 8}, {8, 4}, {8, 5}, {8, 6}, {8, 8}};
 // nb_min, nb_max: bounds from the epilogue.  small: only the tiles up to (4, 5),
 // for the operand types that no caller uses above 160 rows (bf16, int8).
 FragTile frag_tile(int M, int N, bool small, int nb_min, int nb_max) {
@@ -698,6 +702,7 @@ void launch_frag(const FragOps& o, const FragTile& t, const FragEpi& e, hipStrea
     const int tile = 16 * t.nb + t.mb;
     if constexpr (EPI != SF_EPI_HEADS) {
         switch (tile) {
+            case 16 * 2 + 1: launch_frag_tile<2, 1, 8, 2, EPI>(o, t, e, s); return;
             case 16 * 2 + 2: launch_frag_tile<2, 2, 8, 2, EPI>(o, t, e, s); return;
             case 16 * 2 + 3: launch_frag_tile<2, 3, 4, 2, EPI>(o, t, e, s); return;
             case 16 * 2 + 5: launch_frag_tile<2, 5, 4, 2, EPI>(o, t, e, s); return;
@@ -709,6 +714,7 @@ void launch_frag(const FragOps& o, const FragTile& t, const FragEpi& e, hipStrea
         }
     }
     switch (tile) {
+        case 16 * 4 + 1: launch_frag_tile<4, 1, 4, 2, EPI>(o, t, e, s); return;
         case 16 * 4 + 2: launch_frag_tile<4, 2, 4, 2, EPI>(o, t, e, s); return;
         case 16 * 4 + 3: launch_frag_tile<4, 3, 4, 2, EPI>(o, t, e, s); return;
         case 16 * 4 + 4: launch_frag_tile<4, 4, 4, 2, EPI>(o, t, e, s); return;

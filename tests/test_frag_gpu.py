@@ -80,7 +80,8 @@ def test_pack_layouts():
                                     (67, 6144, 1088), (81, 96, 320), (33, 32, 4096), (134, 8192, 576), (67, 2048, 8192),
                                     (402, 2048, 320), (539, 2048, 192), (640, 2048, 256), (603, 6144, 2048),
                                     (500, 6144, 448), (1072, 2048, 64), (1000, 2048, 704), (450, 6144, 128),
-                                    (700, 4096, 128), (999, 384, 192)])
+                                    (700, 4096, 128), (999, 384, 192), (15, 2048, 2048), (19, 2048, 320),
+                                    (64, 2048, 192), (65, 1024, 2048), (48, 6144, 128)])
 @pytest.mark.parametrize("kind,adt", [("w16", torch.bfloat16), ("w16", torch.float16), ("int8", torch.bfloat16),
                                       ("int8", torch.float16)])
 def test_plain(M, N, Kd, kind, adt):
@@ -110,7 +111,7 @@ def test_row_does_not_depend_on_the_batch(kind, dt, full):
             assert torch.equal(K.gemm_frag(M, to_frag(a[:M].contiguous()), wf, w_scale=s), whole[:M])
 
 
-@pytest.mark.parametrize("M,N", [(67, 2048), (134, 2048), (5, 64), (97, 4096), (640, 2048), (1072, 2048), (402, 1024)])
+@pytest.mark.parametrize("M,N", [(67, 2048), (134, 2048), (5, 64), (16, 2048), (19, 2048), (49, 2048), (19, 4096), (97, 4096), (640, 2048), (1072, 2048), (402, 1024)])
 @pytest.mark.parametrize("kind,adt,ndt", [("w16", torch.bfloat16, torch.bfloat16), ("int8", torch.bfloat16, torch.float16),
                                           ("w16", torch.float16, torch.float16)])
 def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
@@ -131,7 +132,7 @@ def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
     assert rel(got, ref) < 2e-5
 
 
-@pytest.mark.parametrize("B,S,H", [(1, 67, 32), (2, 67, 32), (3, 11, 2), (1, 160, 1)])
+@pytest.mark.parametrize("B,S,H", [(1, 67, 32), (2, 67, 32), (3, 11, 2), (1, 160, 1), (1, 19, 32), (1, 32, 32), (1, 4, 32)])
 @pytest.mark.parametrize("kind", ["w16", "int8"])
 def test_heads(B, S, H, kind):
     M, D = B * S, H * 64
@@ -160,7 +161,7 @@ def test_norm_frag(rows, cols, dt):
     assert rel(ss, x.double().view(rows, -1, 64).square().sum(-1)) < 1e-6
 
 
-@pytest.mark.parametrize("M,N,kind", [(67, 2048, "w16"), (134, 256, "int8"), (81, 4096, "w16"), (160, 2048, "int8"),
+@pytest.mark.parametrize("M,N,kind", [(67, 2048, "w16"), (19, 2048, "w16"), (134, 256, "int8"), (81, 4096, "w16"), (160, 2048, "int8"),
                                       (640, 2048, "w16"), (1072, 512, "w16")])
 def test_fp16_rows_out_of_range(M, N, kind):
     """Deferred fp16 rows whose x * gamma leaves fp16's range, is far below
