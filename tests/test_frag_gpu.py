@@ -47,10 +47,10 @@ def randn(seed, *shape, dtype=torch.float32, std=1.0):
 def weights(seed, N, Kd, kind, adt):
     """(fragment-ordered copy, scale or None, float64 values the copy means)."""
     w = randn(seed, N, Kd, std=0.02)
-    if kind == "int8":
+    if kind in ("int8", "codes16"):   # codes16: int8 codes widened to fp16, with their scale
         s = w.abs().amax(1) / 127
         q = torch.clamp(torch.round(w / s[:, None]), -127, 127).to(torch.int8)
-        return K.frag_pack([q], [torch.int8])[0], s, q.double() * s.double()[:, None]
+        return K.frag_pack([q], [torch.int8 if kind == "int8" else adt])[0], s, q.double() * s.double()[:, None]
     w = w.to(torch.bfloat16)
     return K.frag_pack([w], [adt])[0], None, w.to(adt).double()
 
@@ -83,7 +83,7 @@ def test_pack_layouts():
                                     (700, 4096, 128), (999, 384, 192), (15, 2048, 2048), (19, 2048, 320),
                                     (64, 2048, 192), (65, 1024, 2048), (48, 6144, 128)])
 @pytest.mark.parametrize("kind,adt", [("w16", torch.bfloat16), ("w16", torch.float16), ("int8", torch.bfloat16),
-                                      ("int8", torch.float16)])
+                                      ("int8", torch.float16), ("codes16", torch.float16)])
 def test_plain(M, N, Kd, kind, adt):
     a, (wf, s, w64) = randn(3, M, Kd, dtype=adt), weights(4, N, Kd, kind, adt)
     b = randn(5, N)
@@ -113,7 +113,7 @@ def test_row_does_not_depend_on_the_batch(kind, dt, full):
 
 @pytest.mark.parametrize("M,N", [(67, 2048), (134, 2048), (5, 64), (16, 2048), (19, 2048), (49, 2048), (19, 4096), (97, 4096), (640, 2048), (1072, 2048), (402, 1024)])
 @pytest.mark.parametrize("kind,adt,ndt", [("w16", torch.bfloat16, torch.bfloat16), ("int8", torch.bfloat16, torch.float16),
-                                          ("w16", torch.float16, torch.float16)])
+                                          ("w16", torch.float16, torch.float16), ("codes16", torch.float16, torch.float16)])
 def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
     """The deferred pair: x * gamma and tile sums out of one projection, the
     row scale applied by the next, against the normalised rows' product."""
@@ -134,14 +134,22 @@ def test_add_norm_and_its_consumer(M, N, kind, adt, ndt):
 
 @pytest.mark.parametrize("B,S,H", [(1, 67, 32), (2, 67, 32), (3, 11, 2), (1, 160, 1), (1, 19, 32), (1, 32, 32), (1, 4, 32)])
 @pytest.mark.parametrize("kind", ["w16", "int8"])
-def test_heads(B, S, H, kind):
+@pytest.mark.parametrize("deferred", [False, True])
+def test_heads(B, S, H, kind, deferred):
+    """Finished rows, and the rows of a deferred norm: their 1/rms after the product."""
     M, D = B * S, H * 64
     a, (wf, s, w64) = randn(15, M, D, dtype=torch.bfloat16), weights(16, 3 * D, D, kind, torch.bfloat16)
+    af, rows, row = to_frag(a), a.double(), {}
+    if deferred:
+        x = randn(22, M, D) * torch.linspace(0.1, 30, M, device=DEV)[:, None]
+        af, ss = K.norm_frag(x, 1 + randn(23, D, std=0.1), out_dtype=torch.bfloat16, deferred=True)
+        rows = from_frag(af, M).double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-6)
+        row = {"row_ss": ss, "row_n": D}
     b = randn(17, 3 * D)
     gq, gk = 1 + randn(18, 64, std=0.1), 1 + randn(19, 64, std=0.1)
     outs = [torch.full((B, H, S, 64), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3)]
-    K.gemm_frag_heads(M, to_frag(a), wf, b, S, H, outs, (gq, gk, None), w_scale=s)
-    ref = (a.double() @ w64.t() + b.double()).view(B, S, 3, H, 64).permute(2, 0, 3, 1, 4)
+    K.gemm_frag_heads(M, af, wf, b, S, H, outs, (gq, gk, None), w_scale=s, **row)
+    ref = (rows @ w64.t() + b.double()).view(B, S, 3, H, 64).permute(2, 0, 3, 1, 4)
     for j, g in enumerate((gq, gk, None)):
         r = ref[j]
         if g is not None:
@@ -246,14 +254,20 @@ def test_attention_frag_output(B, H, Sq, Sk, dt):
 
 # query blocks, key splits, the unsplit 80-row grid with a partial chunk, keys
 # of the short-key kernel (the ring kernel takes them), exact P.V
-@pytest.mark.parametrize("B,H,Sq,Sk,exact", [(1, 32, 67, 517, False), (1, 32, 67, 4374, False), (2, 32, 67, 4374, True),
-                                             (8, 32, 67, 300, False), (1, 4, 133, 2000, False), (1, 8, 19, 40, True)])
-def test_attention_fp32_q_rows(B, H, Sq, Sk, exact):
-    """Q as fp32 projection rows, normalised on load: bit for bit the
+# and V in bf16 or, as the model's cross-attention caches it, in fp16
+@pytest.mark.parametrize("B,H,Sq,Sk,form", [(1, 32, 67, 517, "bf16"), (1, 32, 67, 517, "fp16"), (1, 32, 67, 4374, "bf16"),
+                                            (1, 32, 67, 4374, "fp16"), (2, 32, 67, 4374, "exact"), (8, 32, 67, 300, "bf16"),
+                                            (8, 32, 67, 300, "fp16"), (1, 4, 133, 2000, "fp16"), (1, 8, 19, 40, "exact"),
+                                            (1, 8, 19, 40, "fp16")])
+def test_attention_fp32_q_rows(B, H, Sq, Sk, form):
+    """Q as fp32 projection rows, normalised on load, against the oracle's
     attention over rows normalised and rounded to bf16 beforehand."""
+    exact = form == "exact"
     rows = randn(30, B * Sq, H * 64, std=3.0)
     gamma = 1 + randn(31, 64, std=0.1)
     k, v = (randn(32 + i, B, H, Sk, 64, dtype=torch.bfloat16) for i in range(2))
+    if form == "fp16":
+        v = v.to(torch.float16)
     q32 = rows.view(B, Sq, H, 64).permute(0, 2, 1, 3)
     r64 = q32.double()
     q = (r64 * torch.rsqrt(r64.square().mean(-1, keepdim=True) + 1e-6) * gamma.double()).to(torch.bfloat16).contiguous()

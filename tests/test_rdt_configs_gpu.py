@@ -190,11 +190,17 @@ def test_loop_large_batch_graph_and_oracle(batch, int8):
         assert_within_floor(eager[b:b + 1], ref, floor, f"loop B={batch} slot {b}")
 
 
-@pytest.mark.parametrize("batch,int8", [(3, 0), (3, 1), (3, 2), (1, 0)])
-def test_weight_writes_reach_the_fp16_copies(batch, int8):
-    """The runtime multiplies fp16 copies of weights -- above 160 rows every
-    projection's, at batch 1 with bf16 weights the FFN matrices' -- rebuilt
-    before a pass only when the parameters may have changed.  A write
+FC2 = "blocks.1.ffn.fc2.weight"
+
+
+@pytest.mark.parametrize("batch,int8,name", [(3, 0, FC2), (3, 1, FC2), (3, 2, FC2), (1, 0, FC2), (10, 0, FC2), (1, 1, FC2),
+                                             (1, 0, "blocks.0.attn.qkv.weight"), (1, 1, "blocks.0.attn.qkv.weight"),
+                                             (1, 1, "blocks.1.cross_attn.q.weight"), (3, 0, "blocks.1.cross_attn.q.weight")])
+def test_weight_writes_reach_the_fp16_copies(batch, int8, name):
+    """The runtime multiplies copies of the block projections' weights -- in
+    fragment order up to 640 rows, int8 models at batch 1 included, row-major
+    fp16 above -- rebuilt before a pass only when the parameters may have
+    changed.  A write
     through sf_rdt_param_data after a pass (param_write), and a write
     through a pointer taken before a pass followed by sf_rdt_params_changed,
     both reach the next graph replay: its result matches the oracle on the
@@ -214,7 +220,6 @@ def test_weight_writes_reach_the_fp16_copies(batch, int8):
     base = loop()
     oc = oracle_cfg(c)
     for how in ("param_write", "raw_pointer"):
-        name = "blocks.1.ffn.fc2.weight"
         idx = R.lib().sf_rdt_find_param(m.h, name.encode())
         p0 = m.state_dict()
         if int8:
