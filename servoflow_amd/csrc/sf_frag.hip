@@ -57,10 +57,12 @@ constexpr int kFragRowTiles = 64;   // tile sums of a deferred row: 16 in each o
 // with a mean square of at least 1 each x * gamma is at least as large as the
 // normalised element.  Rows in range, every row of a model whose residual is
 // not degenerate, pay the comparison; a row's result does not depend on whether
-// its neighbours are in range.
+// its neighbours are in range.  A row that falls back takes its workgroup through
+// K again with scalar loads: 67 x 2048 x 2048 takes 30 us against 5.6 with one
+// such row or all of them, 402 x 6144 112 us with one and 309 with all against 22.
 enum RowKind { kRowPlain = 0, kRowDeferred = 1, kRowGuarded = 2 };
-constexpr float kGuardTopSq = 1.f / 4194304.f;   // times N: the mark's square
 constexpr float kF16Max = 65504.f;
+inline float guard_min(int cols) { return sqrtf((float)cols) / 2048.f; }   // the mark of a row of cols
 
 // The epilogue's arguments (the operands' pointers and sizes are scalar kernel
 // arguments of their own, see gemm_frag_kernel).
@@ -79,7 +81,7 @@ struct FragEpi {
     const float* norm_gamma;
     uint16_t* norm_out;
     float* norm_ss;
-    int norm_f16;
+    float norm_min;   // fp16: the range guard's mark (guard_min); bf16: 0
     // kRowGuarded: the fp32 rows [M][x_ld] and the norm's gamma
     const float* x;
     const float* x_gamma;
@@ -105,9 +107,13 @@ __device__ __forceinline__ float sum_groups(float x) {
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
-// Whether x holds in any of those four lanes.
+// Whether x holds in any of those four lanes (a few scalar operations on the
+// comparison's mask: the epilogue that asks is the end of its wave's path).
 __device__ __forceinline__ bool any_groups(bool x) {
-    return ((__ballot(x) >> (threadIdx.x & 15)) & 0x0001000100010001ull) != 0;
+    uint64_t q = __ballot(x);
+    q |= q >> 32;
+    q |= q >> 16;
+    return __builtin_amdgcn_inverse_ballot_w64((q & 0xffff) * 0x0001000100010001ull);
 }
 
 // One workgroup of 4 waves per (16 NB columns x 16 MB rows) of C over all of
@@ -454,6 +460,7 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int j = 0; j < EN; ++j) *reinterpret_cast<uint2*>(o + 16 * j + 4 * g4) = pack_kind4(v[j], false);
         } else if constexpr (kAddNorm) {
+            const bool norm_f16 = e.norm_min > 0.f;
             float ss = 0.f, top = 0.f;
             f32x4 u[EN];
 #pragma unroll
@@ -466,15 +473,15 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
                     top = fmaxf(top, fabsf(u[j][q]));
                 }
             }
-            if (e.norm_f16 && top > kF16Max) ss = INFINITY;   // the guard's marks
+            if (norm_f16 && top > kF16Max) ss = INFINITY;   // the guard's marks
             ss = sum_groups(ss);
-            if (e.norm_f16 && !any_groups(top * top >= kGuardTopSq * (float)e.N)) ss = -ss;
+            if (!any_groups(top >= e.norm_min)) ss = -ss;
             if (m >= M) continue;
 #pragma unroll
             for (int j = 0; j < EN; ++j) {
                 const int n = n0 + 16 * (EN * it + j) + 4 * g4;
                 *reinterpret_cast<f32x4*>(static_cast<float*>(e.c) + (int64_t)m * e.ldc + n) = v[j];
-                *reinterpret_cast<uint2*>(e.norm_out + frag_off(m, n, e.N)) = pack_kind4(u[j], e.norm_f16 != 0);
+                *reinterpret_cast<uint2*>(e.norm_out + frag_off(m, n, e.N)) = pack_kind4(u[j], norm_f16);
             }
             if (g4 == 0) e.norm_ss[(int64_t)m * (ntiles * IT) + tile * IT + it] = ss;
         } else {
@@ -505,7 +512,7 @@ __global__ __launch_bounds__(64 * kFragWaves) __attribute__((amdgpu_waves_per_eu
 // 64 columns of tile t.
 constexpr int kNormFragPer = 2;   // cols <= 2 * 256 * 8 = 4096
 __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t ldx, const float* gamma, uint16_t* out,
-                                                        int f16, float* ss, int cols, float eps) {
+                                                        int f16, float* ss, int cols, float eps, float min_top) {
     __shared__ float red[4];
     const int row = blockIdx.x;
     f32x4 v[kNormFragPer][2], gq[kNormFragPer][2];
@@ -538,7 +545,7 @@ __global__ __launch_bounds__(256) void norm_frag_kernel(const float* x, int64_t 
 #pragma unroll
                     for (int j = 0; j < 4; ++j) top = fmaxf(top, fabsf(v[i][h][j] * gq[i][h][j]));
                 if (top > kF16Max) sum[i] = INFINITY;
-                small = !((__ballot(top * top >= kGuardTopSq * (float)cols) >> (threadIdx.x & 56)) & 255);
+                small = !((__ballot(top >= min_top) >> (threadIdx.x & 56)) & 255);
             }
             const float t = row8_sum(sum[i]) * (small ? -1.f : 1.f);
             const int c = 8 * ((int)threadIdx.x + 256 * i);
@@ -792,7 +799,7 @@ extern "C" int sf_norm_frag(const float* x, int64_t ldx, const float* gamma, voi
     if ((cols & 63) || cols > 2048 * sfk::kNormFragPer) return SF_ENOTSUP;
     if ((ldx & 3) || !fal16(x) || !fal16(gamma) || !fal16(out)) return SF_EINVAL;
     hipLaunchKernelGGL(sfk::norm_frag_kernel, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream), x, ldx, gamma,
-                       static_cast<uint16_t*>(out), out_dtype == SF_F16 ? 1 : 0, ss, cols, eps);
+                       static_cast<uint16_t*>(out), out_dtype == SF_F16 ? 1 : 0, ss, cols, eps, sfk::guard_min(cols));
     return hipGetLastError() == hipSuccess ? SF_OK : SF_ELAUNCH;
 }
 
@@ -867,7 +874,7 @@ extern "C" int sf_gemm_frag(const sf_frag_gemm_desc* d, void* stream) {
         a.ldc = d->ldc;
         a.norm_gamma = d->norm_gamma;
         a.norm_out = static_cast<uint16_t*>(d->norm_out);
-        a.norm_f16 = d->norm_dtype == SF_F16;
+        a.norm_min = d->norm_dtype == SF_F16 ? sfk::guard_min(d->N) : 0.f;
         a.norm_ss = d->norm_ss;
     } else if (d->epilogue == SF_EPI_PLAIN) {
         if (!d->C) return SF_EINVAL;
