@@ -111,17 +111,19 @@ typedef struct sf_rdt_config {
     int32_t num_steps;           /* 5 Euler steps */
     int32_t batch;
     int32_t int8_weights;        /* nonzero: block projections as int8 + fp32
-                                    row scale.  At batch * (horizon + 3) > 160
-                                    the runtime (int8 or not) also holds fp16
-                                    copies of the block and final-layer
-                                    matrices (2 bytes per weight), rewritten
-                                    before the first pass after the parameters
-                                    may have changed; with 2, no copy of the
-                                    int8 matrices sf_gemm multiplies directly
-                                    there (sf_gemm_int8_direct: every block
-                                    matrix with K = 2048), which read their
-                                    1-byte codes instead -- less memory and
-                                    half the weight bytes, slower products */
+                                    row scale.  int8 or not, the passes
+                                    multiply copies of the block matrices (all
+                                    but the cross K/V) and of the final layer's
+                                    (see sf_rdt_param_data): with rows = batch *
+                                    (horizon + 3), 2 bytes per weight, int8
+                                    models at rows <= 160 1 byte (the codes).
+                                    With 2, at rows > 160, no copy of the int8
+                                    matrices sf_gemm multiplies directly
+                                    (sf_gemm_int8_direct: every block matrix
+                                    with K = 2048), which read their 1-byte
+                                    codes instead -- less memory and half the
+                                    weight bytes, slower products; at rows <=
+                                    160 it is the same as 1 */
     float eps;                   /* 1e-6 */
     int32_t mlp_ratio;           /* FFN hidden = mlp_ratio * hidden (1; 0 means 1) */
 } sf_rdt_config;
@@ -141,16 +143,19 @@ int sf_rdt_init_random(sf_rdt* m, uint64_t seed, float std, void* stream);
 int32_t sf_rdt_num_params(const sf_rdt* m);
 int sf_rdt_param_info(const sf_rdt* m, int32_t idx, const char** name, int32_t* dtype,
                       int32_t* ndim, int64_t shape[4]);
-/* Device pointer to parameter idx.  The runtime multiplies fp16 copies of
- * some weights (above 160 projection rows, batch * 67, every block and
- * final-layer matrix but, with int8_weights = 2, the int8 ones read
- * directly; at most 160 rows with bf16 weights, the FFN matrices, whose
- * inputs are fp16); they are rebuilt before the first pass after this
- * call, after
- * sf_rdt_init_random / sf_rdt_load_safetensors, and after
- * sf_rdt_params_changed -- a caller that writes through a pointer it
- * obtained before a pass must call sf_rdt_params_changed before the next
- * one. */
+/* Device pointer to parameter idx.  The passes read biases, norm weights, int8
+ * row scales, the adaptors' and embedders' and the cross K/V matrices in place,
+ * but multiply copies of every other block matrix and of the final layer's: up
+ * to 640 rows, batch * (horizon + 3), in the order of the matrix operands
+ * (bf16 or fp16; int8 codes as codes at most at 160 rows, else as fp16), above
+ * row-major fp16 (but, with int8_weights = 2 above 160 rows, the int8 ones
+ * read directly).  The copies are rebuilt before the first pass after this
+ * call, after sf_rdt_init_random / sf_rdt_load_safetensors, and after
+ * sf_rdt_params_changed -- a caller that writes through a pointer it obtained
+ * before a pass must call sf_rdt_params_changed before the next one, or the
+ * pass multiplies the old weights.  At 28 layers of 2048 that pass takes 0.6
+ * (int8) to 0.9 ms longer.  A graph that the caller recorded from passes holds
+ * the rebuild only if it was due when the pass was recorded. */
 void* sf_rdt_param_data(sf_rdt* m, int32_t idx);
 /* Parameters were written through pointers from sf_rdt_param_data: the
  * weight copies are rebuilt (and sf_rdt_infer's cached condition
@@ -165,7 +170,9 @@ int32_t sf_rdt_find_param(const sf_rdt* m, const char* name);
  * position embeddings and projects every block's cross-attention K/V once,
  * and embeds the control-frequency token and the timestep tokens of the
  * sampler's schedule (they depend on the weights only), so set or load the
- * weights before the condition. */
+ * weights before the condition.  Where the language rows have changed
+ * (sf_rdt_set_lang_rows) the sampler's graph is taken down, which waits on the
+ * host for its last replay. */
 int sf_rdt_set_condition(sf_rdt* m, const void* lang_c, const int32_t* lang_len,
                          const void* img_c, const void* state_tok, void* stream);
 /* Raw tokens: lang bf16 [B, lang_max, 4096], img bf16 [B, img_len, 1152],
@@ -197,7 +204,8 @@ int sf_rdt_denoise_step(sf_rdt* m, const float* x_t, float t, float* velocity, v
  * use_graph != 0 captures the loop into a hipGraph on the first call and
  * replays it afterwards (inputs are copied in and out around the graph).
  * Like every entry point here it works on the stream it is given, NULL being
- * the device's default stream. */
+ * the device's default stream: two models' calls there run one after the
+ * other, on streams of their own they can overlap. */
 int sf_rdt_sample(sf_rdt* m, float* x, int32_t use_graph, void* stream);
 
 /* InferenceEngine::infer (src/engine/inference_engine.cpp:99-175) on this

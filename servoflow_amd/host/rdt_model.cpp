@@ -83,7 +83,11 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // rows 69 vs 98 us, 536 rows 82 vs 117.  The line lies where the QKV product's
 // 128 x 128 tiles need a second round of workgroups (hidden 2048: 5 x 48 = 240
 // up to 640 rows): five steps of 4 layers take 3.34 vs 3.64 ms at 536 rows,
-// 3.70 vs 4.00 at 603, 4.15 vs 4.14 at 670, 4.48 vs 4.39 at 804.
+// 3.70 vs 4.00 at 603, 4.15 vs 4.14 at 670, 4.48 vs 4.39 at 804.  Narrower products
+// need that round later and wider ones sooner; up to 603 rows no hidden size
+// loses (two steps of 4 layers at 201 / 402 / 603 rows: 512 645 vs 456, 674 vs
+// 495, 691 vs 508 us; 1024 715 vs 497, 783 vs 610, 859 vs 689; 4096 1770 vs 1519,
+// 2143 vs 2120, 2790 vs 2689), above 640 narrower ones were not measured.
 // int8_weights = 2 above 160 rows keeps no 16-bit copies and stays with sf_gemm.
 constexpr int64_t kFragStepRows = 640;
 constexpr int64_t kSmallStepRows = 160;   // bf16 projection inputs, per-head QKV epilogue
@@ -203,11 +207,16 @@ struct sf_rdt {
     // weights rounded), at most 160 rows bf16, fp16 for the matrices whose
     // inputs are fp16 (fc1, fc2, the final fc2), or the int8 codes
     // (sf_frag_pack).  Otherwise (w16_params) row-major fp16 copies of the same
-    // matrices (sf_weights_to_f16).
+    // matrices (sf_weights_to_f16); int8_weights = 2 keeps none of the int8
+    // block matrices there, but its codes in fragment order at most 160 rows.
     // Up to eight matrices per launch, made before the first pass and again before
     // the first pass after the parameters may have changed (copies_stale), on
-    // the pass's stream and outside any graph capture -- not once per loop:
-    // a batch-16 loop refreshing them in its graph took 0.8 ms more.
+    // the pass's stream and outside the sampler's capture -- not once per loop:
+    // a batch-16 loop refreshing them in its graph took 0.8 ms more.  28 layers
+    // of 2048, the first pass after a weight change against the next: batch 1
+    // 2.54 vs 1.65 ms, int8 2.15 vs 1.57 (with copies of the FFN matrices only
+    // and split-K products 2.23 vs 2.09, int8 without any 2.12); batch 6 4.10 vs
+    // 3.16 (4.52 vs 3.80).
     // copy_of[param] is a weight's copy (fixed at creation).
     char* copies = nullptr;
     size_t copies_bytes = 0;
@@ -217,7 +226,7 @@ struct sf_rdt {
     // The copies may no longer match the weights: set by every call that
     // writes parameters or hands out a pointer to them (and by
     // sf_rdt_params_changed), cleared by the refresh at the start of the
-    // next pass.
+    // next pass unless a caller's capture records it.
     bool copies_stale = true;
 
     hipGraph_t graph = nullptr;
@@ -1108,7 +1117,7 @@ extern "C" int sf_rdt_create(const sf_rdt_config* cfg, sf_rdt** out) {
     sf_rdt* m = new sf_rdt();
     m->cfg = c;
     // fp16 FFN inputs at every batch size; the other projection inputs in
-    // fp16 once the block GEMMs leave the fragment-ordered step (M > 160 rows)
+    // fp16 above kSmallStepRows
     m->ffn_dtype = SF_F16;
     const int64_t step_rows = (int64_t)c.batch * (c.horizon + 3);
     m->act16 = step_rows <= kSmallStepRows ? SF_BF16 : SF_F16;
