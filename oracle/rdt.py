@@ -16,8 +16,8 @@ are rounded, to model a pipeline that stores them in 16-bit types:
   False  none: the pure fp32 restatement;
   a set  of point names rounded to bf16;
   a dict point name -> "bf16" or "f16", e.g. storage_points(ffn16=True) for
-         the MI355X runtime at batch <= 2, which stores the FFN inputs (the
-         norm3 output and the GELU hidden) in fp16.
+         the MI355X runtime (runtime_points), which stores the FFN inputs
+         (the norm3 output and the GELU hidden) in fp16.
 The residual stream stays fp32 throughout; the block's projection outputs
 stay fp32 except at the "gemm" point.  The reference's own bf16 build rounds
 at all of these points and also rounds the residual (norm.cuh:146).
@@ -75,8 +75,8 @@ def storage_points(ffn16, gemm16=False, act16=False):
     ffn16: the FFN inputs n3 and h in fp16;
     gemm16: the block projections' products ("gemm", "hgemm") in bf16
             (fp32 otherwise);
-    act16 (the runtime above 160 rows, with ffn16): every projection input
-            in fp16 (norm outputs "n1" / "n2", attention outputs "a"), the
+    act16 (the runtime above 160 rows, with ffn16; up to 640 rows its
+            "gemm" is fp32, runtime_points): every projection input in fp16 (norm outputs "n1" / "n2", attention outputs "a"), the
             products in fp16 ("gemm", "hgemm"), the self-attention's per-head
             q / k / v in fp16 ("qkv"); the cross-attention's q ("cq") stays
             bf16 (its K / V cache is bf16)."""
@@ -91,16 +91,21 @@ def storage_points(ffn16, gemm16=False, act16=False):
     return pts
 
 
-def runtime_points(rows):
-    """The MI355X runtime's storage at `rows` = batch * 67 projection rows:
-    the split-K regime (<= 160) keeps bf16 inputs with fp16 FFN inputs and
-    fp32 products, and norm1 / norm2 in their deferred form ("defer": the
-    rows x * gamma are stored, the projection's output rows scaled by
-    1/rms after the product); the library regime (> 160) keeps fp16 inputs
-    and fp16 products (storage_points)."""
+def runtime_points(rows, library=None):
+    """The MI355X runtime's storage at `rows` = batch * 67 projection rows.
+    Up to 640 the fragment-ordered step: norm1, norm2 and norm3 in their
+    deferred form ("defer": the rows x * gamma are stored, the projection's
+    output rows scaled by 1/rms after the product), the residual products
+    ("gemm") in fp32; at most 160 rows bf16 inputs with fp16 FFN inputs and
+    the per-head products ("hgemm") in fp32, above them fp16 inputs and fp16
+    per-head products.  Above 640 (library; int8_weights = 2: above 160) fp16
+    inputs and products, the norms finished (storage_points)."""
+    if library is None:
+        library = rows > 640
     pts = storage_points(True, act16=rows > 160)
-    if rows <= 160:
+    if not library:
         pts["defer"] = True
+        pts["gemm"] = "fp32"
     return pts
 
 
@@ -156,6 +161,12 @@ def _deferred_linear(x, gamma, W, b, eps, rb, point):
     return O.linear(a, W) * s + np.asarray(b, np.float32)
 
 
+def _gelu(x):
+    """GELU (tanh form, elementwise.cuh:35-54) of what O.linear gives without its activation."""
+    x = np.asarray(x, np.float64)
+    return (0.5 * x * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (x + 0.044715 * x ** 3)))).astype(np.float32)
+
+
 def rdt_block(p, i, x, ck, cv, cond_len, cfg, rb=True):
     """RDTBlock::forward, src/models/rdt1b/dit_block.cu:349-387, with the
     cross-attention K/V precomputed (cross_kv).  x [B,S,D] fp32, updated."""
@@ -187,8 +198,12 @@ def rdt_block(p, i, x, ck, cv, cond_len, cfg, rb=True):
     ca = _r(O.head_to_seq(O.attention_f32(cq, ck, cv, valid_len=cond_len)), rb, "a")
     x = x + _r(O.linear(ca, p[pre + "cross_attn.proj.weight"], p[pre + "cross_attn.proj.bias"]), rb, "gemm")
     # FFN branch (Mlp::forward, dit_block.cu:143-163: fc1 + GELU, fc2)
-    n3 = _r(O.rms_norm(x, p[pre + "norm3.weight"], cfg.eps), rb, "n3")
-    h = _r(O.linear(n3, p[pre + "ffn.fc1.weight"], p[pre + "ffn.fc1.bias"], act=1), rb, "h")
+    if defer:
+        h = _r(_gelu(_deferred_linear(x, p[pre + "norm3.weight"], p[pre + "ffn.fc1.weight"], p[pre + "ffn.fc1.bias"],
+                                      cfg.eps, rb, "n3")), rb, "h")
+    else:
+        n3 = _r(O.rms_norm(x, p[pre + "norm3.weight"], cfg.eps), rb, "n3")
+        h = _r(O.linear(n3, p[pre + "ffn.fc1.weight"], p[pre + "ffn.fc1.bias"], act=1), rb, "h")
     return x + _r(O.linear(h, p[pre + "ffn.fc2.weight"], p[pre + "ffn.fc2.bias"]), rb, "gemm")
 
 

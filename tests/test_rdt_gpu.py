@@ -56,12 +56,14 @@ def bf(x):
 
 def rb_of(c):
     """The oracle's storage model of the runtime at config c
-    (OR.runtime_points): at batch * 67 <= 160 rows bf16 everywhere except
-    the FFN inputs (norm3 output, GELU hidden) in fp16, products in fp32;
-    above 160 rows every projection input, the products and the
-    self-attention's q / k / v in fp16, the cross-attention's q and the K/V
-    cache in bf16."""
-    return OR.runtime_points(c.batch * (c.horizon + 3))
+    (OR.runtime_points): up to 640 rows deferred norms and fp32 residual
+    products, at batch * 67 <= 160 rows bf16 everywhere except the FFN inputs
+    (norm3 output, GELU hidden) in fp16; above 160 rows every projection
+    input, the per-head products and the self-attention's q / k / v in fp16,
+    the cross-attention's q and the K/V cache in bf16; above 640 rows
+    (int8_weights = 2: 160) finished norms and fp16 products."""
+    rows = c.batch * (c.horizon + 3)
+    return OR.runtime_points(rows, rows > (160 if c.int8_weights == 2 else 640))
 
 
 def make_condition(c, seed=5, lang_len=None):
