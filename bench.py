@@ -585,8 +585,8 @@ def main():
                     help="build one large-batch model and replay its loop 3 times (for rocprofv3)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print(f"bench.py: this build measures one GPU; --gpus {args.gpus} is not supported "
-              "(every GPU box here has one MI355X).", file=sys.stderr)
+        print(f"bench.py: the benchmark measures one GPU; --gpus {args.gpus} is not supported "
+              "(the path does not shard).", file=sys.stderr)
         sys.exit(2)
 
     import numpy as np

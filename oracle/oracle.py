@@ -61,7 +61,7 @@ def _c32(a):
 
 
 def randn(seed: int, shape, std: float = 1.0) -> np.ndarray:
-    """SplitMix64 -> Box-Muller N(0, std^2) (the build's deterministic inputs)."""
+    """SplitMix64 -> Box-Muller N(0, std^2) (deterministic inputs)."""
     n = int(np.prod(shape))
     out = np.empty(n, dtype=np.float32)
     lib().sfo_randn(seed & 0xFFFFFFFFFFFFFFFF, n, std, out)

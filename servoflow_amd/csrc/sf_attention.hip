@@ -1039,7 +1039,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnArgs a) {
 constexpr int kShortMaxKeys = 128;
 // B*H from which a workgroup takes all of a head's query blocks, one wave
 // each, sharing one LDS copy of the head's K and V (27 KB at 67 keys).
-// Same-box A/B, self-attention over the QKV rows with q/k norm on load,
+// Timed in turn, self-attention over the QKV rows with q/k norm on load,
 // against one-wave workgroups: B=8 7.2 vs 8.6 us (per-wave V copies),
 // B=16 12.5 vs 15.2, B=32 22.5 vs 23.3.  (With a V copy per wave, 77 KB per
 // workgroup, the grouped form had lost at B*H = 1024: 20.9 vs 19.4 us.)
@@ -1270,7 +1270,7 @@ __global__ __launch_bounds__(64 * NW) void attn_short_kernel(const AttnArgs a) {
 // 74.3, 20.2, 8.5, 86.6.  Few keys and large grids take fewer (f32_waves).
 // The query blocks on one XCD and these operand orders, against query blocks
 // spread over up to five XCDs, K loads of 16-byte pieces and 4-byte V loads (same
-// timing, another box): B = 2 x 4374 keys 76.7 -> 72.8, B = 1 60.3 -> 45.3, B = 8
+// timing, another card): B = 2 x 4374 keys 76.7 -> 72.8, B = 1 60.3 -> 45.3, B = 8
 // 379 -> 247, 517 keys 13.4 -> 12.5, 67 keys 5.8 -> 5.2, B = 8 ragged 63.7 -> 46.1.
 // The call of 11 keys took 4.04 us with the XCD's group found by three divisions
 // and the arguments fetched in three rounds, 3.57 with neither.

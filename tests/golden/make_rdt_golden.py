@@ -2,8 +2,8 @@
 composition at a reduced size, computed by the reference's own PyTorch
 definition of the model.
 
-Run from the repository root, in the build container only (the reference
-tree does not exist on the GPU box, and nothing there runs this script):
+Run from the repository root where the reference tree is at hand (the tests
+need only the file that it writes):
 
     python tests/golden/make_rdt_golden.py
 
